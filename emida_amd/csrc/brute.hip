@@ -6,12 +6,16 @@
 // inner, as fused multiply-adds (the reference's nvcc build contracts
 // `sum += a * b`), so double and float results are bit-identical to that order.
 //
-// Three kernels: a register-blocked one (below, "tiled") for slices up to 128 pixels
-// wide, correlation windows up to 256 wide and launches of at least 256 workgroups;
-// for other shapes whose slices fit in LDS, one with eight x-shifts per thread sliding
-// a register window over zero-padded rows ("x8"); and a thread-per-shift one for the
-// rest: one workgroup per (slice, 4-row band of shifts, 64-column band of shifts),
-// staged in LDS when both slices fit in 64 KiB.
+// Float and double run on the matrix cores (cross_corr_mm_kernel); slices too wide for its
+// LDS rows take the thread-per-shift kernel: one workgroup per (slice, 4-row band of shifts,
+// 64-column band of shifts), staged in LDS when both slices fit in 64 KiB.  int32 has no
+// matrix instruction with its wrapping sums and keeps the vector kernels: a register-blocked
+// one ("tiled") for slices up to 128 pixels wide, windows up to 256 wide and launches of at
+// least 256 workgroups, one with eight x-shifts per thread sliding a register window over
+// zero-padded rows ("x8") for other slices that fit in LDS, and the thread-per-shift one.
+#include <algorithm>
+#include <type_traits>
+
 #include "kernels.hpp"
 
 namespace emida_amd {
@@ -336,9 +340,395 @@ __global__ __launch_bounds__(256, 2) void cross_corr_tiled_kernel(const T* __res
     }
 }
 
-// Workgroups of the register-blocked kernel for this launch, or 0 when the
-// thread-per-shift kernel runs instead (shape outside the tiled limits, or fewer
-// workgroups than CUs, where the finer grid of the thread-per-shift kernel is faster).
+// ------------------------------------------------------------------ matrix-core kernel
+// The same sums for float and double on the matrix cores, bit for bit: on gfx950
+// v_mfma_f64_4x4x4 and v_mfma_f32_16x16x4 round like a chain of fused multiply-adds over
+// k = 0..3 that starts at the accumulator (subnormals kept), so one accumulator per shift
+// fed with ascending pattern columns of ascending rows sees its terms y outer, x inner.
+//
+// For one slice and reference row y, C[sy][sx] += sum_c P[y + sy][c] * R[y][c - sx]: the
+// rows of A are 16 consecutive y-shifts (pattern rows), the columns of B are x-shifts (a
+// Toeplitz matrix of the reference row), k runs over 4 pattern columns.  No batch of
+// patterns is needed, so a single pattern fills the matrix cores as a batch does.
+//
+// A wave holds tiles of 16 y-shifts x NJ TB x-shifts, TB fragments of NJ x-shifts each
+// (double: NJ = 4, the four 4 x 4 blocks of the instruction being 4 groups of y-shifts;
+// float: NJ = 16).  Fragment n at column step t reads G(t - n NJ / 4), with
+// G(u)[k][j] = R[base + 4 u + k - j]: a step loads one A fragment and one G and keeps the
+// earlier G's in registers.  Steps in which a fragment's Toeplitz block is zero are left
+// out.  Double: where the window is wide, tiles lie on one side of shift 0, so the zero
+// steps are a triangle at the start of a tile (sx >= 0) or at its end (sx < 0), written out
+// as straight-line blocks of 8 steps.  Float: a condition per fragment and 4 steps.
+// Rows outside the slice read a zero row and columns past it read zero padding: those
+// terms add a product with an exact zero.  Such a term is not neutral for infinities and
+// NaN, so a workgroup that stages one sums its shifts term by term instead.
+//
+// Bound: the matrix pipe (72 TFLOP/s measured for v_mfma_f64_4x4x4 alone).  FP64, 100 ROIs
+// of 128 x 128, 16 patterns, 255 x 255 window: 15.4 ms (register-blocked vector kernel
+// 27.8 ms; 65 TFLOP/s executed, of which 55 useful); FP64, 25 ROIs of 32 x 32, 16 patterns: 46 us (8-shift vector
+// kernel 98 us; 800 workgroups on 256 CUs, 12 us of it staging and results);
+// float, 63 ROIs of 75 x 61, 12 patterns, 41 x 33 window: 210 us (935 us; the
+// window is computed as 48 x 48).
+typedef float mm_f4 __attribute__((ext_vector_type(4)));
+
+template <class T>
+struct mm_frag;
+template <>
+struct mm_frag<double> {
+    using acc = double;
+    static constexpr int NJ = 4, REGS = 1;
+    static __device__ __forceinline__ void mac(acc& c, double a, double b) {
+        c = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ double get(const acc& c, int) { return c; }
+    // lane l holds D[4 ((l % 16) / 4) + l / 16][l % 4]
+    static __device__ __forceinline__ int row(int lane, int) { return 4 * (lane % 16 / 4) + lane / 16; }
+    static __device__ __forceinline__ int col(int lane) { return lane % 4; }
+};
+template <>
+struct mm_frag<float> {
+    using acc = mm_f4;
+    static constexpr int NJ = 16, REGS = 4;
+    static __device__ __forceinline__ void mac(acc& c, float a, float b) {
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ float get(const acc& c, int r) { return c[r]; }
+    // lane l, register r holds D[4 (l / 16) + r][l % 16]
+    static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane / 16) + r; }
+    static __device__ __forceinline__ int col(int lane) { return lane % 16; }
+};
+
+constexpr int kMmTY = 16;  // y-shifts of a tile
+
+struct mm_shape {
+    int tb;              // fragments per tile
+    int x0;              // first x-shift of tile 0
+    int ntx, nty;        // tiles of a slice
+    int wx, wy;          // waves along x-shift tiles and y-shift tiles (wx * wy = 4)
+    int ntw;             // x-shift tiles per wave (1 or 2)
+    int nxb, nyb;        // workgroups of one slice along x and y
+    int cy;              // reference rows per staged chunk
+    int prows;           // pattern rows per staged chunk
+    int pitch, rpitch;   // LDS row lengths of pattern and reference rows
+    int padl;            // zeros before the first reference row
+    size_t lds;
+};
+
+template <class T>
+inline bool mm_plan(size2 size, size2 res, uint64_t total, mm_shape& m) {
+    constexpr int NJ = mm_frag<T>::NJ;
+    const int rx = (int)(res.x - 1) / 2, w = (int)res.x, S = (int)size.x;
+    if (size.x > 4096 || size.y > 65536) return false;
+    m.nty = div_up((int)res.y, kMmTY);
+    // Tile width: a wide tile reads fewer fragments per product, a narrow one rounds the
+    // window and the slice width up less; a narrower one has to save an eighth (a 41 x 33
+    // window of 75 x 61 slices in float: 48 wide 217 us, 32 wide 286 us, 16 wide 290 us).
+    m.tb = 0;
+    int best = 0;
+    for (int tb : {32 / NJ, 48 / NJ, 16 / NJ}) {
+        if (NJ == 4 && tb == 12) continue;
+        const int tx = NJ * tb, unit = NJ == 4 ? tx : 16;
+        const int cost = div_up(w, tx) * tx * div_up(S, unit) * unit;
+        if (m.tb == 0 || 8ll * cost < 7ll * best) {
+            best = cost;
+            m.tb = tb;
+        }
+    }
+    const int tx = NJ * m.tb;
+    m.ntx = div_up(w, tx);
+    m.x0 = -rx;
+    const int nneg = div_up(rx, tx);
+    const bool split = nneg + div_up(w - rx, tx) == m.ntx;  // tiles on one side of shift 0 cost nothing
+    if (split) m.x0 = -tx * nneg;
+    // two x-shift tiles per wave (a long and a short one) where that leaves every SIMD four
+    // waves; small launches spread over twice the waves instead
+    m.ntw = m.ntx > 1 && total * m.nty * div_up(m.ntx, 2) >= 4096 ? 2 : 1;
+    const int per = div_up(m.ntx, m.ntw);
+    m.wx = per >= 4 ? 4 : (per >= 2 ? 2 : 1);
+    m.wy = 4 / m.wx;
+    m.nxb = div_up(m.ntx, m.wx * m.ntw);
+    m.nyb = div_up(m.nty, m.wy);
+    // Pattern rows 2 mod 4 doubles (4 mod 8 floats) apart: the rows of an A fragment fall on
+    // distinct banks.  Both kinds of row are followed by the zeros the fragments read past the
+    // slice (a pattern row: a tile's columns; a reference row: those and, for a tile across
+    // shift 0, its width; float fragments read up to 31 past either end).
+    m.pitch = div_up(S, 8) * 8 + (NJ == 4 ? tx + 6 : 20);
+    const int padr = NJ == 4 ? (split ? tx : 2 * tx) + 4 : 36;
+    m.padl = NJ == 4 ? (split ? 4 : tx + 4) : 36;
+    m.rpitch = S + padr;
+    const int span = kMmTY * m.wy - 1;
+    auto bytes = [&](int cy) {
+        m.prows = std::min((int)size.y, cy + span);
+        return ((size_t)(m.prows + 1) * m.pitch + (size_t)cy * m.rpitch + m.padl) * sizeof(T);
+    };
+    // the most rows per chunk that let three workgroups share a CU's 160 KB, else two, else one
+    for (size_t budget : {(size_t)53248, (size_t)79872, (size_t)155648}) {
+        int cy = (int)size.y;
+        while (cy > 0 && bytes(cy) > budget) --cy;
+        if (cy >= std::min(8, (int)size.y)) {
+            m.cy = cy;
+            m.lds = bytes(cy);
+            return true;
+        }
+    }
+    return false;
+}
+
+template <class T>
+__device__ __forceinline__ bool mm_not_finite(T v) {
+    if constexpr (sizeof(T) == 8)
+        return (__builtin_bit_cast(uint64_t, v) >> 52 & 0x7ff) == 0x7ff;
+    else
+        return (__builtin_bit_cast(uint32_t, v) >> 23 & 0xff) == 0xff;
+}
+
+enum { MM_FULL, MM_HEAD, MM_TAIL };
+
+// Rows [y0, y1) of the chunk for one tile.  pa_of(y): this lane's A element of pattern column
+// 0; pr_of(y): its G element of reference column 0 (k - j from the row's start).
+template <int TB, class PA, class PR>
+__device__ __forceinline__ void mm_tile(double (&acc)[TB], int y0, int y1, PA&& pa_of, PR&& pr_of, int s0, int S) {
+    using F = mm_frag<double>;
+    constexpr int TX = F::NJ * TB;
+    static_assert(F::NJ == 4, "a step moves one fragment");
+    double g[TB];  // G(t - n) in g[(t - n) mod TB]; a block of TB steps covers TX columns
+    auto block = [&](const double* pa, const double* pr, auto mode_c) {
+        constexpr int MODE = decltype(mode_c)::value;
+        double a[TB];
+#pragma unroll
+        for (int t = 0; t < TB; ++t) a[t] = pa[4 * t];
+        double h[TB];
+#pragma unroll
+        for (int t = 0; t < (MODE == MM_TAIL ? 1 : TB); ++t) h[t] = pr[4 * t];
+#pragma unroll
+        for (int t = 0; t < TB; ++t) {
+            if (MODE != MM_TAIL || t == 0) g[t] = h[t];
+#pragma unroll
+            for (int n = 0; n < TB; ++n) {
+                if (MODE == MM_HEAD && t < n) continue;
+                if (MODE == MM_TAIL && t > n) continue;
+                F::mac(acc[n], a[t], g[(t - n + TB) % TB]);
+            }
+        }
+    };
+    using full = std::integral_constant<int, MM_FULL>;
+    if (s0 >= 0) {  // columns from s0: the first block is the triangle n <= t
+        const int blocks = (S - s0 + TX - 1) / TX;
+        if (blocks <= 0) return;
+        for (int y = y0; y < y1; ++y) {
+            const double* pa = pa_of(y) + s0;
+            const double* pr = pr_of(y);
+            block(pa, pr, std::integral_constant<int, MM_HEAD>{});
+            for (int b = 1; b < blocks; ++b) block(pa + b * TX, pr + b * TX, full{});
+        }
+    } else {
+        // columns from 0; left of shift 0 the last block is the triangle n >= t (of a slice
+        // padded to a whole number of blocks)
+        const bool neg = s0 + TX <= 0;
+        const int blocks = neg ? (max(0, S + s0) + TX - 1) / TX : (S + TX - 1) / TX;
+        if (neg && S + s0 + TX - 1 <= 0) return;
+        for (int y = y0; y < y1; ++y) {
+            const double* pa = pa_of(y);
+            const double* pr = pr_of(y) - s0;
+#pragma unroll
+            for (int n = 1; n < TB; ++n) g[TB - n] = pr[-4 * n];
+            for (int b = 0; b < blocks; ++b) block(pa + b * TX, pr + b * TX, full{});
+            if (neg) block(pa + blocks * TX, pr + blocks * TX, std::integral_constant<int, MM_TAIL>{});
+        }
+    }
+}
+
+// The same in float, in groups of 4 steps (16 columns, the width of a fragment): fragment n
+// at group c reads the G's of group c - n, which move up one fragment per group.
+template <int TB, class PA, class PR>
+__device__ __forceinline__ void mm_tile(mm_f4 (&acc)[TB], int y0, int y1, PA&& pa_of, PR&& pr_of, int s0, int S) {
+    using F = mm_frag<float>;
+    const int xb = max(0, s0), base = max(0, -s0);
+    auto lo = [&](int n) { return (max(0, s0 + 16 * n) - xb) >> 4; };
+    auto hi = [&](int n) { return (min(S, S + s0 + 16 * n + 15) - xb + 15) >> 4; };
+    const int groups = hi(TB - 1);
+    int all_lo = 0, all_hi = groups;  // groups in which every fragment has terms
+#pragma unroll
+    for (int n = 0; n < TB; ++n) {
+        all_lo = max(all_lo, lo(n));
+        all_hi = min(all_hi, hi(n));
+    }
+    for (int y = y0; y < y1; ++y) {
+        const float* pa = pa_of(y) + xb;
+        const float* pr = pr_of(y) + base;
+        float g[TB][4];
+        auto load = [&](const float* q, bool in, float (&v)[4]) {  // zeros where they lie wholly outside the row
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = in ? q[4 * i] : 0.0f;
+        };
+#pragma unroll
+        for (int n = 1; n < TB; ++n) load(pr - 16 * n, base - 16 * n > -16 && base - 16 * n - 15 < S, g[n - 1]);
+        auto up = [&] {
+#pragma unroll
+            for (int n = TB - 1; n > 0; --n)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) g[n][i] = g[n - 1][i];
+        };
+        auto some = [&](int c) {
+            float a[4];
+            up();
+            load(pa + 16 * c, true, a);
+            load(pr + 16 * c, base + 16 * c - 15 < S, g[0]);
+#pragma unroll
+            for (int n = 0; n < TB; ++n) {
+                if (c < lo(n) || c >= hi(n)) continue;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) F::mac(acc[n], a[i], g[n][i]);
+            }
+        };
+        int c = 0;
+        for (; c < min(all_lo, groups); ++c) some(c);
+        if (c < all_hi) {
+            // the next group's fragments load while this one's products run
+            float a[4], an[4], gn[4];
+            load(pa + 16 * c, true, a);
+            load(pr + 16 * c, true, gn);
+            for (; c < all_hi; ++c) {
+                up();
+#pragma unroll
+                for (int i = 0; i < 4; ++i) g[0][i] = gn[i];
+                const int d = min(c + 1, all_hi - 1);
+                load(pa + 16 * d, true, an);
+                load(pr + 16 * d, true, gn);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int n = 0; n < TB; ++n) F::mac(acc[n], a[i], g[n][i]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) a[i] = an[i];
+            }
+        }
+        for (; c < groups; ++c) some(c);
+    }
+}
+
+template <class T, int TB>
+__global__ __launch_bounds__(256, 3) void cross_corr_mm_kernel(const T* __restrict__ pics, const T* __restrict__ ref,
+                                                               T* __restrict__ res, size2 size, size2 res_size,
+                                                               uint32_t nb, uint32_t npat, mm_shape m,
+                                                               uint32_t n_wg) {
+    using F = mm_frag<T>;
+    constexpr int NJ = F::NJ, TX = NJ * TB, NT = 256;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    T* prow = reinterpret_cast<T*>(smem_raw);  // prows pattern rows, then one zero row
+    T* zrow = prow + (size_t)m.prows * m.pitch;
+    T* rrow = zrow + m.pitch;                  // cy reference rows between zeros
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int S = (int)size.x, SY = (int)size.y;
+    const int rx = (int)(res_size.x - 1) / 2, ry = (int)(res_size.y - 1) / 2;
+    // the workgroups of one slice, then the patterns of one ROI, run back to back on one XCD
+    const uint32_t L = xcd_remap(blockIdx.x, n_wg);
+    const uint32_t per = (uint32_t)(m.nxb * m.nyb), slab = L / per, in = L - slab * per;
+    const uint32_t roi = slab / npat, sn = (slab - roi * npat) * nb + roi;
+    // workgroups that start together on one CU (32 CUs apart in this order) and waves on one
+    // SIMD take different y-shift bands: the central ones are several times longer
+    const uint32_t turn = slab + (slab >> 4);
+    const uint32_t in_t = (in + turn) % per;
+    const int yb = (int)(in_t / (uint32_t)m.nxb), xb = (int)in_t - yb * m.nxb;
+    const T* p = pics + (size_t)sn * size.area();
+    const T* q = ref + (size_t)roi * size.area();
+
+    const int wv = (wave + (int)(turn / per)) & 3;
+    const int wxi = wv % m.wx, wyi = wv / m.wx;
+    const int sy0g = yb * kMmTY * m.wy - ry;       // first y-shift of the workgroup
+    const int sy0 = sy0g + kMmTY * wyi;            // and of the wave
+    int s0[2];                                     // first x-shift of the wave's tiles
+    bool on[2];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        const int ti = xb * m.wx * m.ntw + wxi + w * m.wx;
+        on[w] = w < m.ntw && ti < m.ntx && yb * m.wy + wyi < m.nty;
+        s0[w] = m.x0 + TX * ti;
+    }
+    const int arow = lane % 16, k = lane / 16, j = F::col(lane);
+
+    for (int e = tid; (size_t)e * sizeof(T) < m.lds; e += NT) prow[e] = T(0);
+    // staging: element e = tid + NT i lies in row e / S, column e % S
+    const int row0 = tid / S, col0 = tid % S, drow = NT / S, dcol = NT % S;
+
+    typename F::acc acc[2][TB];
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+        for (int n = 0; n < TB; ++n) acc[w][n] = typename F::acc{};
+    bool bad = false;
+
+    const int y_lo = max(0, -(sy0g + kMmTY * m.wy - 1)), y_hi = min(SY, SY - sy0g);
+    for (int yc = y_lo; yc < y_hi; yc += m.cy) {
+        const int ye = min(y_hi, yc + m.cy);
+        const int Ya = max(0, yc + sy0g), Yb = min(SY, ye - 1 + sy0g + kMmTY * m.wy);
+        __syncthreads();
+        constexpr int V = 8;  // loads in flight per thread
+        auto stage = [&](const T* src, int rows, T* dst, int pitch) {
+            const int n = rows * S;
+            int col = col0, at = row0 * pitch + col0;  // of element e: e % S and its LDS place
+            for (int e0 = tid; e0 < n; e0 += NT * V) {
+                T v[V];
+#pragma unroll
+                for (int i = 0; i < V; ++i) v[i] = src[min(e0 + i * NT, n - 1)];
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    bad |= mm_not_finite(v[i]);
+                    if (e0 + i * NT < n) dst[at] = v[i];
+                    const bool wrap = col + dcol >= S;
+                    col += dcol - (wrap ? S : 0);
+                    at += drow * pitch + dcol + (wrap ? pitch - S : 0);
+                }
+            }
+        };
+        stage(p + (size_t)Ya * S, Yb - Ya, prow, m.pitch);
+        stage(q + (size_t)yc * S, ye - yc, rrow + m.padl, m.rpitch);
+        __syncthreads();
+        auto pa_of = [&](int y) {
+            const int Y = y + sy0 + arow;
+            return ((unsigned)Y < (unsigned)SY ? prow + (Y - Ya) * m.pitch : zrow) + k;
+        };
+        auto pr_of = [&](int y) { return rrow + (y - yc) * m.rpitch + m.padl + k - j; };
+#pragma unroll
+        for (int w = 0; w < 2; ++w)
+            if (on[w])
+                mm_tile<TB>(acc[w], max(yc, -(sy0 + kMmTY - 1)), min(ye, SY - sy0), pa_of, pr_of, s0[w], S);
+    }
+
+    T* out = res + (size_t)sn * res_size.area();
+    if (__syncthreads_or(bad)) {
+        const int nx = TX * m.wx * m.ntw, x0 = m.x0 + nx * xb;
+        for (int e = tid; e < nx * kMmTY * m.wy; e += NT) {
+            const int sx = x0 + e % nx, sy = sy0g + e / nx;
+            if (sx < -rx || sx + rx >= (int)res_size.x || sy + ry >= (int)res_size.y) continue;
+            T sum = 0;
+            for (int y = max(-sy, 0); y < min(SY, SY - sy); ++y)
+                for (int x = max(-sx, 0); x < min(S, S - sx); ++x)
+                    sum = mac<T>(p[(size_t)(y + sy) * S + x + sx], q[(size_t)y * S + x], sum);
+            out[(size_t)(sy + ry) * res_size.x + sx + rx] = sum;
+        }
+        return;
+    }
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        if (!on[w]) continue;
+#pragma unroll
+        for (int n = 0; n < TB; ++n) {
+            const int sx = s0[w] + NJ * n + j;
+            if (sx < -rx || sx + rx >= (int)res_size.x) continue;
+#pragma unroll
+            for (int r = 0; r < F::REGS; ++r) {
+                const int sy = sy0 + F::row(lane, r);
+                if (sy + ry < (int)res_size.y) out[(size_t)(sy + ry) * res_size.x + sx + rx] = F::get(acc[w][n], r);
+            }
+        }
+    }
+}
+
+// Workgroups of the register-blocked kernel for this launch, or 0 where it does not run
+// (shape outside the tiled limits, or fewer workgroups than CUs, where the finer grids of
+// the other vector kernels are faster).
 template <class T>
 uint64_t tiled_workgroups(size2 size, size2 res_size, uint32_t ref_slices, uint32_t batch, tiled_shape& sh) {
     if (!tiled_plan<T>(size, res_size, sh)) return 0;
@@ -347,13 +737,20 @@ uint64_t tiled_workgroups(size2 size, size2 res_size, uint32_t ref_slices, uint3
     return (n_wg >= 256 && n_wg <= (1u << 24)) ? n_wg : 0;
 }
 
+// Workgroups of the matrix-core kernel, or 0 when the thread-per-shift kernel runs instead
+// (slices too wide for its LDS rows).
+template <class T>
+uint64_t mm_workgroups(size2 size, size2 res_size, uint32_t ref_slices, uint32_t batch, mm_shape& m) {
+    const uint64_t total = (uint64_t)ref_slices * batch;
+    const uint64_t n = mm_plan<T>(size, res_size, total, m) ? total * m.nxb * m.nyb : 0;
+    return n <= 0x7fffffffu ? n : 0;
+}
+
 const char* cross_corr_kernel_name(bool is_double, size2 size, size2 res_size, uint32_t ref_slices, uint32_t batch) {
-    tiled_shape sh;
-    const uint64_t n = is_double ? tiled_workgroups<double>(size, res_size, ref_slices, batch, sh)
-                                 : tiled_workgroups<float>(size, res_size, ref_slices, batch, sh);
-    if (n) return "cross_corr_tiled_kernel";
-    const size_t xn = is_double ? xn_lds_elems<double>(size) * sizeof(double) : xn_lds_elems<float>(size) * sizeof(float);
-    return xn <= kBruteLds ? "cross_corr_x8_kernel" : "cross_corr_kernel";
+    mm_shape m;
+    const uint64_t n = is_double ? mm_workgroups<double>(size, res_size, ref_slices, batch, m)
+                                 : mm_workgroups<float>(size, res_size, ref_slices, batch, m);
+    return n ? "cross_corr_mm_kernel" : "cross_corr_kernel";
 }
 
 template <class T>
@@ -364,24 +761,47 @@ void launch_cross_corr(const T* pics, const T* ref, T* res, size2 size, size2 re
     const uint32_t total = ref_slices * batch;
     if (total == 0 || res_size.area() == 0) return;
     tiled_shape sh;
-    if (const uint64_t n_wg = tiled_workgroups<T>(size, res_size, ref_slices, batch, sh)) {
-        auto kern = cross_corr_tiled_kernel<T>;
-        static const hipError_t attr =
-            hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-        EMIDA_HIP(attr);
-        kern<<<(uint32_t)n_wg, 64 * sh.wx * sh.wy, sh.lds, st>>>(pics, ref, res, size, res_size, ref_slices, batch,
-                                                                   sh, (uint32_t)n_wg);
-        EMIDA_LAUNCHED("cross_corr_tiled_kernel");
-        return;
+    const uint64_t n_tiled = tiled_workgroups<T>(size, res_size, ref_slices, batch, sh);
+    // more slices than a grid's z extent only where the register-blocked rule holds
+    if (!n_tiled && total > 65535u) throw arg_error("cross_corr: more than 65535 slices in one launch");
+    if constexpr (std::is_floating_point<T>::value) {
+        mm_shape m;
+        if (const uint64_t n_wg = mm_workgroups<T>(size, res_size, ref_slices, batch, m)) {
+            auto launch = [&](auto tb) {
+                auto kern = cross_corr_mm_kernel<T, decltype(tb)::value>;
+                static const hipError_t attr =
+                    hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 155648);
+                EMIDA_HIP(attr);
+                kern<<<(uint32_t)n_wg, 256, m.lds, st>>>(pics, ref, res, size, res_size, ref_slices, batch, m,
+                                                         (uint32_t)n_wg);
+                EMIDA_LAUNCHED("cross_corr_mm_kernel");
+            };
+            constexpr int NJ = mm_frag<T>::NJ;
+            if (m.tb == 32 / NJ) launch(std::integral_constant<int, 32 / NJ>{});
+            else if (m.tb == 16 / NJ) launch(std::integral_constant<int, 16 / NJ>{});
+            else if constexpr (NJ == 16) launch(std::integral_constant<int, 3>{});
+            return;
+        }
     }
-    if (total > 65535u) throw arg_error("cross_corr: more than 65535 slices in one launch");
-    if (xn_lds_elems<T>(size) * sizeof(T) <= kBruteLds) {
-        dim3 block(kXNTX, kXNTY);
-        dim3 grid(div_up(res_size.x, (uint32_t)(kXNTX * kXN)), div_up(res_size.y, (uint32_t)kXNTY), total);
-        cross_corr_x8_kernel<T><<<grid, block, xn_lds_elems<T>(size) * sizeof(T), st>>>(pics, ref, res, size,
-                                                                                        res_size, ref_slices);
-        EMIDA_LAUNCHED("cross_corr_x8_kernel");
-        return;
+    if constexpr (!std::is_floating_point<T>::value) {
+        if (const uint64_t n_wg = n_tiled) {
+            auto kern = cross_corr_tiled_kernel<T>;
+            static const hipError_t attr =
+                hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+            EMIDA_HIP(attr);
+            kern<<<(uint32_t)n_wg, 64 * sh.wx * sh.wy, sh.lds, st>>>(pics, ref, res, size, res_size, ref_slices,
+                                                                       batch, sh, (uint32_t)n_wg);
+            EMIDA_LAUNCHED("cross_corr_tiled_kernel");
+            return;
+        }
+        if (xn_lds_elems<T>(size) * sizeof(T) <= kBruteLds) {
+            dim3 block(kXNTX, kXNTY);
+            dim3 grid(div_up(res_size.x, (uint32_t)(kXNTX * kXN)), div_up(res_size.y, (uint32_t)kXNTY), total);
+            cross_corr_x8_kernel<T><<<grid, block, xn_lds_elems<T>(size) * sizeof(T), st>>>(pics, ref, res, size,
+                                                                                            res_size, ref_slices);
+            EMIDA_LAUNCHED("cross_corr_x8_kernel");
+            return;
+        }
     }
     dim3 block(kBruteTX, kBruteTY);
     dim3 grid(div_up(res_size.x, (uint32_t)kBruteTX), div_up(res_size.y, (uint32_t)kBruteTY), total);
