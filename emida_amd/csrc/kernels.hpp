@@ -41,6 +41,18 @@ void launch_cross_corr(const T* pics, const T* ref, T* res, size2 size, size2 re
 // Name of the kernel launch_cross_corr picks for this shape (float or double).
 const char* cross_corr_kernel_name(bool is_double, size2 size, size2 res_size, uint32_t ref_slices, uint32_t batch);
 
+// Most patterns per launch for which the refined matrix-core policy is run as the brute
+// policy (the same results): the screen's tiles hold 32 patterns and cost the same for one,
+// the brute kernel's cost grows with each.  Brute / screen and refinement, us, 400 ROIs, in
+// double: 32 x 32 one pattern 67 / 210, 4: 157 / 235, 8: 284 / 255; 64 x 64 2: 829 / 894,
+// 4: 1503 / 934; 128 x 128 one: 4267 / 7052, 2: 8045 / 7139; in float 64 x 64 2: 644 / 892,
+// 4: 1141 / 932; 128 x 128 2: 5581 / 7125.  25 and 100 ROIs cross over at the same counts or
+// above.
+inline uint32_t mfma_direct_patterns(bool is_double, size2 size) {
+    const uint32_t n = (uint32_t)(128.0 / std::sqrt((double)size.area()));
+    return is_double ? n : n + 1;
+}
+
 // ---- peak.hip
 // Offsets of the least-squares tables for fitsize 3, 5, 7, 9 in the device table.
 int lstsq_offset(int fit);

@@ -152,7 +152,7 @@ struct emida_offset_s {
     void* d_sums = nullptr;
     void* d_ref = nullptr;     // brute: prepared reference slices; FFT: spectra
     void* d_slices = nullptr;  // brute: prepared pattern slices
-    void* d_corr = nullptr;    // brute: correlation buffers
+    void* d_corr = nullptr;    // brute (and refined matrix-core launches of few patterns): correlation buffers
     emida_mfma_mode mfma_mode = EMIDA_MFMA_AUTO;  // as set; mfma_mode_used() is the one in effect
     bool mfma_refine = true;   // matrix-core policy: exact peak from T-precision values
     void* d_ref_lo = nullptr;  // matrix-core policy: lo halves of the reference slices
@@ -218,6 +218,7 @@ struct emida_offset_s {
         void* cnt = nullptr;
         void* ent = nullptr;
         void* pn2 = nullptr;
+        uint32_t direct = 0;  // patterns whose correlation buffers fit corr (mfma_direct)
     };
     static constexpr int kParts = 9;
     static size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -249,6 +250,10 @@ struct emida_offset_s {
         for (int i = 0; i < kParts; ++i) sum += parts[i];
         return sum;
     }
+    // Launches of up to this many patterns run the brute kernels (refined matrix-core policy).
+    uint32_t mfma_direct() const {
+        return policy == EMIDA_CROSS_POLICY_BRUTE_MFMA && mfma_refine ? mfma_direct_patterns(T == EMIDA_F64, slice) : 0;
+    }
     size_t scratch_bytes(uint32_t n_pat) const {
         size_t parts[kParts];
         return scratch_sizes(n_pat, parts);
@@ -262,12 +267,19 @@ struct emida_offset_s {
             ptr[i] = parts[i] ? b : nullptr;
             b += parts[i];
         }
-        return {ptr[0], ptr[1], ptr[2], ptr[3], ptr[4], ptr[5], ptr[6], ptr[7], ptr[8]};
+        scratch_t sc{ptr[0], ptr[1], ptr[2], ptr[3], ptr[4], ptr[5], ptr[6], ptr[7], ptr[8]};
+        if (const uint32_t n = mfma_direct()) {
+            // a launch of few patterns leaves the candidate lists unused: its correlation
+            // buffers take their place, as many as fit (so the scratch does not grow)
+            sc.corr = sc.ent;
+            sc.direct = (uint32_t)std::min<size_t>(n, parts[7] / ((size_t)nb * cross.area() * t_bytes()));
+        }
+        return sc;
     }
     const void* float_hx() const { return d_hxf ? d_hxf : d_hx; }
     const void* float_hy() const { return d_hyf ? d_hyf : d_hy; }
     scratch_t own_scratch() const {
-        return {d_sums, d_slices, d_corr, d_pic_hi, d_pic_lo, d_smax, d_cnt, d_ent, d_pn2};
+        return {d_sums, d_slices, d_corr, d_pic_hi, d_pic_lo, d_smax, d_cnt, d_ent, d_pn2, std::min(batch, mfma_direct())};
     }
 
     size_t ti_bytes() const { return T == EMIDA_F32 ? 8 : 16; }
@@ -475,6 +487,8 @@ struct emida_offset_s {
                     d_cnt = alloc(scratch_total * cross.y * sizeof(uint32_t));
                     d_ent = alloc(scratch_total * cross.y * kListCap * sizeof(cand_entry));
                     d_pn2 = alloc(scratch_total * 2 * sizeof(double));  // norms, then zero-shift products
+                    const size_t direct = (size_t)nb * std::min(batch, mfma_direct());
+                    if (direct) d_corr = alloc(direct * cross.area() * t_bytes());
                 } else {
                     d_corr = alloc(scratch_total * cross.area() * sizeof(float));
                 }
@@ -608,6 +622,7 @@ struct emida_offset_s {
     void run(const void* d_pics, uint32_t n_pat, void* maxes, void* neigh, double* offsets, double* coefs,
              const scratch_t& sc, hipStream_t st) {
         const uint32_t tn = nb * n_pat;
+        const bool direct = n_pat <= sc.direct;  // refined matrix-core policy, few patterns
         hipEvent_t t0 = nullptr, t1 = nullptr;
         with_T(T, [&](auto t) {
             using TT = decltype(t);
@@ -616,7 +631,8 @@ struct emida_offset_s {
                 using ST = decltype(sm);
                 const IT* pics = (const IT*)d_pics;
                 ST* sums = (ST*)sc.sums;
-                if (policy == EMIDA_CROSS_POLICY_BRUTE) {
+                if (policy == EMIDA_CROSS_POLICY_BRUTE || direct) {
+                    const TT* ref = (const TT*)(direct ? d_ref_t : d_ref);
                     if (!fused_prepare<IT, ST, TT, _Float16>(pics, sums, (TT*)sc.slices, nullptr, nullptr, nullptr, tn,
                                                              st)) {
                         launch_sum<IT, ST>(pics, sums, d_begins, src, slice, nb, tn, st);
@@ -624,8 +640,7 @@ struct emida_offset_s {
                                                    d_begins, src, slice, slice, nb, tn, st);
                     }
                     if (timing) t0 = record_start(st);
-                    launch_cross_corr<TT>((const TT*)sc.slices, (const TT*)d_ref, (TT*)sc.corr, slice, cross, nb, n_pat,
-                                          st);
+                    launch_cross_corr<TT>((const TT*)sc.slices, ref, (TT*)sc.corr, slice, cross, nb, n_pat, st);
                     if (timing) record_stop(st, t0);
                     launch_peak<TT>((const TT*)sc.corr, (size_t)tn * cross.area(), cross.area(), cross, POLICY_BRUTE,
                                     fit, (data_index<TT>*)maxes, (TT*)neigh, offsets, coefs, tn, st);
