@@ -8,6 +8,7 @@
 // double without contraction in the reference's order, so it matches the CPU
 // result bit for bit.
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "kernels.hpp"
@@ -301,8 +302,9 @@ __global__ void subpixel_kernel(const T* __restrict__ neigh, int s, uint32_t n, 
 // without a finite screen maximum is swept whole: every shift of the window is
 // evaluated exactly, box by box, so its arg-max is the brute policy's as well.
 constexpr int kRefineCap = 512;
-constexpr int kSweepRows = 8;  // sweep boxes: kSweepRows x kBoxW shifts (one per thread)
-constexpr int kRefineNT = 256;
+// Boxes tried on candidates too wide for one before the rest are evaluated one chain per
+// lane (128 x 128 double slices: a box 0.05 to 0.1 ms, a round of chains 0.7 ms).
+constexpr int kSpreadBoxes = 6;
 constexpr int kRowList = 256;  // screens of at most this many rows use the row maxima
 
 template <class T>
@@ -343,85 +345,186 @@ __device__ inline T exact_at(size_t g, size_t corr_len, const T* p, const T* r, 
     return exact_corr<T>(p + (size_t)sn * a, r + (size_t)(sn % nb) * a, s, sx, sy);
 }
 
-// Exact values of a box of shifts of one slice, all threads of the workgroup
-// together: thread t < bw * bh takes position (x0 + t % bw, y0 + t / bw) of the cross
-// buffer (shift = position - (cross - 1) / 2).  The lanes of a wave walk the union of the
-// box's overlaps in lockstep (y outer, x inner): chunks of kBoxY rows of the pattern
-// slice are staged in LDS with zeros wherever a shift leaves the slice (row stride
-// below), every lane takes the same x at each step, and the reference value of that
-// step is the same for every lane, read through the scalar unit; LDS serves one
-// operand per fma.  The terms a lane adds outside its own overlap are exact zeros
-// (fma(0, r, acc) == acc for finite values, and the accumulator is never -0), so each
-// value equals exact_corr's bit for bit.  LDS: kBoxY + kBoxRows - 1 rows of
-// box_stride(s.x + kBoxW - 1), which also holds the box values afterwards; boxes of at
-// most 14 rows keep it at 23 KB for 128-wide double slices.
-constexpr int kBoxRows = 14;
-constexpr int kBoxW = 32;
-constexpr int kBoxY = 4;
-static_assert(kSweepRows * kBoxW <= kRefineNT && kSweepRows <= kBoxRows, "sweep box exceeds a box evaluation");
-
-// Row stride of the allocation (elements): the smallest stride >= sx congruent to 9 mod
-// 32.  A box whose conflict-free stride does not fit it falls back to this stride, on
-// which consecutive box rows start 18 banks apart (at most 2-way conflicts).
-__host__ __device__ constexpr int box_stride(int sx) { return sx + ((9 - sx % 32) + 32) % 32; }
-
-template <class T, int NT>
-__device__ inline void eval_box(const T* __restrict__ p, const T* __restrict__ r, size2 s, size2 cross, int x0,
-                                int y0, int bw, int bh, T* prow, T* out) {
-    const int tid = threadIdx.x, S = (int)s.x, SY = (int)s.y;
-    const int rx = (int)(cross.x - 1) / 2, ry = (int)(cross.y - 1) / 2;
-    const int sx_lo = x0 - rx, sy_lo = y0 - ry;  // shift range of the box
-    const int sx_hi = sx_lo + bw - 1, sy_hi = sy_lo + bh - 1;
-    const int xlo = max(0, -sx_hi), xhi = min(S, S - sx_lo);  // union of the overlaps
-    const int ylo = max(0, -sy_hi), yhi = min(SY, SY - sy_lo);
-    const int cw = xhi - xlo + bw - 1, c0 = xlo + sx_lo;  // staged columns, first one
-    // a row stride congruent to bw modulo the 32 banks of 4 bytes makes the addresses of
-    // a step, row * PS + column for position t = row * bw + column, consecutive modulo
-    // the banks, so a step's reads are free of bank conflicts (refining 128x128 double
-    // slices, the fallback stride cost 4.9 conflict cycles per LDS instruction, this 0.02)
-    constexpr int kSweep = 128 / (int)sizeof(T);
-    const int PSc = cw + ((bw - cw) % kSweep + kSweep) % kSweep;
-    const int PS = PSc <= box_stride(S + kBoxW - 1) ? PSc : box_stride(cw);
-    const int n = bw * bh;
-    const bool wave_on = tid - tid % kWave < n;  // waves with no position skip the sums
-    const int t = min(tid, n - 1), lx = t % bw, ly = t / bw;
-    T acc = 0;
-    for (int yc = ylo; yc < yhi; yc += kBoxY) {
-        const int ny = min(kBoxY, yhi - yc);
-        __syncthreads();
-        for (int e = tid; e < (ny + bh - 1) * cw; e += NT) {
-            const int j = e / cw, cc = e % cw, c = cc + c0, Y = yc + sy_lo + j;
-            prow[j * PS + cc] = (Y >= 0 && Y < SY && c >= 0 && c < S) ? p[(size_t)Y * S + c] : T(0);
-        }
-        __syncthreads();
-        if (!wave_on) continue;
-        for (int k = 0; k < ny; ++k) {
-            const T* pr = prow + (k + ly) * PS + lx - xlo;  // pr[x] = pattern (y + sy, x + sx)
-            // the reference row is the same for every lane: read through the scalar unit
-            // (before, a v_readlane pair per product broadcast it from the lane holding it)
-            const T* rr = r + (size_t)(yc + k) * S;
-            int x = xlo;
-            // the operands of 8 products are loaded before their 8 dependent fmas
-            for (; x + 8 <= xhi; x += 8) {
-                T u[8], q[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    u[i] = pr[x + i];
-                    q[i] = rr[x + i];
-                }
-#pragma unroll
-                for (int i = 0; i < 8; ++i) acc = fma(u[i], q[i], acc);
-            }
-            for (; x < xhi; ++x) acc = fma(pr[x], rr[x], acc);
-        }
-    }
-    __syncthreads();  // out may alias the staged rows
-    if (tid < n) out[tid] = acc;
-    __syncthreads();
+// Orders a wave's LDS accesses.
+__device__ __forceinline__ void box_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <class T, int NT>
-__global__ __launch_bounds__(NT) void refine_kernel(const float* __restrict__ screen, size_t corr_len,
+// Exact values of a box of up to kBoxRows x kBoxW shifts of one slice, by one wave on the
+// matrix cores, in the brute order: v_mfma_f64_4x4x4 and v_mfma_f32_16x16x4 round like a chain
+// of fused multiply-adds over ascending k that starts at the accumulator, so one accumulator
+// per shift fed with the pattern columns in order, reference row after reference row, gives
+// exact_corr's bits.  The rows of A are the 16 y-shifts, the columns of B the x-shifts
+// (the Toeplitz matrix of the reference row); terms outside a shift's overlap multiply an
+// exact zero (finite values).
+//
+// A reference row moves the 16 pattern rows by one.  They stay in registers (lane l holds
+// columns l / 16 + 4 t of the row Y with Y mod 16 = l % 16); each step loads the one new row
+// into the lanes of the one that left, and the accumulators, which belong to y-shifts, move
+// to the next row of D instead.  Only the reference row passes through LDS (one row per
+// buffer, zeros around it).  That leaves a wave its own LDS of 13 KB and 12 waves on a CU;
+// pattern rows staged in LDS (one shift per lane, vector FMAs, waves waiting on LDS 77% of
+// the time) took 5.5 ms for 12,800 slices of 128 x 128 in double where this takes 1.95 ms.
+constexpr int kBoxRows = 16;
+constexpr int kBoxW = 32;
+constexpr int kRowBuf = 192;  // elements of a reference row buffer
+
+template <class T>
+struct box_frag;
+template <>
+struct box_frag<double> {
+    using acc = double;
+    static constexpr int NJ = 4, REGS = 1;
+    static __device__ __forceinline__ void mac(acc& c, double a, double b) {
+        c = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ double get(const acc& c, int) { return c; }
+    // lane l holds D[4 ((l % 16) / 4) + l / 16][l % 4]
+    static __device__ __forceinline__ int row(int lane, int) { return 4 * (lane % 16 / 4) + lane / 16; }
+    static __device__ __forceinline__ int col(int lane) { return lane % 4; }
+    // every row of D becomes the next one's (15 becomes 0's)
+    static __device__ __forceinline__ void turn(acc& c, int lane) {
+        const int m = (row(lane, 0) + 15) & 15;
+        c = __shfl(c, 16 * (m & 3) + 4 * (m >> 2) + lane % 4);
+    }
+};
+typedef float box_f4 __attribute__((ext_vector_type(4)));
+template <>
+struct box_frag<float> {
+    using acc = box_f4;
+    static constexpr int NJ = 16, REGS = 4;
+    static __device__ __forceinline__ void mac(acc& c, float a, float b) {
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ float get(const acc& c, int r) { return c[r]; }
+    // lane l, register r holds D[4 (l / 16) + r][l % 16]
+    static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane / 16) + r; }
+    static __device__ __forceinline__ int col(int lane) { return lane % 16; }
+    static __device__ __forceinline__ void turn(acc& c, int lane) {
+        const float up = __shfl(c[3], (lane + 48) & 63);
+        c = box_f4{up, c[0], c[1], c[2]};
+    }
+};
+
+// Shifts [sx0, sx0 + NJ NF) x [sy0, sy0 + 16) over the reference rows [y0, y1); KS column
+// steps of 4 cover the slice (S a multiple of 8, at most 4 KS).  out: [16][kBoxW].
+template <class T, int KS, int NF>
+__device__ __forceinline__ void box_sums(const T* __restrict__ p, const T* __restrict__ r, int S, int SY, int sx0,
+                                         int sy0, int y0, int y1, T* rbuf, T* out) {
+    using F = box_frag<T>;
+    constexpr int NJ = F::NJ, SH = NJ / 4, SPAN = NJ * NF - 1, PER = kRowBuf / kWave;
+    constexpr int GS = KS < 8 ? KS : 8;
+    static_assert(4 * KS + SPAN <= kRowBuf, "reference row buffer");
+    const int lane = threadIdx.x % kWave, i = lane % 16, k = lane / 16, j = F::col(lane);
+    // groups of GS steps that hold terms of the box
+    const int g0 = max(0, sx0) / (4 * GS), g1 = (min(S, S + sx0 + SPAN) + 4 * GS - 1) / (4 * GS);
+    typename F::acc acc[NF];
+#pragma unroll
+    for (int n = 0; n < NF; ++n) acc[n] = typename F::acc{};
+    T a[KS];
+    {
+        const int Yb = y0 + sy0, Y = Yb + ((i - Yb) & 15);
+        const bool in = Y >= 0 && Y < SY;
+        const T* src = p + (size_t)(in ? Y : 0) * S + k;
+#pragma unroll
+        for (int t = 0; t < KS; ++t) a[t] = in && 4 * t < S ? src[4 * t] : T(0);
+    }
+    // element e of the row buffer: reference column e - (SPAN + sx0)
+    T next[PER];
+    auto fetch = [&](int y) {
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int c = lane + kWave * q - (SPAN + sx0);
+            const bool in = c >= 0 && c < S;
+            const T v = r[(size_t)y * S + (in ? c : 0)];
+            next[q] = in ? v : T(0);
+        }
+    };
+    auto put = [&](int y) {
+#pragma unroll
+        for (int q = 0; q < PER; ++q) rbuf[(y & 1) * kRowBuf + lane + kWave * q] = next[q];
+        box_sync();
+    };
+    if (y0 < y1) {
+        fetch(y0);
+        put(y0);
+    }
+    for (int y = y0; y < y1; ++y) {
+        fetch(min(y + 1, y1 - 1));
+        const T* rb = rbuf + (y & 1) * kRowBuf + k - j + SPAN;
+        const int Yn = y + sy0 + 16;  // the row that takes the place of y + sy0
+        const bool take = ((Yn - i) & 15) == 0, in = Yn >= 0 && Yn < SY;
+        const T* src = p + (size_t)(in ? Yn : 0) * S + k;
+#pragma unroll
+        for (int g = 0; g < KS / GS; ++g) {
+            if (g < g0 || g >= g1) continue;
+            constexpr int LEAD = SH * (NF - 1);
+            T b[GS + LEAD];
+#pragma unroll
+            for (int u = 0; u < GS + LEAD; ++u) b[u] = rb[4 * (GS * g + u - LEAD)];
+#pragma unroll
+            for (int tt = 0; tt < GS; ++tt)
+#pragma unroll
+                for (int n = 0; n < NF; ++n) F::mac(acc[n], a[GS * g + tt], b[tt + LEAD - SH * n]);
+            if (take) {
+#pragma unroll
+                for (int tt = 0; tt < GS; ++tt) {
+                    const int t = GS * g + tt;
+                    a[t] = in && 4 * t < S ? src[4 * t] : T(0);
+                }
+            }
+        }
+        put(y + 1);
+#pragma unroll
+        for (int n = 0; n < NF; ++n) F::turn(acc[n], lane);
+    }
+#pragma unroll
+    for (int n = 0; n < NF; ++n)
+#pragma unroll
+        for (int q = 0; q < F::REGS; ++q)
+            out[((F::row(lane, q) - y1 - sy0) & 15) * kBoxW + NJ * n + j] = F::get(acc[n], q);
+    box_sync();
+}
+
+// Exact values of positions [x0, x0 + bw) x [y0, y0 + bh) of the cross buffer (shift =
+// position - (cross - 1) / 2) into out[row * kBoxW + column]; bw <= kBoxW, bh <= kBoxRows.
+// All NT threads of the workgroup call it; with four waves each takes a quarter of the
+// columns (rbuf: two row buffers per wave).
+template <class T, int NT, int KS>
+__device__ __forceinline__ void eval_box(const T* __restrict__ p, const T* __restrict__ r, size2 s, size2 cross,
+                                         int x0, int y0, int bw, int bh, T* rbuf, T* out) {
+    if (bw <= 0 || bh <= 0) return;
+    constexpr int NJ = box_frag<T>::NJ, NW = NT / kWave;
+    const int S = (int)s.x, SY = (int)s.y, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int sx0 = x0 - (int)(cross.x - 1) / 2, sy0 = y0 - (int)(cross.y - 1) / 2;
+    const int ya = max(0, -(sy0 + bh - 1)), yb = max(ya, min(SY, SY - sy0));  // rows with terms of the box
+    if constexpr (NW > 1) __syncthreads();  // out may still be read
+    auto run = [&](auto nf) {
+        constexpr int NF = decltype(nf)::value;
+        const int x = NJ * NF * wv;
+        if (x < bw)
+            box_sums<T, KS, NF>(p, r, S, SY, sx0 + x, sy0, ya, yb, rbuf + 2 * kRowBuf * wv, out + x);
+    };
+    // the fewest fragments that hold the box's columns
+    if constexpr (NJ * NW == 4) {
+        if (bw <= 8) run(std::integral_constant<int, 2>{});
+        else if (bw <= 12) run(std::integral_constant<int, 3>{});
+        else if (bw <= 16) run(std::integral_constant<int, 4>{});
+        else run(std::integral_constant<int, 8>{});
+    } else if constexpr (NJ * NW == 16) {
+        if (bw <= 16) run(std::integral_constant<int, 1>{});
+        else run(std::integral_constant<int, 2>{});
+    } else {
+        run(std::integral_constant<int, 1>{});
+    }
+    if constexpr (NW > 1) __syncthreads();
+}
+
+// NT = 64: one wave per slice; 256: four.  KS column steps of 4 cover the slice width.
+template <class T, int NT, int KS>
+__global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__ screen, size_t corr_len,
                                                     const T* __restrict__ p, const T* __restrict__ r, size2 s,
                                                     size2 cross, uint32_t nb, double tol_rel, double tol_abs,
                                                     int fit, const double* __restrict__ lsq,
@@ -439,11 +542,12 @@ __global__ __launch_bounds__(NT) void refine_kernel(const float* __restrict__ sc
     __shared__ T nbv[81];
     __shared__ double cf[6];
     __shared__ int bb[4];
-    extern __shared__ __align__(16) unsigned char refine_lds[];
-    T* prow = reinterpret_cast<T*>(refine_lds);  // staged pattern rows of eval_box
-    T* boxv = prow;  // the box values eval_box leaves (over the staged rows)
-    const uint32_t sn = blockIdx.x;
-    if (sn >= total) return;
+    __shared__ T rbuf[NT / kWave * 2 * kRowBuf];  // reference rows of eval_box
+    __shared__ T boxv[kBoxRows * kBoxW];          // the box values it leaves
+    if (blockIdx.x >= total) return;
+    // the patterns of one ROI run back to back on one XCD (one reference slice in its L2)
+    const uint32_t L = xcd_remap(blockIdx.x, total), npat = total / nb;
+    const uint32_t sn = (L % npat) * nb + L / npat;
     const int tid = threadIdx.x;
     const uint32_t area = cross.area();
     const size_t a = (size_t)s.x * s.y;
@@ -598,64 +702,100 @@ __global__ __launch_bounds__(NT) void refine_kernel(const float* __restrict__ sc
     }
     __syncthreads();
     const int k = fit * fit, rad = (fit - 1) / 2;
-    // One box evaluation when the candidates' box grown by the fit radius fits the
-    // workgroup: it holds every candidate and the in-window neighbourhood of any of
-    // them (the chains of one box run side by side; a second box would run after).
+    // One box when the candidates' box grown by the fit radius fits: it holds every candidate
+    // and the in-window neighbourhood of any of them.  Else one box of the candidates; else
+    // (spread candidates) boxes of 16 x 16 around the first one left, and after a few of them
+    // one chain per lane for the rest; a swept slice takes the whole window in boxes.
     const int cbw = bb[2] - bb[0] + 1, cbh = bb[3] - bb[1] + 1;
     const int ex0 = max(0, bb[0] - rad), ey0 = max(0, bb[1] - rad);
     const int ebw = min((int)cross.x - 1, bb[2] + rad) - ex0 + 1, ebh = min((int)cross.y - 1, bb[3] + rad) - ey0 + 1;
-    const bool merged = !sweep && ebh <= kBoxRows && ebw <= kBoxW && ebw * ebh <= NT;
-    const bool boxed = merged || (!sweep && cbh <= kBoxRows && cbw <= kBoxW && cbw * cbh <= NT);
-    const int bx0 = merged ? ex0 : bb[0], by0 = merged ? ey0 : bb[1], bw = merged ? ebw : cbw;
-    if (boxed) eval_box<T, NT>(ps, rs, s, cross, bx0, by0, bw, merged ? ebh : cbh, prow, boxv);
+    const bool merged = !sweep && ebh <= kBoxRows && ebw <= kBoxW;
+    const bool boxed = merged || (!sweep && cbh <= kBoxRows && cbw <= kBoxW);
     T best = lowest<T>();
     uint32_t bi = 0xffffffffu;
-    for (uint32_t c = tid; c < nc; c += NT) {
-        const uint32_t i = cand[c];
-        const int cx = (int)(i % cross.x), cy = (int)(i / cross.x);
-        const T v = boxed ? boxv[(cy - by0) * bw + (cx - bx0)]
-                          : exact_at<T>((size_t)sn * area + i, corr_len, p, r, s, cross, nb);
+    auto offer = [&](T v, uint32_t i) {
         if (v > best || (v == best && i < bi)) {
             best = v;
             bi = i;
         }
-    }
-    if (sweep) {
-        // the whole window, kSweepRows x kBoxW shifts at a time (one per thread)
-        for (int y0 = 0; y0 < (int)cross.y; y0 += kSweepRows)
-            for (int x0 = 0; x0 < (int)cross.x; x0 += kBoxW) {
-                const int w = min(kBoxW, (int)cross.x - x0), h = min(kSweepRows, (int)cross.y - y0);
-                eval_box<T, NT>(ps, rs, s, cross, x0, y0, w, h, prow, boxv);
-                if (tid < w * h) {
-                    const uint32_t i = (uint32_t)(y0 + tid / w) * cross.x + (uint32_t)(x0 + tid % w);
-                    const T v = boxv[tid];
-                    if (v > best || (v == best && i < bi)) {
-                        best = v;
-                        bi = i;
-                    }
-                }
-                __syncthreads();  // the next box stages over these values
+    };
+    size2 mp{0, 0};
+    int bx0 = 0, by0 = 0, bw = 0, bh = 0, spread = 0;
+    enum { CANDIDATES, SWEEP, PEAK };
+    for (int mode = sweep ? SWEEP : CANDIDATES;;) {
+        if (mode == CANDIDATES) {
+            if (boxed) {
+                bx0 = merged ? ex0 : bb[0];
+                by0 = merged ? ey0 : bb[1];
+                bw = merged ? ebw : cbw;
+                bh = merged ? ebh : cbh;
+            } else {
+                uint32_t first = 0xffffffffu;
+                for (uint32_t c = tid; c < nc; c += NT) first = min(first, cand[c]);
+                first = block_min_u32<NT>(first, si);
+                bx0 = max(0, (int)(first % cross.x) - 8);
+                by0 = (int)(first / cross.x);
+                bw = min(16, (int)cross.x - bx0);
+                bh = min(16, (int)cross.y - by0);
             }
+        } else if (mode == SWEEP) {
+            bw = min(kBoxW, (int)cross.x - bx0);
+            bh = min(kBoxRows, (int)cross.y - by0);
+        } else {
+            bx0 = max(0, (int)mp.x - rad);
+            by0 = max(0, (int)mp.y - rad);
+            bw = min((int)cross.x - 1, (int)mp.x + rad) - bx0 + 1;
+            bh = min((int)cross.y - 1, (int)mp.y + rad) - by0 + 1;
+        }
+        eval_box<T, NT, KS>(ps, rs, s, cross, bx0, by0, bw, bh, rbuf, boxv);
+        if (mode == PEAK) break;
+        if (mode == CANDIDATES) {
+            uint32_t left = 0;
+            for (uint32_t c = tid; c < nc; c += NT) {
+                const uint32_t i = cand[c];
+                if (i == 0xffffffffu) continue;
+                const int x = (int)(i % cross.x) - bx0, y = (int)(i / cross.x) - by0;
+                if (x >= 0 && y >= 0 && x < bw && y < bh) {
+                    offer(boxv[y * kBoxW + x], i);
+                    cand[c] = 0xffffffffu;  // done
+                } else {
+                    ++left;
+                }
+            }
+            if (__syncthreads_or((int)left)) {
+                if (++spread < kSpreadBoxes * (int)div_up(nc, (uint32_t)NT)) continue;
+                for (uint32_t c = tid; c < nc; c += NT) {
+                    const uint32_t i = cand[c];
+                    if (i != 0xffffffffu)
+                        offer(exact_at<T>((size_t)sn * area + i, corr_len, p, r, s, cross, nb), i);
+                }
+            }
+        } else {
+            for (int e = tid; e < bw * bh; e += NT) {
+                const int x = e % bw, y = e / bw;
+                offer(boxv[y * kBoxW + x], (uint32_t)(by0 + y) * cross.x + (uint32_t)(bx0 + x));
+            }
+            bx0 += kBoxW;
+            if (bx0 >= (int)cross.x) {
+                bx0 = 0;
+                by0 += kBoxRows;
+            }
+            if (by0 < (int)cross.y) continue;
+        }
+        block_argmax<T, NT>(best, bi, sv, si);
+        mp = shift_pos(POLICY_BRUTE, bi, cross);
+        if (merged) break;
+        mode = PEAK;
     }
-    block_argmax<T, NT>(best, bi, sv, si);
 
-    // neighbourhood, exact: the in-window part from the merged box or as its own box,
-    // positions the clamp puts one past the window (spilling into the next row or
-    // slice) one chain each
-    const size2 mp = shift_pos(POLICY_BRUTE, bi, cross);
-    int nx0 = bx0, ny0 = by0, nbw = bw;
-    if (!merged) {
-        nx0 = max(0, (int)mp.x - rad);
-        ny0 = max(0, (int)mp.y - rad);
-        nbw = min((int)cross.x - 1, (int)mp.x + rad) - nx0 + 1;
-        const int nbh = min((int)cross.y - 1, (int)mp.y + rad) - ny0 + 1;
-        eval_box<T, NT>(ps, rs, s, cross, nx0, ny0, nbw, nbh, prow, boxv);
-    }
+    // neighbourhood, exact: the in-window part from the last box, positions the clamp puts
+    // one past the window (spilling into the next row or slice) one chain each
     for (int t = tid; t < k; t += NT) {
         const int i = t % fit, j = t / fit;
         const size2 c = clamp_pos((int)mp.x - rad + i, (int)mp.y - rad + j, cross);
-        const T v = (c.x < cross.x && c.y < cross.y)
-                        ? boxv[((int)c.y - ny0) * nbw + ((int)c.x - nx0)]
+        const int x = (int)c.x - bx0, y = (int)c.y - by0;
+        const T v = c.x < cross.x && c.y < cross.y && x >= 0 && y >= 0 && x < bw && y < bh
+                        ? boxv[y * kBoxW + x]
                         : exact_at<T>(pos_index(POLICY_BRUTE, sn, c, cross), corr_len, p, r, s, cross, nb);
         nbv[t] = v;
         if (neigh) neigh[(size_t)sn * k + t] = v;
@@ -720,6 +860,8 @@ void launch_subpixel(const T* neigh, int s, uint32_t n, const data_index<T>* max
     EMIDA_LAUNCHED("subpixel_kernel");
 }
 
+constexpr uint32_t kRefineOneWave = 768;
+
 template <class T>
 void launch_refine(const float* screen, size_t corr_len, const T* p, const T* r, size2 s, size2 cross, uint32_t nb,
                    double tol_rel, double tol_abs, int fit, data_index<T>* maxes, T* neigh, double* offsets,
@@ -732,10 +874,26 @@ void launch_refine(const float* screen, size_t corr_len, const T* p, const T* r,
     if (!lists && !screen) throw arg_error("exact refinement: no screen");
     screen_lists none{};
     const double* lsq = lstsq_device_table() + lstsq_offset(fit);
-    const size_t lds = (size_t)(kBoxY + kBoxRows - 1) * box_stride((int)s.x + kBoxW - 1) * sizeof(T);
-    refine_kernel<T, kRefineNT><<<total, kRefineNT, lds, st>>>(screen, corr_len, p, r, s, cross, nb, tol_rel, tol_abs,
-                                                          fit, lsq, maxes, neigh, offsets, coefs, total,
-                                                          screen_max, lists ? *lists : none);
+    if (nb == 0 || total % nb) throw arg_error("exact refinement: slices must be whole sets of ROIs");
+    if (s.x % 8) throw arg_error("exact refinement needs a slice width that is a multiple of 8");
+    // One wave per slice; four, which split a box's columns and the chains of spread candidates,
+    // where that leaves most SIMDs without a wave (a pass in double at 128 x 128 and 100, 400,
+    // 1,000, 1,600, 6,400 slices: one wave 2.09, 2.12, 2.25, 2.40, 5.95 ms, four 2.04, 2.10,
+    // 2.36, 2.69, 7.10 ms).
+    auto launch = [&](auto ks) {
+        auto go = [&](auto nt) {
+            constexpr int NT = decltype(nt)::value;
+            refine_kernel<T, NT, decltype(ks)::value><<<total, NT, 0, st>>>(
+                screen, corr_len, p, r, s, cross, nb, tol_rel, tol_abs, fit, lsq, maxes, neigh, offsets, coefs, total,
+                screen_max, lists ? *lists : none);
+        };
+        if (total >= kRefineOneWave) go(std::integral_constant<int, kWave>{});
+        else go(std::integral_constant<int, 4 * kWave>{});
+    };
+    if (s.x <= 16) launch(std::integral_constant<int, 4>{});
+    else if (s.x <= 32) launch(std::integral_constant<int, 8>{});
+    else if (s.x <= 64) launch(std::integral_constant<int, 16>{});
+    else launch(std::integral_constant<int, 32>{});
     EMIDA_LAUNCHED("refine_kernel");
 }
 template void launch_refine<float>(const float*, size_t, const float*, const float*, size2, size2, uint32_t, double,
