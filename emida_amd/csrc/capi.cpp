@@ -240,7 +240,7 @@ int emida_offset_get_timing(emida_offset* h, const char** kernel_name, double* t
         h->tev.clear();
         if (kernel_name)
             *kernel_name = h->policy == EMIDA_CROSS_POLICY_FFT
-                               ? (h->fftg ? "fftg_rows_kernel+fftg_cols_kernel+fftg_rows_inv_kernel+peak_kernel"
+                               ? (h->fftg ? "fftg_rows_kernel+fftg_cols_kernel+fftg_rows_inv_kernel"
                                           : fft_padded(h->side) > 128 ? "fft256_kernel" : "fft_kernel")
                                : (h->policy == EMIDA_CROSS_POLICY_BRUTE_MFMA && h->batch > h->mfma_direct()
                                       ? "mfma_corr_kernel"

@@ -202,4 +202,33 @@ __device__ inline uint32_t block_min_u32(uint32_t v, uint32_t* sv) {
     return v;
 }
 
+// ------------------------------------------------------------------ quadratic peak
+// One coefficient: sum_i M[row][i] * nb[i] in double, i ascending
+// (src/subpixel_max.hpp:14-29).
+template <class T>
+__device__ inline double fit_coef(const double* __restrict__ mrow, const T* nb, int k) {
+#pragma clang fp contract(off)
+    double sum = 0;
+    for (int i = 0; i < k; ++i) sum += mrow[i] * (double)nb[i];
+    return sum;
+}
+
+// Peak of the fitted quadratic (src/subpixel_max.hpp:91-92).
+__device__ inline void fit_peak(const double* c, double& ox, double& oy) {
+#pragma clang fp contract(off)
+    const double b = c[1], cc = c[2], d = c[3], e = c[4], f = c[5];
+    oy = (b * e - 2 * cc * d) / (4 * f * d - e * e);
+    ox = (-e * oy - b) / (2 * d);
+}
+
+// Offset formula of finalize (src/gpu_offset.hpp:291-297).
+__device__ inline void finalize_offset(uint32_t index, size2 cross, int policy, int fit, double sx, double sy,
+                                       double& ox, double& oy) {
+#pragma clang fp contract(off)
+    const size2 mp = shift_pos(policy, index, cross);
+    const int r = (fit - 1) / 2;
+    ox = -((int)mp.x - ((int)cross.x / 2) - r + sx);
+    oy = -((int)mp.y - ((int)cross.y / 2) - r + sy);
+}
+
 }  // namespace emida_amd

@@ -625,7 +625,7 @@ void launch_fft_corr_prepared(const T* pics, const T* ref, T* res, size2 side, u
     cplx<T>* spectra = nullptr;
     void* work = nullptr;
     if (fftg_needed(dbl, side)) {
-        const size_t chunk = fftg_chunk(dbl, side, std::max(ref_slices, ref_slices * batch), 0);
+        const size_t chunk = fftg_chunk(dbl, side, std::max(ref_slices, ref_slices * batch));
         EMIDA_HIP(hipMallocAsync((void**)&spectra, fftg_spectrum_bytes(dbl, side) * ref_slices, st));
         EMIDA_HIP(hipMallocAsync(&work, chunk * fftg_slice_work_bytes(dbl, side), st));
         launch_fftg_corr_prepared<T>(pics, ref, res, side, ref_slices, batch, spectra, work, chunk, st);

@@ -51,6 +51,17 @@ __device__ __forceinline__ cplx<T> twiddle16(cplx<T> v, int j) {
     }
 }
 
+// v * W_32^j, j < 16: correctly rounded cos/sin of multiples of pi/16.
+template <class T, bool INV>
+__device__ __forceinline__ cplx<T> twiddle32(cplx<T> v, int j) {
+    if (j % 2 == 0) return twiddle16<T, INV>(v, j / 2);
+    constexpr double c1 = 0.9807852804032304, s1 = 0.19509032201612828;  // pi/16
+    constexpr double c3 = 0.8314696123025452, s3 = 0.5555702330196022;   // 3 pi/16
+    const double co = j == 1 ? c1 : j == 3 ? c3 : j == 5 ? s3 : j == 7 ? s1 : j == 9 ? -s1 : j == 11 ? -s3 : j == 13 ? -c3 : -c1;
+    const double si = j == 1 || j == 15 ? s1 : j == 3 || j == 13 ? s3 : j == 5 || j == 11 ? c3 : c1;
+    return cmul(v, cplx<T>{T(co), T(INV ? si : -si)});
+}
+
 __host__ __device__ constexpr int ilog2(int n) { return n <= 1 ? 0 : 1 + ilog2(n / 2); }
 __host__ __device__ constexpr int brev_c(int v, int bits) {
     int r = 0;
@@ -86,13 +97,30 @@ __device__ __forceinline__ void dft4(cplx<T>& a0, cplx<T>& a1, cplx<T>& a2, cplx
     }
 }
 
-// In-register DFT of N <= 16 points, natural order in and out.  N = 16: radix 4
+// In-register DFT of N <= 32 points, natural order in and out.  N = 32: one radix-2 pass,
+// then two 16-point DFTs (even and odd outputs).  N = 16: radix 4
 // (n = n0 + 4 n1, k = k1 + 4 k0: 4-point DFTs over n1, twiddles W_16^(n0 k1), 4-point
 // DFTs over n0; 8 non-trivial twiddle products instead of radix 2's 10); smaller N:
 // radix-2 decimation in frequency.  The final digit reversal only renames registers.
 template <class T, int N, bool INV, bool HALF_ZERO = false>
 __device__ __forceinline__ void dft_reg(cplx<T> (&x)[N]) {
-    static_assert(N >= 1 && N <= 16 && (N & (N - 1)) == 0, "N must be a power of two <= 16");
+    static_assert(N >= 1 && N <= 32 && (N & (N - 1)) == 0, "N must be a power of two <= 32");
+    if constexpr (N == 32) {
+        cplx<T> e[16], o[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            e[k] = HALF_ZERO ? x[k] : cadd(x[k], x[k + 16]);
+            o[k] = twiddle32<T, INV>(HALF_ZERO ? x[k] : csub(x[k], x[k + 16]), k);
+        }
+        dft_reg<T, 16, INV>(e);
+        dft_reg<T, 16, INV>(o);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            x[2 * k] = e[k];
+            x[2 * k + 1] = o[k];
+        }
+        return;
+    }
     if constexpr (N == 16) {
 #pragma unroll
         for (int n0 = 0; n0 < 4; ++n0) {

@@ -11,18 +11,23 @@
 //  1. rows: two real rows packed as one complex row (prepared from the pattern or
 //     read from prepared slices), an Mx-point transform, split into the two half
 //     spectra (the split's factor 1/2 omitted: results come out doubled);
-//  2. columns: a tile of adjacent half-spectrum columns staged through LDS, an
-//     My-point transform each, the product with the conjugate reference spectrum
-//     (src/hadamard.cu:39-40) and the inverse transform - or, for the reference, the
-//     scaled spectrum stored ([roi][kx][ky], column-major, read by lanes in order);
+//  2. columns: an My-point transform of each half-spectrum column, the product with the
+//     conjugate reference spectrum (src/hadamard.cu:39-40) and the inverse transform, in
+//     place - or, for the reference, the scaled spectrum stored ([roi][kx][ky],
+//     column-major, read by lanes in order);
 //  3. rows, inverse: two output rows packed as Ga + i Gb (Hermitian extension, DC and
-//     Nyquist imaginary parts dropped, as a C2R does), one inverse transform yields
-//     both real rows, written as the reference's (2s.x x 2s.y) circular correlation
-//     buffer; arg-max, gather (cross_res_pos_policy_fft, src/kernels.cuh:36-53), fit
-//     and finalize follow in peak_kernel.
-// Transforms are Stockham autosort FFTs (radix 4, one radix-2 pass for odd log2)
-// in LDS, run by a group of lanes of one wave (Govindaraju et al., "High performance
-// discrete Fourier transforms on graphics processors", SC 2008).
+//     Nyquist imaginary parts dropped, as a C2R does), one inverse transform yields both
+//     real rows of the reference's (2s.x x 2s.y) circular correlation; one workgroup per
+//     slice keeps the largest value, runs the row pairs of the neighbourhood again
+//     (cross_res_pos_policy_fft, src/kernels.cuh:36-53), fits and finalizes, so the
+//     correlation itself is not written (the seams write it instead).
+// A transform runs on L lanes of one wave with R = M / L values each in registers and one
+// transpose through LDS (fft_common.hpp).
+//
+// Bound: the half spectra in HBM.  8 patterns x 81 ROIs of 96 x 96 in double (256 x 256):
+// 0.77 GB written and read, 240 us (rows 35, columns 119, inverse rows 86); radix-4 passes through LDS, a staged column tile and
+// the correlation written for a peak kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in
+// float (512 x 256): 381 us, before 606 us.
 //
 // Scale: the pattern's spectrum comes out doubled (the omitted split factor); the
 // stored reference spectrum is 2 s.x s.y / (Mx My) times the true one (the same
@@ -39,79 +44,84 @@ namespace emida_amd {
 
 namespace {
 
-constexpr int kGNT = 256;  // threads of the row kernels
+constexpr int kGNT = 256;  // threads of every kernel
 
-// lanes per transform of N points: one radix-4 butterfly per lane and pass, at most a wave
-__host__ __device__ constexpr int gsize(int n) { return n / 4 < 1 ? 1 : (n / 4 > kWave ? kWave : n / 4); }
-// Stockham passes of N points (radix 4, plus one radix-2 pass for odd log2 N)
-__host__ __device__ constexpr int npasses(int n) { return ilog2(n) / 2 + (ilog2(n) & 1); }
-
-template <class T, bool INV>
-__device__ __forceinline__ cplx<T> tw_at(const cplx<T>* tw, int t) {
-    cplx<T> w = tw[t];
-    if (INV) w.im = -w.im;
-    return w;
-}
-
-// Radix-4 DFT of v (forward: W_4 = -i; inverse: +i).
-template <class T, bool INV>
-__device__ __forceinline__ void radix4(cplx<T> (&v)[4]) {
-    const cplx<T> a0 = cadd(v[0], v[2]), a1 = csub(v[0], v[2]), a2 = cadd(v[1], v[3]);
-    const cplx<T> d = csub(v[1], v[3]);
-    const cplx<T> a3 = INV ? cplx<T>{-d.im, d.re} : cplx<T>{d.im, -d.re};  // d * (+-i)
-    v[0] = cadd(a0, a2);
-    v[2] = csub(a0, a2);
-    v[1] = cadd(a1, a3);
-    v[3] = csub(a1, a3);
-}
-
-// Stockham autosort FFT of N points by the G lanes of one group (all in one wave):
-// input in a (natural order), b scratch, both N complex in LDS; tw[t] = W_N^t =
-// exp(-2 pi i t / N).  Returns the buffer holding the result in natural order (a
-// when npasses(N) is even, b when odd).
-template <class T, int N, bool INV, int G>
-__device__ __forceinline__ cplx<T>* stockham(cplx<T>* a, cplx<T>* b, const cplx<T>* tw, int lane) {
-    using C = cplx<T>;
-    int ns = 1;
-#pragma unroll
-    for (int pass = 0; pass < ilog2(N) / 2; ++pass) {
-        const int step = N / (4 * ns);
-        for (int j = lane; j < N / 4; j += G) {
-            const int k = j & (ns - 1);
-            C v[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = a[j + r * (N / 4)];
-            if (ns > 1) {
-#pragma unroll
-                for (int r = 1; r < 4; ++r) v[r] = cmul(v[r], tw_at<T, INV>(tw, r * k * step));
-            }
-            radix4<T, INV>(v);
-            const int d = (j - k) * 4 + k;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) b[d + r * ns] = v[r];
-        }
-        wave_sync();
-        C* t = a;
-        a = b;
-        b = t;
-        ns *= 4;
-    }
-    if constexpr (ilog2(N) & 1) {  // ns = N / 2
-        for (int j = lane; j < N / 2; j += G) {
-            const C v0 = a[j], v1 = cmul(a[j + N / 2], tw_at<T, INV>(tw, j));
-            b[j] = cadd(v0, v1);
-            b[j + N / 2] = csub(v0, v1);
-        }
-        wave_sync();
-        a = b;
-    }
-    return a;
-}
-
-// W_n^t for t < n from the twiddle tables (table of n at offset n - 4).
+// Lanes and values per lane of an M-point transform.
+constexpr int glanes(int m) { return m >= 256 ? 16 : m >= 64 ? 8 : m >= 16 ? 4 : 2; }
+constexpr int gregs(int m) { return m / glanes(m); }
+// LDS of one lane group, in T: the transpose scratch of the real or the imaginary parts,
+// which also holds a whole real row.  Half of a complex scratch: twice the workgroups per CU
+// (256-point transforms in double: 39 KB instead of 74).
+constexpr int gslot(int m) { return glanes(m) * (gregs(m) + 1); }
 template <class T>
-__device__ __forceinline__ void init_tw(cplx<T>* tw, const cplx<T>* table, int n, int tid, int nt) {
-    for (int t = tid; t < n; t += nt) tw[t] = table[n - 4 + t];
+constexpr size_t glds(int m) {
+    return (size_t)(2 + kGNT / glanes(m)) * gslot(m) * sizeof(T);  // twiddles (complex), slots
+}
+
+// fft_fwd and fft_inv of fft_common.hpp with the transpose in two passes, real parts then
+// imaginary parts, through L (R + 1) values of T.
+template <class T, int M, bool HALF_ZERO>
+__device__ __forceinline__ void gfft_fwd(cplx<T> (&x)[gregs(M)], int lane, T* scr, const cplx<T>* tw) {
+    constexpr int L = glanes(M), R = gregs(M), Q = R / L;
+    dft_reg<T, R, false, HALF_ZERO>(x);
+#pragma unroll
+    for (int k1 = 1; k1 < R; ++k1) x[k1] = cmul(x[k1], tw[tw_index<R, true>(lane, k1)]);
+#pragma unroll
+    for (int k1 = 0; k1 < R; ++k1) scr[lane * (R + 1) + k1] = x[k1].re;
+    wave_sync();
+    cplx<T> y[Q][L];
+#pragma unroll
+    for (int i = 0; i < Q; ++i)
+#pragma unroll
+        for (int m = 0; m < L; ++m) y[i][m].re = scr[m * (R + 1) + lane + L * i];
+    wave_sync();
+#pragma unroll
+    for (int k1 = 0; k1 < R; ++k1) scr[lane * (R + 1) + k1] = x[k1].im;
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < Q; ++i)
+#pragma unroll
+        for (int m = 0; m < L; ++m) y[i][m].im = scr[m * (R + 1) + lane + L * i];
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+        dft_reg<T, L, false>(y[i]);
+#pragma unroll
+        for (int k2 = 0; k2 < L; ++k2) x[i * L + k2] = y[i][k2];
+    }
+}
+
+template <class T, int M>
+__device__ __forceinline__ void gfft_inv(cplx<T> (&x)[gregs(M)], int lane, T* scr, const cplx<T>* tw) {
+    constexpr int L = glanes(M), R = gregs(M), Q = R / L;
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+        cplx<T> y[L];
+#pragma unroll
+        for (int k2 = 0; k2 < L; ++k2) y[k2] = x[i * L + k2];
+        dft_reg<T, L, true>(y);
+#pragma unroll
+        for (int n2 = 0; n2 < L; ++n2)
+            x[i * L + n2] = n2 == 0 ? y[0] : cmul_conj(y[n2], tw[tw_index<R, true>(n2, lane + L * i)]);
+    }
+    T re[R];
+#pragma unroll
+    for (int i = 0; i < Q; ++i)
+#pragma unroll
+        for (int n2 = 0; n2 < L; ++n2) scr[n2 * (R + 1) + lane + L * i] = x[i * L + n2].re;
+    wave_sync();
+#pragma unroll
+    for (int k1 = 0; k1 < R; ++k1) re[k1] = scr[lane * (R + 1) + k1];
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < Q; ++i)
+#pragma unroll
+        for (int n2 = 0; n2 < L; ++n2) scr[n2 * (R + 1) + lane + L * i] = x[i * L + n2].im;
+    wave_sync();
+#pragma unroll
+    for (int k1 = 0; k1 < R; ++k1) x[k1] = cplx<T>{re[k1], scr[lane * (R + 1) + k1]};
+    wave_sync();
+    dft_reg<T, R, true>(x);
 }
 
 }  // namespace
@@ -138,23 +148,32 @@ struct fftg_args {
     cplx<T>* spectra_out;    // reference spectra (column kernel, spectrum out)
     T scale;                 // spectrum out: factor; product: factor on the product
     size2 out;               // output layout of the inverse rows kernel (2s.x x 2s.y)
-    T* corr;                 // [slice - first][out.y][out.x]
+    T* corr;                 // [slice - first][out.y][out.x] (the seams)
+    uint32_t npat;           // patterns of a chunk of whole patterns, else 0
     const cplx<T>* twt;      // twiddle tables (fft_twiddles)
+    int fit;                 // peak outputs (as launch_fft_pipe)
+    const double* lsq;
+    data_index<T>* maxes;
+    T* neigh;
+    double* offsets;
+    double* coefs;
 };
 
 // ---------------------------------------------------------------- kernel 1: rows
-template <class T, class IN, class SUM, int MX, bool FROM_PATTERN>
-__global__ __launch_bounds__(kGNT) void fftg_rows_kernel(fftg_args<T, IN, SUM> a) {
+// HZ: the second half of every row is zero padding (slices of at most Mx / 2 columns).
+// Grid: (slices, splits); a slice's splits take its row pairs in turn (uint16: each sums
+// the whole slice for the mean).
+template <class T, class IN, class SUM, int MX, bool FROM_PATTERN, bool HZ>
+__global__ __launch_bounds__(kGNT, 2) void fftg_rows_kernel(fftg_args<T, IN, SUM> a) {
     using C = cplx<T>;
-    constexpr int G = gsize(MX), NG = kGNT / G, NCX = MX / 2 + 1;
+    constexpr int L = glanes(MX), R = gregs(MX), NG = kGNT / L, NCX = MX / 2 + 1, RIN = HZ ? R / 2 : R;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C* tw = reinterpret_cast<C*>(lds_raw);
     __shared__ uint32_t red_u[kGNT / kWave];
-    const int tid = threadIdx.x, g = tid / G, lane = tid % G;
-    C* A = tw + MX + g * 2 * MX;
-    C* Bf = A + MX;
+    const int tid = threadIdx.x, g = tid / L, lane = tid % L;
+    T* slot = reinterpret_cast<T*>(tw + gslot(MX)) + gslot(MX) * g;
     const uint32_t sl = blockIdx.x, sn = a.first + sl;
-    init_tw<T>(tw, a.twt, MX, tid, kGNT);
+    load_twiddles_2d<T, MX, R>(tw, a.twt, tid, kGNT);
 
     const IN* pic = nullptr;
     const T* pre = nullptr;
@@ -165,8 +184,19 @@ __global__ __launch_bounds__(kGNT) void fftg_rows_kernel(fftg_args<T, IN, SUM> a
         pic = a.pics + (size_t)(sn / a.nb) * a.src.area() + (size_t)b0.y * a.src.x + b0.x;
         if constexpr (std::is_same<IN, uint16_t>::value) {
             uint32_t su = 0;
-            for (int y = tid / 64; y < sy; y += kGNT / 64)
-                for (int x = tid % 64; x < sx; x += 64) su += pic[(size_t)y * a.src.x + x];
+            constexpr int U = 8;  // rows in flight per wave
+            for (int x = tid % kWave; x < sx; x += kWave)
+                for (int y0 = tid / kWave; y0 < sy; y0 += kGNT / kWave * U) {
+                    uint32_t v[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int y = y0 + kGNT / kWave * u;
+                        v[u] = pic[(size_t)min(y, sy - 1) * a.src.x + x];
+                        v[u] = y < sy ? v[u] : 0u;
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) su += v[u];
+                }
             su = wave_reduce(su, 0u, [](uint32_t x, uint32_t y) { return x + y; });
             if (tid % kWave == 0) red_u[tid / kWave] = su;
             __syncthreads();
@@ -184,157 +214,280 @@ __global__ __launch_bounds__(kGNT) void fftg_rows_kernel(fftg_args<T, IN, SUM> a
 
     C* w = a.work + (size_t)sl * a.my * NCX;
     const int npairs = (sy + 1) / 2;
-    for (int p0 = 0; p0 < npairs; p0 += NG) {
-        const int p = p0 + g;
-        const bool act = p < npairs, second = 2 * p + 1 < sy;
-        for (int n = lane; n < MX; n += G) {
-            T v0 = T(0), v1 = T(0);
-            if (act && n < sx) {
-                if constexpr (FROM_PATTERN) {
-                    v0 = prep_px<T, IN>(pic[(size_t)(2 * p) * a.src.x + n], mean, a.hx[n], a.hy[2 * p]);
-                    if (second) v1 = prep_px<T, IN>(pic[(size_t)(2 * p + 1) * a.src.x + n], mean, a.hx[n], a.hy[2 * p + 1]);
-                } else {
-                    v0 = pre[(size_t)(2 * p) * a.pitch + n];
-                    if (second) v1 = pre[(size_t)(2 * p + 1) * a.pitch + n];
-                }
+    for (int p = g + NG * (int)blockIdx.y; p < npairs; p += NG * (int)gridDim.y) {
+        const bool second = 2 * p + 1 < sy;
+        const int y0 = 2 * p, y1 = second ? 2 * p + 1 : 2 * p;
+        C x[R];
+#pragma unroll
+        for (int n1 = 0; n1 < R; ++n1) x[n1] = C{T(0), T(0)};
+        T wy0 = T(0), wy1 = T(0);
+        if constexpr (FROM_PATTERN) {
+            wy0 = a.hy[y0];
+            wy1 = a.hy[y1];
+        }
+#pragma unroll
+        for (int n1 = 0; n1 < RIN; ++n1) {
+            const int n = L * n1 + lane, nc = min(n, sx - 1);
+            T v0, v1;
+            if constexpr (FROM_PATTERN) {
+                const T wx = a.hx[nc];
+                v0 = prep_px<T, IN>(pic[(size_t)y0 * a.src.x + nc], mean, wx, wy0);
+                v1 = prep_px<T, IN>(pic[(size_t)y1 * a.src.x + nc], mean, wx, wy1);
+            } else {
+                v0 = pre[(size_t)y0 * a.pitch + nc];
+                v1 = pre[(size_t)y1 * a.pitch + nc];
             }
-            A[n] = C{v0, v1};
+            if (n < sx) x[n1] = C{v0, second ? v1 : T(0)};
+        }
+        gfft_fwd<T, MX, HZ>(x, lane, slot, tw);
+        // split: frequencies k and Mx - k through the slot, real parts, then imaginary parts
+        constexpr int NK = MX / 2 / L + 1;  // frequencies lane + L i <= Mx / 2 of a lane
+        T sre[NK], dre[NK];
+        auto put = [&](auto&& part) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) slot[lane + L * (r / L) + R * (r % L)] = part(x[r]);
+            wave_sync();
+        };
+        put([](const C& v) { return v.re; });
+#pragma unroll
+        for (int i = 0; i < NK; ++i) {
+            const int k = lane + L * i;
+            const T z = slot[k], m = slot[(MX - k) & (MX - 1)];
+            sre[i] = z + m;
+            dre[i] = m - z;
         }
         wave_sync();
-        const C* X = stockham<T, MX, false, G>(A, Bf, tw, lane);
-        if (act) {
-            C* r0 = w + (size_t)(2 * p) * NCX;
-            for (int k = lane; k < NCX; k += G) {
-                const C z = X[k], m = X[(MX - k) & (MX - 1)];
-                r0[k] = C{z.re + m.re, z.im - m.im};
-                if (second) r0[NCX + k] = C{z.im + m.im, m.re - z.re};
+        put([](const C& v) { return v.im; });
+        C* r0 = w + (size_t)y0 * NCX;
+#pragma unroll
+        for (int i = 0; i < NK; ++i) {
+            const int k = lane + L * i;
+            const T z = slot[k], m = slot[(MX - k) & (MX - 1)];
+            if (k < NCX) {
+                r0[k] = C{sre[i], z - m};
+                if (second) r0[NCX + k] = C{z + m, dre[i]};
             }
         }
-        wave_sync();  // X is the next row pair's input or scratch
+        wave_sync();  // the slot is the next row pair's scratch
     }
 }
 
 // ---------------------------------------------------------------- kernel 2: columns
 enum { COLS_PIPE = 0, COLS_SPECTRUM = 1, COLS_STD_PIPE = 2, COLS_STD_SPECTRUM = 3 };
 
-template <class T>
-__host__ __device__ constexpr int col_tile(int my) {
-    // columns per workgroup: at least 64 bytes of a row per load, at least one wave
-    return (sizeof(T) == 4 ? 8 : 4) > kWave / gsize(my) ? (sizeof(T) == 4 ? 8 : 4) : kWave / gsize(my);
-}
-
+// One column per lane group, read and written in place: the NG groups of a workgroup take
+// adjacent columns, so the lanes of a row read at least 64 consecutive bytes.  The columns
+// of the patterns of one ROI run back to back on one XCD (one spectrum column in its L2).
 template <class T, int MY, int MODE>
-__global__ __launch_bounds__(col_tile<T>(MY) * gsize(MY)) void fftg_cols_kernel(fftg_args<T, T, T> a) {
+__global__ __launch_bounds__(kGNT, 2) void fftg_cols_kernel(fftg_args<T, T, T> a, uint32_t nblk) {
     using C = cplx<T>;
-    constexpr int G = gsize(MY), CB = col_tile<T>(MY), NT = CB * G;
-    constexpr bool RES_IN_B = npasses(MY) & 1;  // where stockham leaves a forward result
+    constexpr bool HZ = MODE == COLS_PIPE || MODE == COLS_SPECTRUM;
+    constexpr int L = glanes(MY), R = gregs(MY), NG = kGNT / L, RIN = HZ ? R / 2 : R;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C* tw = reinterpret_cast<C*>(lds_raw);
-    C* tile = tw + MY;  // CB columns x 2 buffers x MY
-    const int tid = threadIdx.x, g = tid / G, lane = tid % G;
-    const uint32_t sl = blockIdx.y, sn = a.first + sl, roi = sn % a.nb;
-    const int ncx = (int)a.mx / 2 + 1, kx0 = blockIdx.x * CB;
-    init_tw<T>(tw, a.twt, MY, tid, NT);
-    C* w = a.work + (size_t)sl * a.my * ncx;
-    const int rows = MODE == COLS_SPECTRUM || MODE == COLS_PIPE ? (int)a.side.y : (int)a.my;
-    // rows of the output the inverse rows kernel reads (the reference layout)
-    const int sy = (int)a.side.y, pady = MY - 2 * sy;
-    for (int e = tid; e < MY * CB; e += NT) {
-        const int y = e / CB, c = e % CB;
-        tile[c * 2 * MY + y] = (y < rows && kx0 + c < ncx) ? w[(size_t)y * ncx + kx0 + c] : C{T(0), T(0)};
-    }
-    __syncthreads();
-    C* A = tile + g * 2 * MY;
-    C* Bf = A + MY;
-    C* X = stockham<T, MY, false, G>(A, Bf, tw, lane);
-    const int kx = kx0 + g;
-    const bool col_ok = kx < ncx;
-    if constexpr (MODE == COLS_SPECTRUM || MODE == COLS_STD_SPECTRUM) {
-        if (col_ok) {
-            for (int k = lane; k < MY; k += G) {
-                const C v = X[k];
-                if constexpr (MODE == COLS_SPECTRUM)
-                    a.spectra_out[((size_t)roi * ncx + kx) * MY + k] = C{v.re * a.scale, v.im * a.scale};
-                else
-                    a.spectra_out[((size_t)roi * MY + k) * ncx + kx] = C{v.re * a.scale, v.im * a.scale};
-            }
-        }
-        return;
+    const int tid = threadIdx.x, g = tid / L, lane = tid % L;
+    T* slot = reinterpret_cast<T*>(tw + gslot(MY)) + gslot(MY) * g;
+    const int ncx = (int)a.mx / 2 + 1;
+    const uint32_t gx = div_up((uint32_t)ncx, (uint32_t)NG), b = xcd_remap(blockIdx.x, nblk);
+    uint32_t sl, col;
+    if (a.npat) {
+        const uint32_t roi = b / (gx * a.npat), in = b - roi * gx * a.npat;
+        col = in / a.npat;
+        sl = (in - col * a.npat) * a.nb + roi;
     } else {
-        C* Y = RES_IN_B ? A : Bf;  // the other buffer
-        for (int k = lane; k < MY; k += G) {
-            C r = C{T(0), T(0)};
-            if (col_ok) {
-                if constexpr (MODE == COLS_PIPE) r = a.spectra[((size_t)roi * ncx + kx) * MY + k];
-                else r = a.spectra[((size_t)roi * MY + k) * ncx + kx];
-            }
-            C h = hadamard(X[k], r);
-            if constexpr (MODE == COLS_STD_PIPE) h = C{h.re * a.scale, h.im * a.scale};
-            Y[k] = h;
+        sl = b / gx;
+        col = b - sl * gx;
+    }
+    const uint32_t roi = (a.first + sl) % a.nb;
+    const int kx = (int)col * NG + g;
+    load_twiddles_2d<T, MY, R>(tw, a.twt, tid, kGNT);
+    C* w = a.work + (size_t)sl * a.my * ncx + min(kx, ncx - 1);
+    const int rows = HZ ? (int)a.side.y : (int)a.my;
+    C x[R];
+#pragma unroll
+    for (int n1 = 0; n1 < R; ++n1) x[n1] = C{T(0), T(0)};
+#pragma unroll
+    for (int n1 = 0; n1 < RIN; ++n1) {
+        const int y = L * n1 + lane;
+        const C v = w[(size_t)min(y, rows - 1) * ncx];
+        x[n1] = y < rows ? v : C{T(0), T(0)};
+    }
+    __syncthreads();  // twiddles
+    if (kx >= ncx) return;
+    // the reference spectrum: in flight during the forward transform where registers allow
+    auto spec_at = [&](int r) {
+        const int k = lane + L * (r / L) + R * (r % L);
+        if constexpr (MODE == COLS_PIPE) return a.spectra[((size_t)roi * ncx + kx) * MY + k];
+        else return a.spectra[((size_t)roi * MY + k) * ncx + kx];
+    };
+    constexpr bool EARLY = R * sizeof(C) <= 256;
+    C spec[EARLY ? R : 1];
+    if constexpr (EARLY && (MODE == COLS_PIPE || MODE == COLS_STD_PIPE)) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) spec[r] = spec_at(r);
+    }
+    gfft_fwd<T, MY, HZ>(x, lane, slot, tw);
+    if constexpr (MODE == COLS_SPECTRUM || MODE == COLS_STD_SPECTRUM) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int k = lane + L * (r / L) + R * (r % L);
+            const C v = C{x[r].re * a.scale, x[r].im * a.scale};
+            if constexpr (MODE == COLS_SPECTRUM) a.spectra_out[((size_t)roi * ncx + kx) * MY + k] = v;
+            else a.spectra_out[((size_t)roi * MY + k) * ncx + kx] = v;
         }
-        wave_sync();
-        C* Z = stockham<T, MY, true, G>(Y, X, tw, lane);
-        __syncthreads();
-        // every group's result sits in the same buffer of its column (same MY)
-        const int zoff = (int)(Z - (tile + g * 2 * MY));
-        for (int e = tid; e < MY * CB; e += NT) {
-            const int y = e / CB, c = e % CB;
-            const bool need = MODE == COLS_STD_PIPE || y <= sy || y > sy + pady;
-            if (need && kx0 + c < ncx) w[(size_t)y * ncx + kx0 + c] = tile[c * 2 * MY + zoff + y];
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if constexpr (EARLY) x[r] = hadamard(x[r], spec[r]);
+            else x[r] = hadamard(x[r], spec_at(r));
+            if constexpr (MODE == COLS_STD_PIPE) x[r] = C{x[r].re * a.scale, x[r].im * a.scale};
+        }
+        gfft_inv<T, MY>(x, lane, slot, tw);
+        // rows of the output the inverse rows kernel reads (the reference layout)
+        const int sy = (int)a.side.y, pady = MY - 2 * sy;
+#pragma unroll
+        for (int n1 = 0; n1 < R; ++n1) {
+            const int y = L * n1 + lane;
+            if (MODE == COLS_STD_PIPE || y <= sy || y > sy + pady) w[(size_t)y * ncx] = x[n1];
         }
     }
 }
 
 // ---------------------------------------------------------------- kernel 3: rows, inverse
+// Output rows 2q and 2q + 1 of the reference layout of one slice, by one lane group: on
+// return lane n2 holds their columns L n1 + n2 (circular) in x[n1].re and x[n1].im.
 template <class T, int MX>
-__global__ __launch_bounds__(kGNT) void fftg_rows_inv_kernel(fftg_args<T, T, T> a) {
+__device__ __forceinline__ void inverse_row_pair(cplx<T> (&x)[gregs(MX)], const cplx<T>* w, int q, int sy, int pady,
+                                                 int lane, T* slot, const cplx<T>* tw) {
     using C = cplx<T>;
-    constexpr int G = gsize(MX), NG = kGNT / G, NCX = MX / 2 + 1, S = MX / 2;
+    constexpr int L = glanes(MX), R = gregs(MX), NCX = MX / 2 + 1, S = MX / 2;
+    // reference-layout row r <= s is circular row r, r > s is r + M - 2s
+    const int ra = 2 * q, rb = 2 * q + 1;
+    const C* ga_row = w + (size_t)(ra <= sy ? ra : ra + pady) * NCX;
+    const C* gb_row = w + (size_t)(rb <= sy ? rb : rb + pady) * NCX;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int k = lane + L * (r / L) + R * (r % L);
+        const bool mirror = k > S;
+        const int col = mirror ? MX - k : k;
+        C ga = ga_row[col], gb = gb_row[col];
+        if (mirror) {
+            ga.im = -ga.im;
+            gb.im = -gb.im;
+        }
+        if (k == 0 || k == S) {
+            ga.im = T(0);
+            gb.im = T(0);
+        }
+        x[r] = C{ga.re - gb.im, ga.im + gb.re};
+    }
+    gfft_inv<T, MX>(x, lane, slot, tw);
+}
+
+// PEAK: one workgroup per slice, arg-max (lowest index on ties), neighbourhood, fit and
+// finalize as peak_kernel; else the rows of the correlation buffer.
+template <class T, int MX, bool PEAK>
+__global__ __launch_bounds__(kGNT, 2) void fftg_rows_inv_kernel(fftg_args<T, T, T> a) {
+    using C = cplx<T>;
+    constexpr int L = glanes(MX), R = gregs(MX), NG = kGNT / L, NCX = MX / 2 + 1;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C* tw = reinterpret_cast<C*>(lds_raw);
-    const int tid = threadIdx.x, g = tid / G, lane = tid % G;
-    C* A = tw + MX + g * 2 * MX;
-    C* Bf = A + MX;
-    const uint32_t sl = blockIdx.x;
-    init_tw<T>(tw, a.twt, MX, tid, kGNT);
+    const int tid = threadIdx.x, g = tid / L, lane = tid % L;
+    T* slot = reinterpret_cast<T*>(tw + gslot(MX)) + gslot(MX) * g;
+    const uint32_t sl = blockIdx.x, sn = a.first + sl;
+    load_twiddles_2d<T, MX, R>(tw, a.twt, tid, kGNT);
     __syncthreads();
     const C* w = a.work + (size_t)sl * a.my * NCX;
-    T* out = a.corr + (size_t)sl * a.out.area();
     // reference-layout index k <= s is circular position k, k > s is k + M - 2s
     const int sx = (int)a.out.x / 2, sy = (int)a.out.y / 2;
     const int padx = MX - (int)a.out.x, pady = (int)a.my - (int)a.out.y;
     const int npairs = (int)a.out.y / 2;
-    for (int q0 = 0; q0 < npairs; q0 += NG) {
-        const int q = q0 + g;
-        const bool act = q < npairs;
-        const int ra = 2 * q, rb = 2 * q + 1;
-        const int ya = act ? (ra <= sy ? ra : ra + pady) : 0, yb = act ? (rb <= sy ? rb : rb + pady) : 0;
-        const C* ga_row = w + (size_t)ya * NCX;
-        const C* gb_row = w + (size_t)yb * NCX;
-        for (int k = lane; k < MX; k += G) {
-            const bool mirror = k > S;
-            const int col = mirror ? MX - k : k;
-            C ga = ga_row[col], gb = gb_row[col];
-            if (mirror) {
-                ga.im = -ga.im;
-                gb.im = -gb.im;
+    T best = -(T)__builtin_huge_val();
+    uint32_t bi = 0xffffffffu;
+    for (int q = g; q < npairs; q += NG) {
+        C x[R];
+        inverse_row_pair<T, MX>(x, w, q, sy, pady, lane, slot, tw);
+        const uint32_t ia = 2 * (uint32_t)q * a.out.x, ib = ia + a.out.x;
+        if constexpr (PEAK) {
+            // a thread meets its positions in index order, so strictly larger keeps the lowest
+            T va = best, vb;
+            int ca = -1, cb = -1;
+#pragma unroll
+            for (int n1 = 0; n1 < R; ++n1) {
+                const int c = L * n1 + lane;
+                if ((c <= sx || c > sx + padx) && x[n1].re > va) va = x[n1].re, ca = c;
             }
-            if (k == 0 || k == S) {
-                ga.im = T(0);
-                gb.im = T(0);
+            vb = va;
+#pragma unroll
+            for (int n1 = 0; n1 < R; ++n1) {
+                const int c = L * n1 + lane;
+                if ((c <= sx || c > sx + padx) && x[n1].im > vb) vb = x[n1].im, cb = c;
             }
-            A[k] = C{ga.re - gb.im, ga.im + gb.re};
+            if (ca >= 0) bi = ia + (uint32_t)(ca <= sx ? ca : ca - padx);
+            if (cb >= 0) bi = ib + (uint32_t)(cb <= sx ? cb : cb - padx);
+            best = vb;
+        } else {
+            T* out = a.corr + (size_t)sl * a.out.area();
+#pragma unroll
+            for (int n1 = 0; n1 < R; ++n1) {
+                const int c = L * n1 + lane;
+                if (c <= sx || c > sx + padx) {
+                    const int rx = c <= sx ? c : c - padx;
+                    out[ia + rx] = x[n1].re;
+                    out[ib + rx] = x[n1].im;
+                }
+            }
         }
-        wave_sync();
-        const C* X = stockham<T, MX, true, G>(A, Bf, tw, lane);
-        if (act) {
-            for (int rx = lane; rx < (int)a.out.x; rx += G) {
-                const C v = X[rx <= sx ? rx : rx + padx];
-                out[(size_t)ra * a.out.x + rx] = v.re;
-                out[(size_t)rb * a.out.x + rx] = v.im;
+    }
+    if constexpr (PEAK) {
+        __shared__ T sv[kGNT / kWave];
+        __shared__ uint32_t si[kGNT / kWave];
+        __shared__ T nbv[81];
+        __shared__ double cf[6];
+        block_argmax<T, kGNT>(best, bi, sv, si);
+        const size2 cross{a.out.x - 1, a.out.y - 1};
+        const size2 mp = shift_pos(POLICY_FFT, bi, cross);
+        const int fit = a.fit, rad = (fit - 1) / 2, kk = fit * fit;
+        // neighbourhood row j: its row pair again, the row kept in slot j
+        static_assert(NG >= 9, "one lane group per neighbourhood row");
+        if (g < fit) {
+            const size2 c = clamp_pos((int)mp.x, (int)mp.y - rad + g, cross);
+            const int ry = (int)((c.y + (a.out.y / 2 + 1)) % a.out.y);
+            C x[R];
+            inverse_row_pair<T, MX>(x, w, ry >> 1, sy, pady, lane, slot, tw);
+#pragma unroll
+            for (int n1 = 0; n1 < R; ++n1) {
+                const T even = x[n1].re, odd = x[n1].im;
+                slot[L * n1 + lane] = ry & 1 ? odd : even;
             }
         }
-        wave_sync();
+        __syncthreads();
+        for (int t = tid; t < kk; t += kGNT) {
+            const int i = t % fit, j = t / fit;
+            const size2 c = clamp_pos((int)mp.x - rad + i, (int)mp.y - rad + j, cross);
+            const int rx = (int)((c.x + (a.out.x / 2 + 1)) % a.out.x);
+            const T v = (reinterpret_cast<const T*>(tw + gslot(MX)) + gslot(MX) * j)[rx <= sx ? rx : rx + padx];
+            nbv[t] = v;
+            if (a.neigh) a.neigh[(size_t)sn * kk + t] = v;
+        }
+        __syncthreads();
+        if (tid < 6) cf[tid] = fit_coef<T>(a.lsq + tid * kk, nbv, kk);
+        __syncthreads();
+        if (tid == 0) {
+            if (a.maxes) {
+                a.maxes[sn].data = best;
+                a.maxes[sn].index = bi;
+            }
+            double px, py, ox, oy;
+            fit_peak(cf, px, py);
+            finalize_offset(bi, cross, POLICY_FFT, fit, px, py, ox, oy);
+            if (a.offsets) {
+                a.offsets[2 * (size_t)sn] = ox;
+                a.offsets[2 * (size_t)sn + 1] = oy;
+            }
+            if (a.coefs)
+                for (int c = 0; c < 6; ++c) a.coefs[6 * (size_t)sn + c] = cf[c];
+        }
     }
 }
 
@@ -351,54 +504,48 @@ void dispatch_n(uint32_t n, F&& f) {
     }
 }
 
-template <class T>
-size_t rows_lds(int mx) {
-    return ((size_t)mx + (size_t)(kGNT / gsize(mx)) * 2 * mx) * sizeof(cplx<T>);
-}
-template <class T>
-size_t cols_lds(int my) {
-    return ((size_t)my + (size_t)col_tile<T>(my) * 2 * my) * sizeof(cplx<T>);
-}
-
 template <class K>
 void set_lds(K kern, size_t bytes) {
     EMIDA_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
 }
 
-template <class T, class IN, class SUM, bool FP>
+template <class T, class IN, class SUM, bool FP, bool HZ>
 void run_rows(const fftg_args<T, IN, SUM>& a, hipStream_t st) {
     dispatch_n<4>(a.mx, [&](auto mc) {
-        constexpr int MX = decltype(mc)::value;
-        auto k = fftg_rows_kernel<T, IN, SUM, MX, FP>;
-        static const bool once = (set_lds(k, rows_lds<T>(MX)), true);
+        constexpr int MX = decltype(mc)::value, NG = kGNT / glanes(MX);
+        auto k = fftg_rows_kernel<T, IN, SUM, MX, FP, HZ>;
+        static const bool once = (set_lds(k, glds<T>(MX)), true);
         (void)once;
-        k<<<a.total, kGNT, rows_lds<T>(MX), st>>>(a);
+        // enough workgroups for every CU to hold a few, at most one row pair per lane group
+        const uint32_t most = div_up((a.in_rows + 1) / 2, (uint32_t)NG);
+        const uint32_t splits = std::max(1u, std::min(most, 1024u / std::max(1u, a.total)));
+        k<<<dim3(a.total, splits), kGNT, glds<T>(MX), st>>>(a);
         EMIDA_LAUNCHED("fftg_rows_kernel");
     });
 }
 
 template <class T, int MODE>
-void run_cols(const fftg_args<T, T, T>& a, hipStream_t st) {
+void run_cols(fftg_args<T, T, T> a, hipStream_t st) {
+    a.npat = a.first % a.nb == 0 && a.total % a.nb == 0 ? a.total / a.nb : 0;
     dispatch_n<4>(a.my, [&](auto mc) {
         constexpr int MY = decltype(mc)::value;
         auto k = fftg_cols_kernel<T, MY, MODE>;
-        static const bool once = (set_lds(k, cols_lds<T>(MY)), true);
+        static const bool once = (set_lds(k, glds<T>(MY)), true);
         (void)once;
-        constexpr int CB = col_tile<T>(MY);
-        const dim3 grid((unsigned)div_up((int)a.mx / 2 + 1, CB), a.total);
-        k<<<grid, CB * gsize(MY), cols_lds<T>(MY), st>>>(a);
+        const uint32_t blocks = div_up(a.mx / 2 + 1, (uint32_t)(kGNT / glanes(MY))) * a.total;
+        k<<<blocks, kGNT, glds<T>(MY), st>>>(a, blocks);
         EMIDA_LAUNCHED("fftg_cols_kernel");
     });
 }
 
-template <class T>
+template <class T, bool PEAK>
 void run_rows_inv(const fftg_args<T, T, T>& a, hipStream_t st) {
     dispatch_n<4>(a.mx, [&](auto mc) {
         constexpr int MX = decltype(mc)::value;
-        auto k = fftg_rows_inv_kernel<T, MX>;
-        static const bool once = (set_lds(k, rows_lds<T>(MX)), true);
+        auto k = fftg_rows_inv_kernel<T, MX, PEAK>;
+        static const bool once = (set_lds(k, glds<T>(MX)), true);
         (void)once;
-        k<<<a.total, kGNT, rows_lds<T>(MX), st>>>(a);
+        k<<<a.total, kGNT, glds<T>(MX), st>>>(a);
         EMIDA_LAUNCHED("fftg_rows_inv_kernel");
     });
 }
@@ -419,6 +566,12 @@ fftg_args<T, T, T> as_t(const fftg_args<T, IN, SUM>& a) {
     b.out = a.out;
     b.corr = a.corr;
     b.twt = a.twt;
+    b.fit = a.fit;
+    b.lsq = a.lsq;
+    b.maxes = a.maxes;
+    b.neigh = a.neigh;
+    b.offsets = a.offsets;
+    b.coefs = a.coefs;
     return b;
 }
 
@@ -438,23 +591,17 @@ size_t fftg_spectrum_bytes(bool is_double, size2 side) {
 
 size_t fftg_slice_work_bytes(bool is_double, size2 side) { return fftg_spectrum_bytes(is_double, side); }
 
-size_t fftg_chunk(bool is_double, size2 side, uint32_t total, size_t extra_per_slice) {
-    const size_t per = fftg_slice_work_bytes(is_double, side) + extra_per_slice;
-    const size_t c = std::max<size_t>(1, kFftgWorkCap / per);
+size_t fftg_chunk(bool is_double, size2 side, uint32_t total) {
+    const size_t c = std::max<size_t>(1, kFftgWorkCap / fftg_slice_work_bytes(is_double, side));
     return std::min<size_t>(c, total);
 }
 
-size_t fftg_ref_work_bytes(bool is_double, size2 side, uint32_t nb) {
-    return fftg_chunk(is_double, side, nb, 0) * fftg_slice_work_bytes(is_double, side);
-}
-
-size_t fftg_work_bytes(bool is_double, size2 side, uint32_t total, bool with_corr) {
-    const size_t corr = with_corr ? (size_t)4 * side.area() * (is_double ? 8 : 4) : 0;
-    return fftg_chunk(is_double, side, total, corr) * (fftg_slice_work_bytes(is_double, side) + corr);
+size_t fftg_work_bytes(bool is_double, size2 side, uint32_t total) {
+    return fftg_chunk(is_double, side, total) * fftg_slice_work_bytes(is_double, side);
 }
 
 // Reference spectra ([roi][kx][ky], 2 s.x s.y / (Mx My) times the true spectrum) from
-// the reference pattern; work holds fftg_ref_work_bytes bytes.
+// the reference pattern; work holds fftg_work_bytes(.., nb) bytes.
 template <class T, class IN, class S>
 void launch_fftg_ref(const IN* pics, const S* sums, const T* hx, const T* hy, const size2* begins, size2 src,
                      size2 side, uint32_t nb, cplx<T>* spectra, void* work, hipStream_t st) {
@@ -479,58 +626,51 @@ void launch_fftg_ref(const IN* pics, const S* sums, const T* hx, const T* hy, co
     a.spectra_out = spectra;
     // the row and column stages double it; s.x s.y / (Mx My) is exact
     a.scale = (T)((double)side.x * side.y / ((double)a.mx * a.my));
-    const size_t chunk = fftg_chunk(sizeof(T) == 8, side, nb, 0);
+    const size_t chunk = fftg_chunk(sizeof(T) == 8, side, nb);
     for (uint32_t f = 0; f < nb; f += (uint32_t)chunk) {
         a.first = f;
         a.total = (uint32_t)std::min<size_t>(chunk, nb - f);
-        run_rows<T, IN, S, true>(a, st);
+        run_rows<T, IN, S, true, true>(a, st);
         run_cols<T, COLS_SPECTRUM>(as_t(a), st);
     }
 }
 
-// Pipeline of `total` slices: correlation buffers into corr (caller's, the whole
-// launch) or the work buffer, then the peak kernel.
+// Pipeline of `total` slices, from the patterns to the offsets.
 template <class T, class IN, class S>
 void launch_fftg_pipe(const IN* pics, const S* sums, const T* hx, const T* hy, const size2* begins, size2 src,
                       size2 side, uint32_t nb, uint32_t total, const cplx<T>* spectra, int fit, data_index<T>* maxes,
-                      T* neigh, double* offsets, double* coefs, T* corr_out, void* work, hipStream_t st) {
+                      T* neigh, double* offsets, double* coefs, void* work, hipStream_t st) {
     if (total == 0) return;
-    const bool dbl = sizeof(T) == 8;
-    const size2 out{2 * side.x, 2 * side.y};
-    const size_t corr_per = (size_t)out.area() * sizeof(T);
-    // the chunk fftg_work_bytes(.., with_corr) sized the work buffer for
-    const size_t chunk = fftg_chunk(dbl, side, total, corr_per);
-    char* wb = (char*)work;
-    T* corr_chunk = corr_out ? nullptr : (T*)(wb + chunk * fftg_slice_work_bytes(dbl, side));
+    fftg_args<T, IN, S> a{};
+    a.twt = fft_twiddles<T>();
+    a.pics = pics;
+    a.sums = sums;
+    a.hx = hx;
+    a.hy = hy;
+    a.begins = begins;
+    a.src = src;
+    a.in_rows = side.y;
+    a.in_cols = side.x;
+    a.side = side;
+    a.mx = fft_padded(side.x);
+    a.my = fft_padded(side.y);
+    a.nb = nb;
+    a.work = (cplx<T>*)work;
+    a.spectra = spectra;
+    a.out = size2{2 * side.x, 2 * side.y};
+    a.fit = fit;
+    a.lsq = lstsq_device_table() + lstsq_offset(fit);
+    a.maxes = maxes;
+    a.neigh = neigh;
+    a.offsets = offsets;
+    a.coefs = coefs;
+    const size_t chunk = fftg_chunk(sizeof(T) == 8, side, total);
     for (uint32_t f = 0; f < total; f += (uint32_t)chunk) {
-        fftg_args<T, IN, S> a{};
-        a.twt = fft_twiddles<T>();
-        a.pics = pics;
-        a.sums = sums;
-        a.hx = hx;
-        a.hy = hy;
-        a.begins = begins;
-        a.src = src;
-        a.in_rows = side.y;
-        a.in_cols = side.x;
-        a.side = side;
-        a.mx = fft_padded(side.x);
-        a.my = fft_padded(side.y);
-        a.nb = nb;
         a.first = f;
         a.total = (uint32_t)std::min<size_t>(chunk, total - f);
-        a.work = (cplx<T>*)work;
-        a.spectra = spectra;
-        a.out = out;
-        a.corr = corr_out ? corr_out + (size_t)f * out.area() : corr_chunk;
-        run_rows<T, IN, S, true>(a, st);
-        const fftg_args<T, T, T> b = as_t(a);
-        run_cols<T, COLS_PIPE>(b, st);
-        run_rows_inv<T>(b, st);
-        launch_peak<T>(a.corr, (size_t)a.total * out.area(), out.area(), size2{out.x - 1, out.y - 1}, POLICY_FFT,
-                       fit, maxes ? maxes + f : nullptr, neigh ? neigh + (size_t)f * fit * fit : nullptr,
-                       offsets ? offsets + 2 * (size_t)f : nullptr, coefs ? coefs + 6 * (size_t)f : nullptr, a.total,
-                       st);
+        run_rows<T, IN, S, true, true>(a, st);
+        run_cols<T, COLS_PIPE>(as_t(a), st);
+        run_rows_inv<T, true>(as_t(a), st);
     }
 }
 
@@ -558,7 +698,7 @@ void launch_fftg_corr_prepared(const T* pics, const T* ref, T* res, size2 side, 
         a.first = f;
         a.total = (uint32_t)std::min<size_t>(chunk, nb - f);
         a.work = (cplx<T>*)work;
-        run_rows<T, T, T, false>(a, st);
+        run_rows<T, T, T, false, true>(a, st);
         fftg_args<T, T, T> b = a;
         b.work = (cplx<T>*)work;
         run_cols<T, COLS_SPECTRUM>(b, st);
@@ -573,9 +713,9 @@ void launch_fftg_corr_prepared(const T* pics, const T* ref, T* res, size2 side, 
         b.spectra = spectra;
         b.spectra_out = nullptr;
         b.corr = res + (size_t)f * b.out.area();
-        run_rows<T, T, T, false>(b, st);
+        run_rows<T, T, T, false, true>(b, st);
         run_cols<T, COLS_PIPE>(b, st);
-        run_rows_inv<T>(b, st);
+        run_rows_inv<T, false>(b, st);
     }
 }
 
@@ -608,9 +748,9 @@ void launch_fftg_std_corr(const T* pic, const cplx<T>* spectra, T* res, size2 si
         b.first = f;
         b.total = (uint32_t)std::min<size_t>(chunk, total - f);
         b.corr = res + (size_t)f * b.out.area();
-        run_rows<T, T, T, false>(b, st);
+        run_rows<T, T, T, false, false>(b, st);
         run_cols<T, COLS_STD_PIPE>(b, st);
-        run_rows_inv<T>(b, st);
+        run_rows_inv<T, false>(b, st);
     }
 }
 
@@ -639,7 +779,7 @@ void launch_fftg_std_r2c(const T* pic, uint32_t pitch, cplx<T>* spectra, size2 s
         fftg_args<T, T, T> b = a;
         b.first = f;
         b.total = (uint32_t)std::min<size_t>(chunk, n - f);
-        run_rows<T, T, T, false>(b, st);
+        run_rows<T, T, T, false, false>(b, st);
         run_cols<T, COLS_STD_SPECTRUM>(b, st);
     }
 }
@@ -649,7 +789,7 @@ void launch_fftg_std_r2c(const T* pic, uint32_t pitch, cplx<T>* spectra, size2 s
                                             uint32_t, cplx<T>*, void*, hipStream_t);                            \
     template void launch_fftg_pipe<T, IN, S>(const IN*, const S*, const T*, const T*, const size2*, size2, size2,\
                                              uint32_t, uint32_t, const cplx<T>*, int, data_index<T>*, T*, double*, \
-                                             double*, T*, void*, hipStream_t);
+                                             double*, void*, hipStream_t);
 INST_FFTG(float, uint16_t, uint32_t)
 INST_FFTG(double, uint16_t, uint32_t)
 INST_FFTG(float, float, float)

@@ -169,18 +169,16 @@ void launch_hadamard(cplx<T>* pics, const cplx<T>* ref, size2 one, uint32_t ref_
 bool fftg_needed(bool is_double, size2 side);               // the single-kernel paths do not take this shape
 size_t fftg_spectrum_bytes(bool is_double, size2 side);      // reference spectrum of one ROI
 size_t fftg_slice_work_bytes(bool is_double, size2 side);    // half spectra of one slice
-size_t fftg_chunk(bool is_double, size2 side, uint32_t total, size_t extra_per_slice);  // slices per launch chunk
-size_t fftg_ref_work_bytes(bool is_double, size2 side, uint32_t nb);  // work of launch_fftg_ref
-// work of launch_fftg_pipe (with_corr: it also holds the chunk's correlation buffers)
-size_t fftg_work_bytes(bool is_double, size2 side, uint32_t total, bool with_corr);
+size_t fftg_chunk(bool is_double, size2 side, uint32_t total);  // slices per launch chunk
+size_t fftg_work_bytes(bool is_double, size2 side, uint32_t total);  // work of launch_fftg_ref and launch_fftg_pipe
 template <class T, class IN, class S>
 void launch_fftg_ref(const IN* pics, const S* sums, const T* hx, const T* hy, const size2* begins, size2 src,
                      size2 side, uint32_t nb, cplx<T>* spectra, void* work, hipStream_t st);
-// as launch_fft_pipe; work: fftg_work_bytes(.., total, true) bytes
+// as launch_fft_pipe without corr_out; work: fftg_work_bytes(.., total) bytes
 template <class T, class IN, class S>
 void launch_fftg_pipe(const IN* pics, const S* sums, const T* hx, const T* hy, const size2* begins, size2 src,
                       size2 side, uint32_t nb, uint32_t total, const cplx<T>* spectra, int fit, data_index<T>* maxes,
-                      T* neigh, double* offsets, double* coefs, T* corr_out, void* work, hipStream_t st);
+                      T* neigh, double* offsets, double* coefs, void* work, hipStream_t st);
 // prepared slices -> (2s.x x 2s.y) circular correlation buffers; spectra: nb ROIs'
 // spectra (fftg_spectrum_bytes each), work: `chunk` slices of half spectra
 template <class T>

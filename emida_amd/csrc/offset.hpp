@@ -244,7 +244,7 @@ struct emida_offset_s {
             }
             parts[5] = al256(tn * cross.y * sizeof(uint32_t));
         } else if (fftg) {
-            parts[2] = al256(fftg_work_bytes(T == EMIDA_F64, slice, (uint32_t)tn, true));  // half spectra + corr
+            parts[2] = al256(fftg_work_bytes(T == EMIDA_F64, slice, (uint32_t)tn));  // half spectra
         }
         size_t sum = 0;
         for (int i = 0; i < kParts; ++i) sum += parts[i];
@@ -396,7 +396,7 @@ struct emida_offset_s {
                     if (!std::is_same<IT, uint16_t>::value)
                         launch_sum<IT, ST>(pic, sums, d_begins, src, slice, nb, nb, compute);
                     if (fftg) {
-                        void* work = dmalloc(fftg_ref_work_bytes(T == EMIDA_F64, slice, nb));
+                        void* work = dmalloc(fftg_work_bytes(T == EMIDA_F64, slice, nb));
                         try {
                             launch_fftg_ref<TT, IT, ST>(pic, sums, (const TT*)d_hx, (const TT*)d_hy, d_begins, src,
                                                         slice, nb, (cplx<TT>*)d_ref, work, compute);
@@ -500,7 +500,7 @@ struct emida_offset_s {
             }
         } else if (fftg) {
             d_ref = alloc(fftg_spectrum_bytes(T == EMIDA_F64, slice) * nb);
-            if (!resident_only) d_corr = alloc(fftg_work_bytes(T == EMIDA_F64, slice, total, true));
+            if (!resident_only) d_corr = alloc(fftg_work_bytes(T == EMIDA_F64, slice, total));
         } else {
             const size_t m = fft_padded(side);
             const size_t spec = (m / 2 + 1) * m * 2 * t_bytes();
@@ -533,7 +533,7 @@ struct emida_offset_s {
             throw unsupported_error("cross_corr_fft, get_cu_pic, get_cu_temp: 2s must be a power of two per axis");
         const size_t buf = (size_t)4 * slice.area() * t_bytes();
         const size_t spec = (size_t)(slice.x + 1) * 2 * slice.y * 2 * t_bytes();
-        seam_chunk = fftg_chunk(dbl, slice, std::max(total, nb), 0);
+        seam_chunk = fftg_chunk(dbl, slice, std::max(total, nb));
         d_seam_pic = alloc(buf * total);
         d_seam_temp = alloc(spec * nb);
         d_seam_res = alloc(buf * std::max(total, nb));
@@ -704,8 +704,7 @@ struct emida_offset_s {
                     if (fftg)
                         launch_fftg_pipe<TT, IT, ST>(pics, sums, (const TT*)d_hx, (const TT*)d_hy, d_begins, src,
                                                      slice, nb, tn, (const cplx<TT>*)d_ref, fit,
-                                                     (data_index<TT>*)maxes, (TT*)neigh, offsets, coefs, nullptr,
-                                                     sc.corr, st);
+                                                     (data_index<TT>*)maxes, (TT*)neigh, offsets, coefs, sc.corr, st);
                     else
                         launch_fft_pipe<TT, IT, ST>(pics, sums, (const TT*)d_hx, (const TT*)d_hy, d_begins, src,
                                                     side, nb, tn, (const cplx<TT>*)d_ref, fit,
