@@ -77,8 +77,8 @@ struct fft_plan {
     static constexpr int WAVES_PER_SIMD = WAVES_PER_SIMD_RAW < 1 ? 1 : (WAVES_PER_SIMD_RAW > 4 ? 4 : WAVES_PER_SIMD_RAW);
 };
 
-static __device__ cplx<float> g_tw_f[2 * kTwMaxM - 4];
-static __device__ cplx<double> g_tw_d[2 * kTwMaxM - 4];
+static __device__ cplx<float> g_tw_f[kTwElems];
+static __device__ cplx<double> g_tw_d[kTwElems];
 
 template <class T>
 const cplx<T>* fft_twiddles() {
@@ -89,10 +89,10 @@ const cplx<T>* fft_twiddles() {
     std::lock_guard<std::mutex> lock(mu);
     if ((int)per_device.size() <= dev) per_device.resize(dev + 1, {nullptr, nullptr});
     if (!per_device[dev].first) {
-        std::vector<cplx<float>> hf(2 * kTwMaxM - 4);
-        std::vector<cplx<double>> hd(2 * kTwMaxM - 4);
+        std::vector<cplx<float>> hf(kTwElems);
+        std::vector<cplx<double>> hd(kTwElems);
         const long double pi = 3.141592653589793238462643383279502884L;
-        for (int m = 4; m <= kTwMaxM; m *= 2)
+        auto fill = [&](int m) {
             for (int t = 0; t < m; ++t) {
                 const long double a = 2 * pi * t / m;
                 long double c = cosl(a), sn = sinl(a);
@@ -100,9 +100,12 @@ const cplx<T>* fft_twiddles() {
                     c = (t == 0) ? 1 : (2 * t == m ? -1 : 0);
                     sn = (4 * t == m) ? 1 : (4 * t == 3 * m ? -1 : 0);
                 }
-                hd[m - 4 + t] = cplx<double>{(double)c, (double)-sn};
-                hf[m - 4 + t] = cplx<float>{(float)c, (float)-sn};
+                hd[tw_offset(m) + t] = cplx<double>{(double)c, (double)-sn};
+                hf[tw_offset(m) + t] = cplx<float>{(float)c, (float)-sn};
             }
+        };
+        for (int m = 4; m <= kTwMaxM; m *= 2) fill(m);
+        for (int m : {192, 384}) fill(m);
         EMIDA_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_tw_f), hf.data(), hf.size() * sizeof(cplx<float>)));
         EMIDA_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_tw_d), hd.data(), hd.size() * sizeof(cplx<double>)));
         void *pf = nullptr, *pd = nullptr;

@@ -326,7 +326,7 @@ struct fft_args {
 // Copy of the M-entry table into LDS.
 template <class T, int M>
 __device__ __forceinline__ void load_twiddles(cplx<T>* tw, const cplx<T>* table, int tid, int nt) {
-    for (int t = tid; t < M; t += nt) tw[t] = table[M - 4 + t];
+    for (int t = tid; t < M; t += nt) tw[t] = table[tw_offset(M) + t];
 }
 // The same values laid out [n][k] = W_M^(n k), n < M / R, k < R, rows of R + 1
 // (M + M / R elements).
@@ -334,7 +334,7 @@ template <class T, int M, int R>
 __device__ __forceinline__ void load_twiddles_2d(cplx<T>* tw, const cplx<T>* table, int tid, int nt) {
     for (int t = tid; t < M + M / R; t += nt) {
         const int n = t / (R + 1), k = t % (R + 1);
-        tw[t] = table[M - 4 + (k < R ? n * k % M : 0)];
+        tw[t] = table[tw_offset(M) + (k < R ? n * k % M : 0)];
     }
 }
 

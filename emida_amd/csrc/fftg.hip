@@ -2,7 +2,7 @@
 // fft256.hip) do not take: non-square slices, double slices of side 65..256 and float
 // slices of side 129..256 (transforms of up to 512 x 512).  cuFFT plans any
 // 2s.x x 2s.y transform for the reference (src/gpu_offset.hpp:121-123,171-183); here
-// the transform is Mx x My, each the power of two >= 2s of its axis, with the same
+// the transform is Mx x My, each the power of two >= 2s of its axis (or 192 or 384), with the same
 // correlation values (zero padding beyond 2s changes no shift |d| < s), read through
 // the reference's 2s.x x 2s.y layout as in fft.hip.
 //
@@ -24,10 +24,11 @@
 // A transform runs on L lanes of one wave with R = M / L values each in registers and one
 // transpose through LDS (fft_common.hpp).
 //
-// Bound: the half spectra in HBM.  8 patterns x 81 ROIs of 96 x 96 in double (256 x 256):
-// 0.77 GB written and read, 240 us (rows 35, columns 119, inverse rows 86); radix-4 passes through LDS, a staged column tile and
-// the correlation written for a peak kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in
-// float (512 x 256): 381 us, before 606 us.
+// Bound: the half spectra in HBM.  8 patterns x 81 ROIs of 96 x 96 in double (192 x 192):
+// 0.58 GB written and read, 197 us (rows 43, columns 75, inverse rows 78); radix-4 passes
+// through LDS over 256 x 256, a staged column tile and the correlation written for a peak
+// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 305 us (sums
+// 20, rows 62, columns 89, inverse rows 123), before 606 us.
 //
 // Scale: the pattern's spectrum comes out doubled (the omitted split factor); the
 // stored reference spectrum is 2 s.x s.y / (Mx My) times the true one (the same
@@ -46,23 +47,59 @@ namespace {
 
 constexpr int kGNT = 256;  // threads of every kernel
 
-// Lanes and values per lane of an M-point transform.
-constexpr int glanes(int m) { return m >= 256 ? 16 : m >= 64 ? 8 : m >= 16 ? 4 : 2; }
-constexpr int gregs(int m) { return m / glanes(m); }
-// LDS of one lane group, in T: the transpose scratch of the real or the imaginary parts,
-// which also holds a whole real row.  Half of a complex scratch: twice the workgroups per CU
-// (256-point transforms in double: 39 KB instead of 74).
-constexpr int gslot(int m) { return glanes(m) * (gregs(m) + 1); }
+// Transform lengths: powers of two, and 192 and (float) 384 as three transforms of a third of
+// the length (every third input) and 3-point DFTs: they move 25% fewer bytes per axis than 256
+// and 512 (161 x 95 in float, 576 slices: 250 us with 384 x 192, 322 with 512 x 256; 96 x 96 in
+// double, 648 slices: 196 and 245).  384 in double spills (161 x 95: 367 and 254 us); 48 and 96
+// gain less in bytes than the longer register transform costs (48 x 24 in float: 229 and 172).
+constexpr bool gthree(int m) { return m % 3 == 0; }
+constexpr int gbase(int m) { return gthree(m) ? m / 3 : m; }  // length of the transforms in registers
+constexpr int glanes(int m) { return gbase(m) >= 256 ? 16 : gbase(m) >= 64 ? 8 : gbase(m) >= 16 ? 4 : 2; }
+constexpr int gsub(int m) { return gbase(m) / glanes(m); }  // values per lane of one of them
+constexpr int gregs(int m) { return m / glanes(m); }        // values per lane
+// Place of a lane's value r: time (input of the forward, output of the inverse transform) ...
+__device__ __forceinline__ constexpr int gtime(int m, int r, int lane) {
+    const int n = glanes(m) * (r % gsub(m)) + lane;
+    return gthree(m) ? 3 * n + r / gsub(m) : n;
+}
+// ... and frequency.
+__device__ __forceinline__ constexpr int gfreq(int m, int r, int lane) {
+    const int q = r / gsub(m), i = r % gsub(m) / glanes(m), k2 = r % gsub(m) % glanes(m);
+    return lane + glanes(m) * i + gsub(m) * k2 + gbase(m) * q;
+}
+// With at most M / 2 input values the second half of every register transform is zero.
+constexpr bool gzero(int m, int r) { return r % gsub(m) >= gsub(m) / 2; }
+
+// LDS: twiddles (complex): [n][k] of the register transforms, then W_M^k and W_M^2k; per lane
+// group, in T: the transpose scratch of the real or the imaginary parts, which also holds a
+// whole real row.  Half of a complex scratch: twice the workgroups per CU (256-point
+// transforms in double: 39 KB instead of 74).
+constexpr int gtw(int m) { return glanes(m) * (gsub(m) + 1) + (gthree(m) ? 2 * gbase(m) : 0); }
+constexpr int gslot(int m) { return gthree(m) ? m + 8 : glanes(m) * (gsub(m) + 1); }
 template <class T>
 constexpr size_t glds(int m) {
-    return (size_t)(2 + kGNT / glanes(m)) * gslot(m) * sizeof(T);  // twiddles (complex), slots
+    return (2 * (size_t)gtw(m) + (size_t)(kGNT / glanes(m)) * gslot(m)) * sizeof(T);
 }
+template <class T, int M>
+__device__ __forceinline__ void gload_twiddles(cplx<T>* tw, const cplx<T>* table, int tid) {
+    constexpr int P = gbase(M);
+    load_twiddles_2d<T, P, gsub(M)>(tw, table, tid, kGNT);
+    if constexpr (gthree(M)) {
+        cplx<T>* t3 = tw + glanes(M) * (gsub(M) + 1);
+        for (int k = tid; k < P; k += kGNT) {
+            t3[k] = table[tw_offset(M) + k];
+            t3[P + k] = table[tw_offset(M) + 2 * k];
+        }
+    }
+}
+
+constexpr double kR3 = 0.8660254037844386;  // sin(pi / 3)
 
 // fft_fwd and fft_inv of fft_common.hpp with the transpose in two passes, real parts then
 // imaginary parts, through L (R + 1) values of T.
-template <class T, int M, bool HALF_ZERO>
-__device__ __forceinline__ void gfft_fwd(cplx<T> (&x)[gregs(M)], int lane, T* scr, const cplx<T>* tw) {
-    constexpr int L = glanes(M), R = gregs(M), Q = R / L;
+template <class T, int R, int L, bool HALF_ZERO>
+__device__ __forceinline__ void gfft_fwd_reg(cplx<T> (&x)[R], int lane, T* scr, const cplx<T>* tw) {
+    constexpr int Q = R / L;
     dft_reg<T, R, false, HALF_ZERO>(x);
 #pragma unroll
     for (int k1 = 1; k1 < R; ++k1) x[k1] = cmul(x[k1], tw[tw_index<R, true>(lane, k1)]);
@@ -91,9 +128,9 @@ __device__ __forceinline__ void gfft_fwd(cplx<T> (&x)[gregs(M)], int lane, T* sc
     }
 }
 
-template <class T, int M>
-__device__ __forceinline__ void gfft_inv(cplx<T> (&x)[gregs(M)], int lane, T* scr, const cplx<T>* tw) {
-    constexpr int L = glanes(M), R = gregs(M), Q = R / L;
+template <class T, int R, int L>
+__device__ __forceinline__ void gfft_inv_reg(cplx<T> (&x)[R], int lane, T* scr, const cplx<T>* tw) {
+    constexpr int Q = R / L;
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
         cplx<T> y[L];
@@ -122,6 +159,61 @@ __device__ __forceinline__ void gfft_inv(cplx<T> (&x)[gregs(M)], int lane, T* sc
     for (int k1 = 0; k1 < R; ++k1) x[k1] = cplx<T>{re[k1], scr[lane * (R + 1) + k1]};
     wave_sync();
     dft_reg<T, R, true>(x);
+}
+
+// M-point transforms: registers in gtime order to gfreq order and back.  HALF_ZERO: the inputs
+// with gzero are zero.
+template <class T, int M, bool HALF_ZERO>
+__device__ __forceinline__ void gfft_fwd(cplx<T> (&x)[gregs(M)], int lane, T* scr, const cplx<T>* tw) {
+    using C = cplx<T>;
+    constexpr int R = gsub(M), L = glanes(M), P = gbase(M);
+    if constexpr (!gthree(M)) {
+        gfft_fwd_reg<T, R, L, HALF_ZERO>(x, lane, scr, tw);
+    } else {
+        C(&x0)[R] = *reinterpret_cast<C(*)[R]>(&x[0]);
+        C(&x1)[R] = *reinterpret_cast<C(*)[R]>(&x[R]);
+        C(&x2)[R] = *reinterpret_cast<C(*)[R]>(&x[2 * R]);
+        gfft_fwd_reg<T, R, L, HALF_ZERO>(x0, lane, scr, tw);
+        gfft_fwd_reg<T, R, L, HALF_ZERO>(x1, lane, scr, tw);
+        gfft_fwd_reg<T, R, L, HALF_ZERO>(x2, lane, scr, tw);
+        const C* t3 = tw + L * (R + 1);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int k = gfreq(P, r, lane);
+            const C a = x[r], b = cmul(x[R + r], t3[k]), c = cmul(x[2 * R + r], t3[P + k]);
+            const C s = cadd(b, c), d = csub(b, c), m{a.re - T(0.5) * s.re, a.im - T(0.5) * s.im};
+            const C t{T(kR3) * d.im, T(-kR3) * d.re};  // -i sin(pi/3) (b - c)
+            x[r] = cadd(a, s);
+            x[R + r] = cadd(m, t);
+            x[2 * R + r] = csub(m, t);
+        }
+    }
+}
+
+template <class T, int M>
+__device__ __forceinline__ void gfft_inv(cplx<T> (&x)[gregs(M)], int lane, T* scr, const cplx<T>* tw) {
+    using C = cplx<T>;
+    constexpr int R = gsub(M), L = glanes(M), P = gbase(M);
+    if constexpr (!gthree(M)) {
+        gfft_inv_reg<T, R, L>(x, lane, scr, tw);
+    } else {
+        const C* t3 = tw + L * (R + 1);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int k = gfreq(P, r, lane);
+            const C a = x[r], s = cadd(x[R + r], x[2 * R + r]), d = csub(x[R + r], x[2 * R + r]);
+            const C m{a.re - T(0.5) * s.re, a.im - T(0.5) * s.im}, t{T(-kR3) * d.im, T(kR3) * d.re};
+            x[r] = cadd(a, s);
+            x[R + r] = cmul_conj(cadd(m, t), t3[k]);
+            x[2 * R + r] = cmul_conj(csub(m, t), t3[P + k]);
+        }
+        C(&x0)[R] = *reinterpret_cast<C(*)[R]>(&x[0]);
+        C(&x1)[R] = *reinterpret_cast<C(*)[R]>(&x[R]);
+        C(&x2)[R] = *reinterpret_cast<C(*)[R]>(&x[2 * R]);
+        gfft_inv_reg<T, R, L>(x0, lane, scr, tw);
+        gfft_inv_reg<T, R, L>(x1, lane, scr, tw);
+        gfft_inv_reg<T, R, L>(x2, lane, scr, tw);
+    }
 }
 
 }  // namespace
@@ -166,14 +258,14 @@ struct fftg_args {
 template <class T, class IN, class SUM, int MX, bool FROM_PATTERN, bool HZ>
 __global__ __launch_bounds__(kGNT, 2) void fftg_rows_kernel(fftg_args<T, IN, SUM> a) {
     using C = cplx<T>;
-    constexpr int L = glanes(MX), R = gregs(MX), NG = kGNT / L, NCX = MX / 2 + 1, RIN = HZ ? R / 2 : R;
+    constexpr int L = glanes(MX), R = gregs(MX), NG = kGNT / L, NCX = MX / 2 + 1;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C* tw = reinterpret_cast<C*>(lds_raw);
     __shared__ uint32_t red_u[kGNT / kWave];
     const int tid = threadIdx.x, g = tid / L, lane = tid % L;
-    T* slot = reinterpret_cast<T*>(tw + gslot(MX)) + gslot(MX) * g;
+    T* slot = reinterpret_cast<T*>(tw + gtw(MX)) + gslot(MX) * g;
     const uint32_t sl = blockIdx.x, sn = a.first + sl;
-    load_twiddles_2d<T, MX, R>(tw, a.twt, tid, kGNT);
+    gload_twiddles<T, MX>(tw, a.twt, tid);
 
     const IN* pic = nullptr;
     const T* pre = nullptr;
@@ -226,8 +318,9 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_kernel(fftg_args<T, IN, SUM
             wy1 = a.hy[y1];
         }
 #pragma unroll
-        for (int n1 = 0; n1 < RIN; ++n1) {
-            const int n = L * n1 + lane, nc = min(n, sx - 1);
+        for (int n1 = 0; n1 < R; ++n1) {
+            if (HZ && gzero(MX, n1)) continue;
+            const int n = gtime(MX, n1, lane), nc = min(n, sx - 1);
             T v0, v1;
             if constexpr (FROM_PATTERN) {
                 const T wx = a.hx[nc];
@@ -245,14 +338,14 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_kernel(fftg_args<T, IN, SUM
         T sre[NK], dre[NK];
         auto put = [&](auto&& part) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) slot[lane + L * (r / L) + R * (r % L)] = part(x[r]);
+            for (int r = 0; r < R; ++r) slot[gfreq(MX, r, lane)] = part(x[r]);
             wave_sync();
         };
         put([](const C& v) { return v.re; });
 #pragma unroll
         for (int i = 0; i < NK; ++i) {
             const int k = lane + L * i;
-            const T z = slot[k], m = slot[(MX - k) & (MX - 1)];
+            const T z = slot[k], m = slot[k == 0 ? 0 : MX - k];
             sre[i] = z + m;
             dre[i] = m - z;
         }
@@ -262,7 +355,7 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_kernel(fftg_args<T, IN, SUM
 #pragma unroll
         for (int i = 0; i < NK; ++i) {
             const int k = lane + L * i;
-            const T z = slot[k], m = slot[(MX - k) & (MX - 1)];
+            const T z = slot[k], m = slot[k == 0 ? 0 : MX - k];
             if (k < NCX) {
                 r0[k] = C{sre[i], z - m};
                 if (second) r0[NCX + k] = C{z + m, dre[i]};
@@ -282,11 +375,11 @@ template <class T, int MY, int MODE>
 __global__ __launch_bounds__(kGNT, 2) void fftg_cols_kernel(fftg_args<T, T, T> a, uint32_t nblk) {
     using C = cplx<T>;
     constexpr bool HZ = MODE == COLS_PIPE || MODE == COLS_SPECTRUM;
-    constexpr int L = glanes(MY), R = gregs(MY), NG = kGNT / L, RIN = HZ ? R / 2 : R;
+    constexpr int L = glanes(MY), R = gregs(MY), NG = kGNT / L;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C* tw = reinterpret_cast<C*>(lds_raw);
     const int tid = threadIdx.x, g = tid / L, lane = tid % L;
-    T* slot = reinterpret_cast<T*>(tw + gslot(MY)) + gslot(MY) * g;
+    T* slot = reinterpret_cast<T*>(tw + gtw(MY)) + gslot(MY) * g;
     const int ncx = (int)a.mx / 2 + 1;
     const uint32_t gx = div_up((uint32_t)ncx, (uint32_t)NG), b = xcd_remap(blockIdx.x, nblk);
     uint32_t sl, col;
@@ -300,15 +393,16 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_cols_kernel(fftg_args<T, T, T> a
     }
     const uint32_t roi = (a.first + sl) % a.nb;
     const int kx = (int)col * NG + g;
-    load_twiddles_2d<T, MY, R>(tw, a.twt, tid, kGNT);
+    gload_twiddles<T, MY>(tw, a.twt, tid);
     C* w = a.work + (size_t)sl * a.my * ncx + min(kx, ncx - 1);
     const int rows = HZ ? (int)a.side.y : (int)a.my;
     C x[R];
 #pragma unroll
     for (int n1 = 0; n1 < R; ++n1) x[n1] = C{T(0), T(0)};
 #pragma unroll
-    for (int n1 = 0; n1 < RIN; ++n1) {
-        const int y = L * n1 + lane;
+    for (int n1 = 0; n1 < R; ++n1) {
+        if (HZ && gzero(MY, n1)) continue;
+        const int y = gtime(MY, n1, lane);
         const C v = w[(size_t)min(y, rows - 1) * ncx];
         x[n1] = y < rows ? v : C{T(0), T(0)};
     }
@@ -316,7 +410,7 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_cols_kernel(fftg_args<T, T, T> a
     if (kx >= ncx) return;
     // the reference spectrum: in flight during the forward transform where registers allow
     auto spec_at = [&](int r) {
-        const int k = lane + L * (r / L) + R * (r % L);
+        const int k = gfreq(MY, r, lane);
         if constexpr (MODE == COLS_PIPE) return a.spectra[((size_t)roi * ncx + kx) * MY + k];
         else return a.spectra[((size_t)roi * MY + k) * ncx + kx];
     };
@@ -330,7 +424,7 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_cols_kernel(fftg_args<T, T, T> a
     if constexpr (MODE == COLS_SPECTRUM || MODE == COLS_STD_SPECTRUM) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const int k = lane + L * (r / L) + R * (r % L);
+            const int k = gfreq(MY, r, lane);
             const C v = C{x[r].re * a.scale, x[r].im * a.scale};
             if constexpr (MODE == COLS_SPECTRUM) a.spectra_out[((size_t)roi * ncx + kx) * MY + k] = v;
             else a.spectra_out[((size_t)roi * MY + k) * ncx + kx] = v;
@@ -347,7 +441,7 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_cols_kernel(fftg_args<T, T, T> a
         const int sy = (int)a.side.y, pady = MY - 2 * sy;
 #pragma unroll
         for (int n1 = 0; n1 < R; ++n1) {
-            const int y = L * n1 + lane;
+            const int y = gtime(MY, n1, lane);
             if (MODE == COLS_STD_PIPE || y <= sy || y > sy + pady) w[(size_t)y * ncx] = x[n1];
         }
     }
@@ -355,19 +449,19 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_cols_kernel(fftg_args<T, T, T> a
 
 // ---------------------------------------------------------------- kernel 3: rows, inverse
 // Output rows 2q and 2q + 1 of the reference layout of one slice, by one lane group: on
-// return lane n2 holds their columns L n1 + n2 (circular) in x[n1].re and x[n1].im.
+// return a lane holds their columns gtime (circular) in x[r].re and x[r].im.
 template <class T, int MX>
 __device__ __forceinline__ void inverse_row_pair(cplx<T> (&x)[gregs(MX)], const cplx<T>* w, int q, int sy, int pady,
                                                  int lane, T* slot, const cplx<T>* tw) {
     using C = cplx<T>;
-    constexpr int L = glanes(MX), R = gregs(MX), NCX = MX / 2 + 1, S = MX / 2;
+    constexpr int R = gregs(MX), NCX = MX / 2 + 1, S = MX / 2;
     // reference-layout row r <= s is circular row r, r > s is r + M - 2s
     const int ra = 2 * q, rb = 2 * q + 1;
     const C* ga_row = w + (size_t)(ra <= sy ? ra : ra + pady) * NCX;
     const C* gb_row = w + (size_t)(rb <= sy ? rb : rb + pady) * NCX;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const int k = lane + L * (r / L) + R * (r % L);
+        const int k = gfreq(MX, r, lane);
         const bool mirror = k > S;
         const int col = mirror ? MX - k : k;
         C ga = ga_row[col], gb = gb_row[col];
@@ -393,9 +487,9 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_inv_kernel(fftg_args<T, T, 
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C* tw = reinterpret_cast<C*>(lds_raw);
     const int tid = threadIdx.x, g = tid / L, lane = tid % L;
-    T* slot = reinterpret_cast<T*>(tw + gslot(MX)) + gslot(MX) * g;
+    T* slot = reinterpret_cast<T*>(tw + gtw(MX)) + gslot(MX) * g;
     const uint32_t sl = blockIdx.x, sn = a.first + sl;
-    load_twiddles_2d<T, MX, R>(tw, a.twt, tid, kGNT);
+    gload_twiddles<T, MX>(tw, a.twt, tid);
     __syncthreads();
     const C* w = a.work + (size_t)sl * a.my * NCX;
     // reference-layout index k <= s is circular position k, k > s is k + M - 2s
@@ -409,28 +503,31 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_inv_kernel(fftg_args<T, T, 
         inverse_row_pair<T, MX>(x, w, q, sy, pady, lane, slot, tw);
         const uint32_t ia = 2 * (uint32_t)q * a.out.x, ib = ia + a.out.x;
         if constexpr (PEAK) {
-            // a thread meets its positions in index order, so strictly larger keeps the lowest
+            // the row's largest value and its first column, row a before row b; later rows have
+            // larger indices, so strictly larger keeps the lowest
             T va = best, vb;
-            int ca = -1, cb = -1;
+            int ca = MX, cb = MX;
 #pragma unroll
             for (int n1 = 0; n1 < R; ++n1) {
-                const int c = L * n1 + lane;
-                if ((c <= sx || c > sx + padx) && x[n1].re > va) va = x[n1].re, ca = c;
+                const int c = gtime(MX, n1, lane);
+                const T v = x[n1].re;
+                if ((c <= sx || c > sx + padx) && (v > va || (gthree(MX) && v == va && c < ca && ca < MX))) va = v, ca = c;
             }
             vb = va;
 #pragma unroll
             for (int n1 = 0; n1 < R; ++n1) {
-                const int c = L * n1 + lane;
-                if ((c <= sx || c > sx + padx) && x[n1].im > vb) vb = x[n1].im, cb = c;
+                const int c = gtime(MX, n1, lane);
+                const T v = x[n1].im;
+                if ((c <= sx || c > sx + padx) && (v > vb || (gthree(MX) && v == vb && c < cb && cb < MX))) vb = v, cb = c;
             }
-            if (ca >= 0) bi = ia + (uint32_t)(ca <= sx ? ca : ca - padx);
-            if (cb >= 0) bi = ib + (uint32_t)(cb <= sx ? cb : cb - padx);
+            if (ca < MX) bi = ia + (uint32_t)(ca <= sx ? ca : ca - padx);
+            if (cb < MX) bi = ib + (uint32_t)(cb <= sx ? cb : cb - padx);
             best = vb;
         } else {
             T* out = a.corr + (size_t)sl * a.out.area();
 #pragma unroll
             for (int n1 = 0; n1 < R; ++n1) {
-                const int c = L * n1 + lane;
+                const int c = gtime(MX, n1, lane);
                 if (c <= sx || c > sx + padx) {
                     const int rx = c <= sx ? c : c - padx;
                     out[ia + rx] = x[n1].re;
@@ -458,7 +555,7 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_inv_kernel(fftg_args<T, T, 
 #pragma unroll
             for (int n1 = 0; n1 < R; ++n1) {
                 const T even = x[n1].re, odd = x[n1].im;
-                slot[L * n1 + lane] = ry & 1 ? odd : even;
+                slot[gtime(MX, n1, lane)] = ry & 1 ? odd : even;
             }
         }
         __syncthreads();
@@ -466,7 +563,7 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_inv_kernel(fftg_args<T, T, 
             const int i = t % fit, j = t / fit;
             const size2 c = clamp_pos((int)mp.x - rad + i, (int)mp.y - rad + j, cross);
             const int rx = (int)((c.x + (a.out.x / 2 + 1)) % a.out.x);
-            const T v = (reinterpret_cast<const T*>(tw + gslot(MX)) + gslot(MX) * j)[rx <= sx ? rx : rx + padx];
+            const T v = (reinterpret_cast<const T*>(tw + gtw(MX)) + gslot(MX) * j)[rx <= sx ? rx : rx + padx];
             nbv[t] = v;
             if (a.neigh) a.neigh[(size_t)sn * kk + t] = v;
         }
@@ -494,11 +591,13 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_inv_kernel(fftg_args<T, T, 
 // ---------------------------------------------------------------- launchers
 namespace {
 
-template <int N, class F>
+template <class T, int N, class F>
 void dispatch_n(uint32_t n, F&& f) {
     if constexpr (N <= 512) {
         if (n == (uint32_t)N) return f(std::integral_constant<int, N>{});
-        return dispatch_n<N * 2>(n, std::forward<F>(f));
+        if constexpr (N == 128 || (N == 256 && sizeof(T) == 4))
+            if (n == (uint32_t)(N / 2 * 3)) return f(std::integral_constant<int, N / 2 * 3>{});
+        return dispatch_n<T, N * 2>(n, std::forward<F>(f));
     } else {
         throw unsupported_error("FFT policy: transform side " + std::to_string(n) + " is beyond 512");
     }
@@ -511,7 +610,7 @@ void set_lds(K kern, size_t bytes) {
 
 template <class T, class IN, class SUM, bool FP, bool HZ>
 void run_rows(const fftg_args<T, IN, SUM>& a, hipStream_t st) {
-    dispatch_n<4>(a.mx, [&](auto mc) {
+    dispatch_n<T, 4>(a.mx, [&](auto mc) {
         constexpr int MX = decltype(mc)::value, NG = kGNT / glanes(MX);
         auto k = fftg_rows_kernel<T, IN, SUM, MX, FP, HZ>;
         static const bool once = (set_lds(k, glds<T>(MX)), true);
@@ -527,7 +626,7 @@ void run_rows(const fftg_args<T, IN, SUM>& a, hipStream_t st) {
 template <class T, int MODE>
 void run_cols(fftg_args<T, T, T> a, hipStream_t st) {
     a.npat = a.first % a.nb == 0 && a.total % a.nb == 0 ? a.total / a.nb : 0;
-    dispatch_n<4>(a.my, [&](auto mc) {
+    dispatch_n<T, 4>(a.my, [&](auto mc) {
         constexpr int MY = decltype(mc)::value;
         auto k = fftg_cols_kernel<T, MY, MODE>;
         static const bool once = (set_lds(k, glds<T>(MY)), true);
@@ -540,7 +639,7 @@ void run_cols(fftg_args<T, T, T> a, hipStream_t st) {
 
 template <class T, bool PEAK>
 void run_rows_inv(const fftg_args<T, T, T>& a, hipStream_t st) {
-    dispatch_n<4>(a.mx, [&](auto mc) {
+    dispatch_n<T, 4>(a.mx, [&](auto mc) {
         constexpr int MX = decltype(mc)::value;
         auto k = fftg_rows_inv_kernel<T, MX, PEAK>;
         static const bool once = (set_lds(k, glds<T>(MX)), true);
@@ -579,6 +678,11 @@ constexpr size_t kFftgWorkCap = (size_t)1 << 30;  // work buffer of one launch c
 
 }  // namespace
 
+uint32_t fftg_padded(bool is_double, uint32_t side) {
+    const uint32_t m = fft_padded(side);
+    return (m == 256 || (m == 512 && !is_double)) && 2 * side <= m / 4 * 3 ? m / 4 * 3 : m;
+}
+
 bool fftg_needed(bool is_double, size2 side) {
     if (side.x != side.y) return true;
     const uint32_t m = fft_padded(side.x);
@@ -586,7 +690,7 @@ bool fftg_needed(bool is_double, size2 side) {
 }
 
 size_t fftg_spectrum_bytes(bool is_double, size2 side) {
-    return (size_t)(fft_padded(side.x) / 2 + 1) * fft_padded(side.y) * (is_double ? 16 : 8);
+    return (size_t)(fftg_padded(is_double, side.x) / 2 + 1) * fftg_padded(is_double, side.y) * (is_double ? 16 : 8);
 }
 
 size_t fftg_slice_work_bytes(bool is_double, size2 side) { return fftg_spectrum_bytes(is_double, side); }
@@ -617,8 +721,8 @@ void launch_fftg_ref(const IN* pics, const S* sums, const T* hx, const T* hy, co
     a.in_rows = side.y;
     a.in_cols = side.x;
     a.side = side;
-    a.mx = fft_padded(side.x);
-    a.my = fft_padded(side.y);
+    a.mx = fftg_padded(sizeof(T) == 8, side.x);
+    a.my = fftg_padded(sizeof(T) == 8, side.y);
     a.nb = nb;
     a.first = 0;
     a.total = nb;
@@ -652,8 +756,8 @@ void launch_fftg_pipe(const IN* pics, const S* sums, const T* hx, const T* hy, c
     a.in_rows = side.y;
     a.in_cols = side.x;
     a.side = side;
-    a.mx = fft_padded(side.x);
-    a.my = fft_padded(side.y);
+    a.mx = fftg_padded(sizeof(T) == 8, side.x);
+    a.my = fftg_padded(sizeof(T) == 8, side.y);
     a.nb = nb;
     a.work = (cplx<T>*)work;
     a.spectra = spectra;
@@ -687,8 +791,8 @@ void launch_fftg_corr_prepared(const T* pics, const T* ref, T* res, size2 side, 
     a.in_rows = side.y;
     a.in_cols = side.x;
     a.side = side;
-    a.mx = fft_padded(side.x);
-    a.my = fft_padded(side.y);
+    a.mx = fftg_padded(sizeof(T) == 8, side.x);
+    a.my = fftg_padded(sizeof(T) == 8, side.y);
     a.nb = nb;
     a.work = (cplx<T>*)work;
     a.spectra_out = spectra;

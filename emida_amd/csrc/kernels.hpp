@@ -124,9 +124,11 @@ void mfma_refine_bounds(int mode, size2 s, bool t_double, double& tol_rel, doubl
 
 // ---- fft.hip, fft256.hip
 // W_M^t = exp(-2 pi i t / M) for every power of two 4 <= M <= kTwMaxM, the table of M at
-// offset M - 4 (M entries), rounded from extended precision; a static device array per
-// GPU, filled on first use (no allocation).
+// offset M - 4 (M entries), then for M = 192 and 384 (tw_offset), rounded from
+// extended precision; a static device array per GPU, filled on first use (no allocation).
 constexpr int kTwMaxM = 512;
+constexpr int kTwElems = 2 * kTwMaxM - 4 + 192 + 384;
+__host__ __device__ constexpr int tw_offset(int m) { return m % 3 ? m - 4 : 2 * kTwMaxM - 4 + m - 192; }
 template <class T>
 const cplx<T>* fft_twiddles();
 // Largest padded FFT side of the single-kernel pipelines: 128 for double, 256 for
@@ -136,6 +138,8 @@ int fft_max_side(bool is_double);
 constexpr uint32_t kFftMaxSlice = 256;
 // Transform side M of a slice side s: the power of two >= 2s (at least 4).
 uint32_t fft_padded(uint32_t side);
+// The same for the general path: also 192 and, in float, 384.
+uint32_t fftg_padded(bool is_double, uint32_t side);
 // Reference spectra: prepared reference slices -> half spectra in the layout the
 // pipeline kernel reads ((M/2+1) columns x M bit-reversed rows per ROI).
 template <class T, class IN, class S>
