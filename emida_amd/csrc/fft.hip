@@ -19,8 +19,8 @@
 //
 // FFT scheme.  A length-M transform is computed by a group of L lanes of
 // one wave, each lane holding R = M/L values: an R-point DFT in registers over
-// n = L*n1 + n2 (lane n2), a twiddle W_M^(n2*k1), one transpose through the group's
-// LDS scratch, and L-point DFTs in registers.  Lane j then holds X[k] for
+// n = L*n1 + n2 (lane n2), one transpose through the group's LDS scratch, and L-point DFTs
+// in registers with the twiddles W_M^(n2*k1) folded into their butterflies.  Lane j then holds X[k] for
 // k = (j + L*i) + R*k2 (i < R/L, k2 < L) - the "frequency layout".  The
 // inverse starts from that layout and ends in natural order, so the product with the
 // reference spectrum (stored in the same layout) needs no reordering.
@@ -69,7 +69,7 @@ struct fft_plan {
     static constexpr int CS = ((need + 7) / 16) * 16 + 8;
     static constexpr int P_OFF = NC * CS - S * S / 2;  // prepared ROI (S*S reals) at the end
     static_assert(P_OFF >= (S / 2) * CS, "prepared ROI overlaps the row stage");
-    static constexpr size_t lds_bytes = (size_t)(NC * CS + M + L) * sizeof(cplx<T>);  // + twiddles [L][R + 1]
+    static constexpr size_t lds_bytes = (size_t)(NC * CS + twist_elems(M, R)) * sizeof(cplx<T>);  // + twiddles
     // waves per SIMD the LDS allows (160 KiB per CU, 4 SIMDs); registers are
     // budgeted for exactly that many
     static constexpr int WG_PER_CU = (int)((160 * 1024) / (lds_bytes + kStaticLds));
@@ -106,6 +106,13 @@ const cplx<T>* fft_twiddles() {
         };
         for (int m = 4; m <= kTwMaxM; m *= 2) fill(m);
         for (int m : {192, 384}) fill(m);
+        for (int m = 4; m <= kTwMaxM; m *= 2)
+            for (int t = 0; t < m / 4; ++t) {
+                // the tangent over the rounded cosine: their product is the sine to one rounding
+                const long double c = cosl(2 * pi * t / m), sn = sinl(2 * pi * t / m);
+                hd[tan_offset(m) + t] = cplx<double>{(double)c, (double)(sn / (double)c)};
+                hf[tan_offset(m) + t] = cplx<float>{(float)c, (float)(sn / (float)c)};
+            }
         EMIDA_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_tw_f), hf.data(), hf.size() * sizeof(cplx<float>)));
         EMIDA_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_tw_d), hd.data(), hd.size() * sizeof(cplx<double>)));
         void *pf = nullptr, *pd = nullptr;
@@ -211,7 +218,7 @@ __global__ __launch_bounds__((fft_plan<T, M>::NT), (fft_plan<T, M>::WAVES_PER_SI
         }
         double lv[kLsqPer];
         load_lsq<NT>(lv, a.lsq, kk, tid);
-        load_twiddles_2d<T, M, R>(tw, a.twt, tid, NT);
+        load_twist<T, M, R>(tw, a.twt, tid, NT);
         store_lsq<NT>(lsq_s, lv, kk, tid);
         T mean;
         if constexpr (std::is_same<IN, uint16_t>::value) {
@@ -238,7 +245,7 @@ __global__ __launch_bounds__((fft_plan<T, M>::NT), (fft_plan<T, M>::WAVES_PER_SI
         for (int e = tid; e < s * s; e += NT) pre[e] = src[e];
         double lv[kLsqPer];
         load_lsq<NT>(lv, a.lsq, kk, tid);
-        load_twiddles_2d<T, M, R>(tw, a.twt, tid, NT);
+        load_twist<T, M, R>(tw, a.twt, tid, NT);
         store_lsq<NT>(lsq_s, lv, kk, tid);
     }
     __syncthreads();
@@ -270,7 +277,7 @@ __global__ __launch_bounds__((fft_plan<T, M>::NT), (fft_plan<T, M>::WAVES_PER_SI
             }
         }
         C* slot = B + p * CS;
-        fft_fwd<T, R, L, M, true, true>(x, lane, slot, tw);
+        fft_fwd<T, R, L, M, true>(x, lane, slot, tw);
 #pragma unroll
         for (int i = 0; i < Q; ++i)
 #pragma unroll
@@ -312,7 +319,7 @@ __global__ __launch_bounds__((fft_plan<T, M>::NT), (fft_plan<T, M>::WAVES_PER_SI
     __syncthreads();  // row spectra consumed; slots become column scratch
     if (c < S) {
         C* slot = B + c * CS;
-        fft_fwd<T, R, L, M, true, true>(x, lane, slot, tw);
+        fft_fwd<T, R, L, M, true>(x, lane, slot, tw);
         if (c == 0) {
             // split the packed real columns: P0[k] = (Z[k] + conj(Z[-k]))/2,
             // PS[k] = (Z[k] - conj(Z[-k]))/(2i), then H0 + i HS (PIPE) or the two
@@ -350,7 +357,7 @@ __global__ __launch_bounds__((fft_plan<T, M>::NT), (fft_plan<T, M>::WAVES_PER_SI
             }
         }
         if constexpr (PIPE) {
-            fft_inv<T, R, L, M, true>(x, lane, slot, tw);
+            fft_inv<T, R, L, M>(x, lane, slot, tw);
             if (c == 0) {
                 C* slot_s = B + S * CS;
 #pragma unroll
@@ -404,7 +411,7 @@ __global__ __launch_bounds__((fft_plan<T, M>::NT), (fft_plan<T, M>::WAVES_PER_SI
         T vmax = -(T)__builtin_huge_val();
         if (q < S && (in_a || in_b)) {
             C* slot = B + q * CS;
-            fft_inv<T, R, L, M, true>(x, lane, slot, tw);
+            fft_inv<T, R, L, M>(x, lane, slot, tw);
             // the maximum through selects (no branch per element); positions outside
             // the reference layout count as -inf (there are none when M = 2s)
             const T lo = -(T)__builtin_huge_val();

@@ -1,6 +1,15 @@
 // Building blocks of the LDS-resident FFT kernels (fft.hip, fft256.hip): complex
 // helpers, the in-register radix-2 DFT, the two-level transform over a lane group
 // and the reference's prepare expression.
+//
+// The single-kernel paths are bound by vector instructions, so the transforms count them: a
+// product for every twiddle between the levels and radix-4 passes took 332 per lane and 16
+// values of an inverse 128-point transform, the folded butterflies below 296, with 8 twiddles
+// read from LDS instead of 15.  25600 slices of 64 px in float: 622 -> 606 us; 6400 in
+// double: 501 -> 476 us; 6400 of 128 px in float: 861 -> 841 us; 648 of 96 px in double
+// (fftg.hip): 221 -> 205 us.  RMS error of a correlation against 64 bits (128 bits for
+// double), white noise: 64 px 2.45e-7 -> 2.33e-7 and 4.6e-16 -> 4.0e-16, 128 px 2.78e-7 ->
+// 2.52e-7.
 #pragma once
 
 #include <type_traits>
@@ -32,34 +41,16 @@ __device__ __forceinline__ cplx<T> hadamard(cplx<T> p, cplx<T> r) {
     return {p.re * r.re + p.im * r.im, -p.re * r.im + p.im * r.re};
 }
 
-// exp(-2 pi i j / 16), j < 8: correctly rounded cos/sin of multiples of pi/8.
-constexpr double kC1 = 0.9238795325112867, kS1 = 0.3826834323650898, kR2 = 0.7071067811865476;
-
-// v * W_16^j (conjugate twiddle when INV); j is a compile-time constant after unrolling.
-template <class T, bool INV>
-__device__ __forceinline__ cplx<T> twiddle16(cplx<T> v, int j) {
-    const T sg = INV ? T(-1) : T(1);
-    switch (j) {
-        case 0: return v;
-        case 4: return INV ? cplx<T>{-v.im, v.re} : cplx<T>{v.im, -v.re};
-        case 2: return cmul(v, cplx<T>{T(kR2), sg * T(-kR2)});
-        case 6: return cmul(v, cplx<T>{T(-kR2), sg * T(-kR2)});
-        case 1: return cmul(v, cplx<T>{T(kC1), sg * T(-kS1)});
-        case 3: return cmul(v, cplx<T>{T(kS1), sg * T(-kC1)});
-        case 5: return cmul(v, cplx<T>{T(-kS1), sg * T(-kC1)});
-        default: return cmul(v, cplx<T>{T(-kC1), sg * T(-kS1)});  // 7
-    }
+// cos and tan of 2 pi q / 32, q < 8; the tangent as the sine over the rounded cosine, so
+// that their product is the sine to one rounding.
+template <class T>
+constexpr T cos32(int q) {
+    return T(q == 0 ? 1 : q == 1 ? 0.9807852804032304 : q == 2 ? 0.9238795325112867 : q == 3 ? 0.8314696123025452
+           : q == 4 ? 0.7071067811865476 : q == 5 ? 0.5555702330196022 : q == 6 ? 0.3826834323650898 : 0.19509032201612828);
 }
-
-// v * W_32^j, j < 16: correctly rounded cos/sin of multiples of pi/16.
-template <class T, bool INV>
-__device__ __forceinline__ cplx<T> twiddle32(cplx<T> v, int j) {
-    if (j % 2 == 0) return twiddle16<T, INV>(v, j / 2);
-    constexpr double c1 = 0.9807852804032304, s1 = 0.19509032201612828;  // pi/16
-    constexpr double c3 = 0.8314696123025452, s3 = 0.5555702330196022;   // 3 pi/16
-    const double co = j == 1 ? c1 : j == 3 ? c3 : j == 5 ? s3 : j == 7 ? s1 : j == 9 ? -s1 : j == 11 ? -s3 : j == 13 ? -c3 : -c1;
-    const double si = j == 1 || j == 15 ? s1 : j == 3 || j == 13 ? s3 : j == 5 || j == 11 ? c3 : c1;
-    return cmul(v, cplx<T>{T(co), T(INV ? si : -si)});
+template <class T>
+constexpr T tan32(int q) {
+    return q == 0 ? T(0) : T(cos32<double>(8 - q) / (double)cos32<T>(q));
 }
 
 __host__ __device__ constexpr int ilog2(int n) { return n <= 1 ? 0 : 1 + ilog2(n / 2); }
@@ -69,107 +60,86 @@ __host__ __device__ constexpr int brev_c(int v, int bits) {
     return r;
 }
 
-// v * W_16^j for any j (W_16^(j + 8) = -W_16^j).
-template <class T, bool INV>
-__device__ __forceinline__ cplx<T> twiddle16_any(cplx<T> v, int j) {
-    j &= 15;
-    const cplx<T> w = twiddle16<T, INV>(v, j & 7);
-    return j >= 8 ? cplx<T>{-w.re, -w.im} : w;
+// Radix-2 butterflies (a, b) -> (a + w b, a - w b), decimation in time: the twiddle before
+// the butterfly folds into it.  w = exp(-+ i p) = cos p (1 -+ i tan p), 0 <= p < pi / 2 (INV:
+// upper sign conjugated): u = b / cos p is two fused operations, a +- cos p u four, six in
+// all where a product and two sums take eight.  The rounding of u scales with the product
+// itself (u times cos p).  TURN: w times a quarter turn more.
+template <class T, bool INV, bool TURN>
+__device__ __forceinline__ void butterfly_tan(cplx<T>& a, cplx<T>& b, T c, T t) {
+    const T ur = fma(INV ? -t : t, b.im, b.re), ui = fma(INV ? t : -t, b.re, b.im);
+    // w b / c, or that times -i (INV: i)
+    const T vr = TURN ? (INV ? -ui : ui) : ur, vi = TURN ? (INV ? ur : -ur) : ui;
+    const cplx<T> s = a;
+    a = cplx<T>{fma(c, vr, s.re), fma(c, vi, s.im)};
+    b = cplx<T>{fma(-c, vr, s.re), fma(-c, vi, s.im)};
+}
+// w = 1, or a quarter turn.
+template <class T, bool INV, bool TURN>
+__device__ __forceinline__ void butterfly_one(cplx<T>& a, cplx<T>& b) {
+    const cplx<T> s = a, v = TURN ? (INV ? cplx<T>{-b.im, b.re} : cplx<T>{b.im, -b.re}) : b;
+    a = cadd(s, v);
+    b = csub(s, v);
 }
 
-// 4-point DFT of (a0, a1, a2, a3) in place (forward: W_4 = -i; INV: +i); HALF_ZERO:
-// a2 = a3 = 0 (not read).
-template <class T, bool INV, bool HALF_ZERO>
-__device__ __forceinline__ void dft4(cplx<T>& a0, cplx<T>& a1, cplx<T>& a2, cplx<T>& a3) {
-    if constexpr (HALF_ZERO) {
-        const cplx<T> t0 = a0, t1 = a1;
-        a0 = cadd(t0, t1);
-        a2 = csub(t0, t1);
-        // -i t1 forward, +i t1 inverse
-        a1 = INV ? cplx<T>{t0.re - t1.im, t0.im + t1.re} : cplx<T>{t0.re + t1.im, t0.im - t1.re};
-        a3 = INV ? cplx<T>{t0.re + t1.im, t0.im - t1.re} : cplx<T>{t0.re - t1.im, t0.im + t1.re};
-    } else {
-        const cplx<T> t0 = cadd(a0, a2), t1 = csub(a0, a2), t2 = cadd(a1, a3), t3 = csub(a1, a3);
-        a0 = cadd(t0, t2);
-        a2 = csub(t0, t2);
-        a1 = INV ? cplx<T>{t1.re - t3.im, t1.im + t3.re} : cplx<T>{t1.re + t3.im, t1.im - t3.re};
-        a3 = INV ? cplx<T>{t1.re + t3.im, t1.im - t3.re} : cplx<T>{t1.re - t3.im, t1.im + t3.re};
+// 32 double points fill the registers: each half is computed where it stands, not moved
+// towards its uses (spills otherwise).
+template <class T, int N>
+__device__ __forceinline__ void hold(cplx<T> (&x)[N]) {
+    if constexpr (sizeof(T) == 8) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) asm volatile("" : "+v"(x[i].re), "+v"(x[i].im));
     }
 }
 
-// In-register DFT of N <= 32 points, natural order in and out.  N = 32: one radix-2 pass,
-// then two 16-point DFTs (even and odd outputs).  N = 16: radix 4
-// (n = n0 + 4 n1, k = k1 + 4 k0: 4-point DFTs over n1, twiddles W_16^(n0 k1), 4-point
-// DFTs over n0; 8 non-trivial twiddle products instead of radix 2's 10); smaller N:
-// radix-2 decimation in frequency.  The final digit reversal only renames registers.
+// In-register DFT of N <= 32 points, natural order in and out (the digit reversal only
+// renames registers).  HALF_ZERO: x[N/2..N-1] = 0, not read.
 template <class T, int N, bool INV, bool HALF_ZERO = false>
 __device__ __forceinline__ void dft_reg(cplx<T> (&x)[N]) {
-    static_assert(N >= 1 && N <= 32 && (N & (N - 1)) == 0, "N must be a power of two <= 32");
-    if constexpr (N == 32) {
+    static_assert(N >= 2 && N <= 32 && (N & (N - 1)) == 0, "N must be a power of two <= 32");
+    if constexpr (N == 32) {  // (in one piece its registers go to scratch)
         cplx<T> e[16], o[16];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            e[k] = HALF_ZERO ? x[k] : cadd(x[k], x[k + 16]);
-            o[k] = twiddle32<T, INV>(HALF_ZERO ? x[k] : csub(x[k], x[k + 16]), k);
+        for (int i = 0; i < 16; ++i) {
+            e[i] = x[HALF_ZERO ? 2 * i % 16 : 2 * i];
+            o[i] = x[HALF_ZERO ? 2 * i % 16 + 1 : 2 * i + 1];
         }
-        dft_reg<T, 16, INV>(e);
-        dft_reg<T, 16, INV>(o);
+        dft_reg<T, 16, INV, HALF_ZERO>(e);
+        hold(e);
+        dft_reg<T, 16, INV, HALF_ZERO>(o);
+        hold(o);
+        butterfly_one<T, INV, false>(e[0], o[0]);
+        butterfly_one<T, INV, true>(e[8], o[8]);
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            x[2 * k] = e[k];
-            x[2 * k + 1] = o[k];
+        for (int j = 1; j < 8; ++j) {
+            butterfly_tan<T, INV, false>(e[j], o[j], cos32<T>(j), tan32<T>(j));
+            butterfly_tan<T, INV, true>(e[j + 8], o[j + 8], cos32<T>(j), tan32<T>(j));
         }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            x[i] = e[i];
+            x[i + 16] = o[i];
+        }
+        hold(x);
         return;
-    }
-    if constexpr (N == 16) {
-#pragma unroll
-        for (int n0 = 0; n0 < 4; ++n0) {
-            cplx<T> a0 = x[n0], a1 = x[n0 + 4], a2, a3;
-            if constexpr (!HALF_ZERO) {
-                a2 = x[n0 + 8];
-                a3 = x[n0 + 12];
-            }
-            dft4<T, INV, HALF_ZERO>(a0, a1, a2, a3);
-            x[n0] = a0;
-            x[n0 + 4] = twiddle16_any<T, INV>(a1, n0);
-            x[n0 + 8] = twiddle16_any<T, INV>(a2, 2 * n0);
-            x[n0 + 12] = twiddle16_any<T, INV>(a3, 3 * n0);
-        }
-        cplx<T> y[16];
-#pragma unroll
-        for (int k1 = 0; k1 < 4; ++k1) {
-            cplx<T> b0 = x[4 * k1], b1 = x[4 * k1 + 1], b2 = x[4 * k1 + 2], b3 = x[4 * k1 + 3];
-            dft4<T, INV, false>(b0, b1, b2, b3);
-            y[k1] = b0;
-            y[k1 + 4] = b1;
-            y[k1 + 8] = b2;
-            y[k1 + 12] = b3;
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) x[i] = y[i];
-        return;
-    }
-    if constexpr (HALF_ZERO && N >= 2) {
-        // first pass with x[N/2..N-1] = 0: x[k] unchanged, x[k + N/2] = x[k] W^k
-#pragma unroll
-        for (int k = 0; k < N / 2; ++k) x[k + N / 2] = twiddle16<T, INV>(x[k], k * (16 / N));
-    }
-#pragma unroll
-    for (int len = HALF_ZERO ? N / 2 : N; len >= 2; len >>= 1) {
-        const int half = len / 2;
-#pragma unroll
-        for (int s0 = 0; s0 < N; s0 += len) {
-#pragma unroll
-            for (int k = 0; k < half; ++k) {
-                const cplx<T> a = x[s0 + k], b = x[s0 + k + half];
-                x[s0 + k] = cadd(a, b);
-                x[s0 + k + half] = twiddle16<T, INV>(csub(a, b), k * (16 / len));
-            }
-        }
     }
     cplx<T> y[N];
 #pragma unroll
-    for (int i = 0; i < N; ++i) y[i] = x[brev_c(i, ilog2(N))];
+    for (int i = 0; i < N; ++i) y[i] = x[HALF_ZERO ? brev_c(i, ilog2(N)) % (N / 2) : brev_c(i, ilog2(N))];
+#pragma unroll
+    for (int n = HALF_ZERO ? 4 : 2; n <= N; n *= 2) {
+#pragma unroll
+        for (int b = 0; b < N; b += n) {
+#pragma unroll
+            for (int j = 0; j < n / 2; ++j) {
+                cplx<T>&p = y[b + j], &q = y[b + j + n / 2];
+                if (j == 0) butterfly_one<T, INV, false>(p, q);
+                else if (4 * j == n) butterfly_one<T, INV, true>(p, q);
+                else if (4 * j < n) butterfly_tan<T, INV, false>(p, q, cos32<T>(32 * j / n), tan32<T>(32 * j / n));
+                else butterfly_tan<T, INV, true>(p, q, cos32<T>(32 * j / n - 8), tan32<T>(32 * j / n - 8));
+            }
+        }
+    }
 #pragma unroll
     for (int i = 0; i < N; ++i) x[i] = y[i];
 }
@@ -181,24 +151,76 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Twiddle W_M^(n k) of the two-level transforms (n < L, k < R): from a table of
-// W_M^m (m < M), or, TW2D, from a table laid out [n][k] with rows of R + 1
-// (load_twiddles_2d), where the address is a per-lane base plus a compile-time offset
-// and the odd row stride keeps the lanes of a group on distinct banks.
-template <int R, bool TW2D>
-__device__ __forceinline__ int tw_index(int n, int k) {
-    return TW2D ? n * (R + 1) + k : n * k;
+// DFT of N points x[m] W_M^(m f) (INV: conjugated), natural order: the twiddles between the
+// two levels of an M-point transform folded into the second level's butterflies.  The pass
+// that joins blocks of n points takes W_M^(f N / n + j M / n), j < n / 2: below a quarter
+// turn for j < n / 4 and n >= 4 with f < M / N, so (cos, tan) from the table, a quarter turn
+// more for the others; n = 2 reaches half a turn: w itself, a - w b as 2 a - (a + w b).
+// tab (load_twist): (cos, tan) of 2 pi t / M, t < M / 4, then W_2R^r, r < R.
+constexpr int twist_elems(int m, int r) { return m / 4 + r; }
+// F: points of the whole DFT where this is the half of its even or odd inputs.
+template <class T, int N, int M, int R, bool INV, int F = N>
+__device__ __forceinline__ void dft_twist(cplx<T> (&x)[N], const cplx<T>* tab, int f) {
+    if constexpr (N == 32) {
+        cplx<T> e[16], o[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            e[i] = x[2 * i];
+            o[i] = x[2 * i + 1];
+        }
+        dft_twist<T, 16, M, R, INV, F>(e, tab, f);
+        hold(e);
+        dft_twist<T, 16, M, R, INV, F>(o, tab, f);
+        hold(o);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const cplx<T> ct = tab[f + j * (M / 32)];
+            butterfly_tan<T, INV, false>(e[j], o[j], ct.re, ct.im);
+            butterfly_tan<T, INV, true>(e[j + 8], o[j + 8], ct.re, ct.im);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            x[i] = e[i];
+            x[i + 16] = o[i];
+        }
+        hold(x);
+        return;
+    }
+    cplx<T> y[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) y[i] = x[brev_c(i, ilog2(N))];
+    const cplx<T> w = tab[M / 4 + f * (F * R / M)];
+#pragma unroll
+    for (int b = 0; b < N; b += 2) {
+        const cplx<T> a = y[b], q = y[b + 1];
+        const T wi = INV ? -w.im : w.im;
+        const T sr = fma(-wi, q.im, fma(w.re, q.re, a.re)), si = fma(wi, q.re, fma(w.re, q.im, a.im));
+        y[b] = cplx<T>{sr, si};
+        y[b + 1] = cplx<T>{fma(T(2), a.re, -sr), fma(T(2), a.im, -si)};
+    }
+#pragma unroll
+    for (int n = 4; n <= N; n *= 2) {
+#pragma unroll
+        for (int j = 0; j < n / 4; ++j) {
+            const cplx<T> ct = tab[f * (F / n) + j * (M / n)];
+#pragma unroll
+            for (int b = 0; b < N; b += n) {
+                butterfly_tan<T, INV, false>(y[b + j], y[b + j + n / 2], ct.re, ct.im);
+                butterfly_tan<T, INV, true>(y[b + j + n / 4], y[b + j + n / 4 + n / 2], ct.re, ct.im);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = y[i];
 }
 
 // Forward transform: lane n2 holds x[n1] = input[L*n1 + n2]; on return lane j holds
 // X[(j + L*i) + R*k2] in x[i*L + k2].  scr: L*(R+1) elements of this group.
 // HALF_ZERO: the inputs x[R/2..R-1] are zero padding.
-template <class T, int R, int L, int M, bool HALF_ZERO, bool TW2D = false>
+template <class T, int R, int L, int M, bool HALF_ZERO>
 __device__ __forceinline__ void fft_fwd(cplx<T> (&x)[R], int lane, cplx<T>* scr, const cplx<T>* tw) {
     constexpr int Q = R / L;
     dft_reg<T, R, false, HALF_ZERO>(x);
-#pragma unroll
-    for (int k1 = 1; k1 < R; ++k1) x[k1] = cmul(x[k1], tw[tw_index<R, TW2D>(lane, k1)]);
 #pragma unroll
     for (int k1 = 0; k1 < R; ++k1) scr[lane * (R + 1) + k1] = x[k1];
     wave_sync();
@@ -210,7 +232,7 @@ __device__ __forceinline__ void fft_fwd(cplx<T> (&x)[R], int lane, cplx<T>* scr,
     wave_sync();
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-        dft_reg<T, L, false>(y[i]);
+        dft_twist<T, L, M, R, false>(y[i], tw, lane + L * i);
 #pragma unroll
         for (int k2 = 0; k2 < L; ++k2) x[i * L + k2] = y[i][k2];
     }
@@ -218,35 +240,23 @@ __device__ __forceinline__ void fft_fwd(cplx<T> (&x)[R], int lane, cplx<T>* scr,
 
 // Inverse (unnormalised) transform from the frequency layout to natural order:
 // on return lane n2 holds output[L*n1 + n2] in x[n1].
-// TW_FIRST: load each L-point DFT's twiddles before it.  tw and scr share LDS, so a
-// twiddle load written after a store to scr stays after it and each product waits for
-// its own load: hidden at four waves per SIMD (fft.hip), exposed at two (fft256.hip,
-// where loading first is 4% faster).
-template <class T, int R, int L, int M, bool TW2D = false, bool TW_FIRST = false>
+template <class T, int R, int L, int M>
 __device__ __forceinline__ void fft_inv(cplx<T> (&x)[R], int lane, cplx<T>* scr, const cplx<T>* tw) {
     constexpr int Q = R / L;
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-        const int k1 = lane + L * i;
-        cplx<T> w[L];
-        if constexpr (TW_FIRST) {
-#pragma unroll
-            for (int n2 = 1; n2 < L; ++n2) w[n2] = tw[tw_index<R, TW2D>(n2, k1)];
-        }
         cplx<T> y[L];
 #pragma unroll
         for (int k2 = 0; k2 < L; ++k2) y[k2] = x[i * L + k2];
         dft_reg<T, L, true>(y);
 #pragma unroll
-        for (int n2 = 0; n2 < L; ++n2)
-            scr[n2 * (R + 1) + k1] =
-                n2 == 0 ? y[0] : cmul_conj(y[n2], TW_FIRST ? w[n2] : tw[tw_index<R, TW2D>(n2, k1)]);
+        for (int n2 = 0; n2 < L; ++n2) scr[n2 * (R + 1) + lane + L * i] = y[n2];
     }
     wave_sync();
 #pragma unroll
     for (int k1 = 0; k1 < R; ++k1) x[k1] = scr[lane * (R + 1) + k1];
     wave_sync();
-    dft_reg<T, R, true>(x);
+    dft_twist<T, R, M, R, true>(x, tw, lane);
 }
 
 // Prepared pixel (src/prepare_pics.cu:36-41), no contraction.
@@ -328,14 +338,11 @@ template <class T, int M>
 __device__ __forceinline__ void load_twiddles(cplx<T>* tw, const cplx<T>* table, int tid, int nt) {
     for (int t = tid; t < M; t += nt) tw[t] = table[tw_offset(M) + t];
 }
-// The same values laid out [n][k] = W_M^(n k), n < M / R, k < R, rows of R + 1
-// (M + M / R elements).
+// The twiddles of dft_twist (twist_elems(M, R) elements).
 template <class T, int M, int R>
-__device__ __forceinline__ void load_twiddles_2d(cplx<T>* tw, const cplx<T>* table, int tid, int nt) {
-    for (int t = tid; t < M + M / R; t += nt) {
-        const int n = t / (R + 1), k = t % (R + 1);
-        tw[t] = table[tw_offset(M) + (k < R ? n * k % M : 0)];
-    }
+__device__ __forceinline__ void load_twist(cplx<T>* tw, const cplx<T>* table, int tid, int nt) {
+    for (int t = tid; t < twist_elems(M, R); t += nt)
+        tw[t] = table[t < M / 4 ? tan_offset(M) + t : tw_offset(M) + (t - M / 4) * (M / (2 * R))];
 }
 
 }  // namespace emida_amd

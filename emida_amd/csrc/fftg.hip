@@ -25,10 +25,10 @@
 // transpose through LDS (fft_common.hpp).
 //
 // Bound: the half spectra in HBM.  8 patterns x 81 ROIs of 96 x 96 in double (192 x 192):
-// 0.58 GB written and read, 197 us (rows 43, columns 75, inverse rows 78); radix-4 passes
+// 0.58 GB written and read, 183 us (rows 31, columns 71, inverse rows 72); radix-4 passes
 // through LDS over 256 x 256, a staged column tile and the correlation written for a peak
-// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 305 us (sums
-// 20, rows 62, columns 89, inverse rows 123), before 606 us.
+// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 282 us (sums
+// 20, rows 60, columns 89, inverse rows 102), before 606 us.
 //
 // Scale: the pattern's spectrum comes out doubled (the omitted split factor); the
 // stored reference spectrum is 2 s.x s.y / (Mx My) times the true one (the same
@@ -49,9 +49,10 @@ constexpr int kGNT = 256;  // threads of every kernel
 
 // Transform lengths: powers of two, and 192 and (float) 384 as three transforms of a third of
 // the length (every third input) and 3-point DFTs: they move 25% fewer bytes per axis than 256
-// and 512 (161 x 95 in float, 576 slices: 250 us with 384 x 192, 322 with 512 x 256; 96 x 96 in
-// double, 648 slices: 196 and 245).  384 in double spills (161 x 95: 367 and 254 us); 48 and 96
-// gain less in bytes than the longer register transform costs (48 x 24 in float: 229 and 172).
+// and 512 (161 x 95 in float, 576 slices: 225 us with 384 x 192, 250 with 512 x 256; 190 x 190,
+// 400: 311 and 370; 96 x 96 in double, 648: 181 and 225).  384 in double spills (161 x 95: 504
+// and 249 us); 48 and 96 gain less in bytes than the longer register transform costs (48 x 24
+// in float: 229 and 172 when both were tried).
 constexpr bool gthree(int m) { return m % 3 == 0; }
 constexpr int gbase(int m) { return gthree(m) ? m / 3 : m; }  // length of the transforms in registers
 constexpr int glanes(int m) { return gbase(m) >= 256 ? 16 : gbase(m) >= 64 ? 8 : gbase(m) >= 16 ? 4 : 2; }
@@ -70,11 +71,11 @@ __device__ __forceinline__ constexpr int gfreq(int m, int r, int lane) {
 // With at most M / 2 input values the second half of every register transform is zero.
 constexpr bool gzero(int m, int r) { return r % gsub(m) >= gsub(m) / 2; }
 
-// LDS: twiddles (complex): [n][k] of the register transforms, then W_M^k and W_M^2k; per lane
+// LDS: twiddles (complex): of the register transforms, then W_M^k and W_M^2k; per lane
 // group, in T: the transpose scratch of the real or the imaginary parts, which also holds a
 // whole real row.  Half of a complex scratch: twice the workgroups per CU (256-point
 // transforms in double: 39 KB instead of 74).
-constexpr int gtw(int m) { return glanes(m) * (gsub(m) + 1) + (gthree(m) ? 2 * gbase(m) : 0); }
+constexpr int gtw(int m) { return twist_elems(gbase(m), gsub(m)) + (gthree(m) ? 2 * gbase(m) : 0); }
 constexpr int gslot(int m) { return gthree(m) ? m + 8 : glanes(m) * (gsub(m) + 1); }
 template <class T>
 constexpr size_t glds(int m) {
@@ -83,9 +84,9 @@ constexpr size_t glds(int m) {
 template <class T, int M>
 __device__ __forceinline__ void gload_twiddles(cplx<T>* tw, const cplx<T>* table, int tid) {
     constexpr int P = gbase(M);
-    load_twiddles_2d<T, P, gsub(M)>(tw, table, tid, kGNT);
+    load_twist<T, P, gsub(M)>(tw, table, tid, kGNT);
     if constexpr (gthree(M)) {
-        cplx<T>* t3 = tw + glanes(M) * (gsub(M) + 1);
+        cplx<T>* t3 = tw + twist_elems(P, gsub(M));
         for (int k = tid; k < P; k += kGNT) {
             t3[k] = table[tw_offset(M) + k];
             t3[P + k] = table[tw_offset(M) + 2 * k];
@@ -101,8 +102,6 @@ template <class T, int R, int L, bool HALF_ZERO>
 __device__ __forceinline__ void gfft_fwd_reg(cplx<T> (&x)[R], int lane, T* scr, const cplx<T>* tw) {
     constexpr int Q = R / L;
     dft_reg<T, R, false, HALF_ZERO>(x);
-#pragma unroll
-    for (int k1 = 1; k1 < R; ++k1) x[k1] = cmul(x[k1], tw[tw_index<R, true>(lane, k1)]);
 #pragma unroll
     for (int k1 = 0; k1 < R; ++k1) scr[lane * (R + 1) + k1] = x[k1].re;
     wave_sync();
@@ -122,7 +121,7 @@ __device__ __forceinline__ void gfft_fwd_reg(cplx<T> (&x)[R], int lane, T* scr, 
     wave_sync();
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-        dft_reg<T, L, false>(y[i]);
+        dft_twist<T, L, R * L, R, false>(y[i], tw, lane + L * i);
 #pragma unroll
         for (int k2 = 0; k2 < L; ++k2) x[i * L + k2] = y[i][k2];
     }
@@ -132,15 +131,7 @@ template <class T, int R, int L>
 __device__ __forceinline__ void gfft_inv_reg(cplx<T> (&x)[R], int lane, T* scr, const cplx<T>* tw) {
     constexpr int Q = R / L;
 #pragma unroll
-    for (int i = 0; i < Q; ++i) {
-        cplx<T> y[L];
-#pragma unroll
-        for (int k2 = 0; k2 < L; ++k2) y[k2] = x[i * L + k2];
-        dft_reg<T, L, true>(y);
-#pragma unroll
-        for (int n2 = 0; n2 < L; ++n2)
-            x[i * L + n2] = n2 == 0 ? y[0] : cmul_conj(y[n2], tw[tw_index<R, true>(n2, lane + L * i)]);
-    }
+    for (int i = 0; i < Q; ++i) dft_reg<T, L, true>(*reinterpret_cast<cplx<T>(*)[L]>(&x[i * L]));
     T re[R];
 #pragma unroll
     for (int i = 0; i < Q; ++i)
@@ -158,7 +149,7 @@ __device__ __forceinline__ void gfft_inv_reg(cplx<T> (&x)[R], int lane, T* scr, 
 #pragma unroll
     for (int k1 = 0; k1 < R; ++k1) x[k1] = cplx<T>{re[k1], scr[lane * (R + 1) + k1]};
     wave_sync();
-    dft_reg<T, R, true>(x);
+    dft_twist<T, R, R * L, R, true>(x, tw, lane);
 }
 
 // M-point transforms: registers in gtime order to gfreq order and back.  HALF_ZERO: the inputs
@@ -176,7 +167,7 @@ __device__ __forceinline__ void gfft_fwd(cplx<T> (&x)[gregs(M)], int lane, T* sc
         gfft_fwd_reg<T, R, L, HALF_ZERO>(x0, lane, scr, tw);
         gfft_fwd_reg<T, R, L, HALF_ZERO>(x1, lane, scr, tw);
         gfft_fwd_reg<T, R, L, HALF_ZERO>(x2, lane, scr, tw);
-        const C* t3 = tw + L * (R + 1);
+        const C* t3 = tw + twist_elems(P, R);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int k = gfreq(P, r, lane);
@@ -197,7 +188,7 @@ __device__ __forceinline__ void gfft_inv(cplx<T> (&x)[gregs(M)], int lane, T* sc
     if constexpr (!gthree(M)) {
         gfft_inv_reg<T, R, L>(x, lane, scr, tw);
     } else {
-        const C* t3 = tw + L * (R + 1);
+        const C* t3 = tw + twist_elems(P, R);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int k = gfreq(P, r, lane);

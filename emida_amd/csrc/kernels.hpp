@@ -124,11 +124,13 @@ void mfma_refine_bounds(int mode, size2 s, bool t_double, double& tol_rel, doubl
 
 // ---- fft.hip, fft256.hip
 // W_M^t = exp(-2 pi i t / M) for every power of two 4 <= M <= kTwMaxM, the table of M at
-// offset M - 4 (M entries), then for M = 192 and 384 (tw_offset), rounded from
-// extended precision; a static device array per GPU, filled on first use (no allocation).
+// offset M - 4 (M entries), then for M = 192 and 384 (tw_offset), then (cos, tan) of
+// 2 pi t / M, t < M / 4, for the powers of two (tan_offset), rounded from extended
+// precision; a static device array per GPU, filled on first use (no allocation).
 constexpr int kTwMaxM = 512;
-constexpr int kTwElems = 2 * kTwMaxM - 4 + 192 + 384;
+constexpr int kTwElems = 2 * kTwMaxM - 4 + 192 + 384 + kTwMaxM / 2 - 1;
 __host__ __device__ constexpr int tw_offset(int m) { return m % 3 ? m - 4 : 2 * kTwMaxM - 4 + m - 192; }
+__host__ __device__ constexpr int tan_offset(int m) { return 2 * kTwMaxM - 4 + 192 + 384 + m / 4 - 1; }
 template <class T>
 const cplx<T>* fft_twiddles();
 // Largest padded FFT side of the single-kernel pipelines: 128 for double, 256 for
