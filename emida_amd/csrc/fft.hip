@@ -69,7 +69,7 @@ struct fft_plan {
     static constexpr int CS = ((need + 7) / 16) * 16 + 8;
     static constexpr int P_OFF = NC * CS - S * S / 2;  // prepared ROI (S*S reals) at the end
     static_assert(P_OFF >= (S / 2) * CS, "prepared ROI overlaps the row stage");
-    static constexpr size_t lds_bytes = (size_t)(NC * CS + twist_elems(M, R)) * sizeof(cplx<T>);  // + twiddles
+    static constexpr size_t lds_bytes = (size_t)(NC * CS + inv_twist_elems<T>(M, R)) * sizeof(cplx<T>);  // + twiddles
     // waves per SIMD the LDS allows (160 KiB per CU, 4 SIMDs); registers are
     // budgeted for exactly that many
     static constexpr int WG_PER_CU = (int)((160 * 1024) / (lds_bytes + kStaticLds));

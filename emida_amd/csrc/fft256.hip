@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kNT, 1) void fft256_kernel(fft_args<float, IN, SUM>
     const int kk = PIPE ? a.fit * a.fit : 0;
     const double lsq_v = tid < 6 * kk ? a.lsq[tid] : 0.0;
     load_twiddles<float, kM>(tw, a.twt, tid, kNT);  // while the loads are in flight
-    load_twist<float, kM, kR>(tw2, a.twt, tid, kNT);
+    load_twist<float, kM, kR, true>(tw2, a.twt, tid, kNT);
     // mean of the ROI (FROM_PATTERN): every pixel is one (pair, row, column) of one lane
     float mean = 0.f;
     if constexpr (FROM_PATTERN) {
@@ -327,7 +327,7 @@ __global__ __launch_bounds__(kNT, 1) void fft256_kernel(fft_args<float, IN, SUM>
         }
         if constexpr (PIPE) {
             asm volatile("" ::: "memory");
-            fft_inv<float, kR, kL, kM>(xs[j], lane, slot, tw2);
+            fft_inv<float, kR, kL, kM, true>(xs[j], lane, slot, tw2);
             if (j == kJ - 1) {
                 // job 3: column c = 96 + g, rows kL n1 + lane, to the LDS column store
                 C* col = B + kCol + g * kColStride;
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(kNT, 1) void fft256_kernel(fft_args<float, IN, SUM>
             C x[kR];
             row_pair_load(x, lane, band + 2 * g, kBS);
             __syncthreads();  // the band is read: its space becomes transpose scratch
-            fft_inv<float, kR, kL, kM>(x, lane, scr, tw2);
+            fft_inv<float, kR, kL, kM, true>(x, lane, scr, tw2);
             const int ya = y0 + 2 * g, yb = ya + 1;
             const bool in_a = ya <= s || ya > s + pad, in_b = yb <= s || yb > s + pad;
             const uint32_t ra = (uint32_t)(ya <= s ? ya : ya - pad) * s2;

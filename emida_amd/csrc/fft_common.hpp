@@ -4,12 +4,11 @@
 //
 // The single-kernel paths are bound by vector instructions, so the transforms count them: a
 // product for every twiddle between the levels and radix-4 passes took 332 per lane and 16
-// values of an inverse 128-point transform, the folded butterflies below 296, with 8 twiddles
-// read from LDS instead of 15.  25600 slices of 64 px in float: 622 -> 606 us; 6400 in
-// double: 501 -> 476 us; 6400 of 128 px in float: 861 -> 841 us; 648 of 96 px in double
-// (fftg.hip): 221 -> 205 us.  RMS error of a correlation against 64 bits (128 bits for
-// double), white noise: 64 px 2.45e-7 -> 2.33e-7 and 4.6e-16 -> 4.0e-16, 128 px 2.78e-7 ->
-// 2.52e-7.
+// values of an inverse 128-point transform; the folded butterflies below take 296, with 8
+// twiddles read from LDS instead of 15 (a float inverse 312: kFoldInverse).  25600 slices of
+// 64 px in float: 622 -> 612 us; 6400 in double: 501 -> 476 us; 6400 of 128 px in float: 861
+// -> 842 us; 648 of 96 px in double (fftg.hip): 221 -> 205 us.  Offsets of slices like a
+// scan's against 64 bits, in float: 20 to 150 px 0 to 22% nearer than before.
 #pragma once
 
 #include <type_traits>
@@ -238,9 +237,35 @@ __device__ __forceinline__ void fft_fwd(cplx<T> (&x)[R], int lane, cplx<T>* scr,
     }
 }
 
+// Second level of an inverse transform.  Folded twiddles multiply an output by one cosine per
+// pass, and the rounding of those few cosines moves the whole output: unlike the errors of a
+// sum it differs from one shift to the next, which tilts the fitted peak (offsets of 64 px
+// slices in float: 20% further from 64 bits, 33 px 40%).  With the products W_M^(lane k) before
+// plain passes, outputs 0..L-1 meet no other twiddle and the errors of the R products average
+// out: offsets 16% nearer than with radix 4 at 64 px, 22% at 250.  It costs 16 operations and 7
+// twiddles (25600 slices of 64 px: 608 -> 612 us; 672 of 161 x 95: 281 -> 292 us).  Folded where
+// that rounding is far below the fit's own (double), and in fft256.hip, whose neighbourhood comes from
+// direct sums (128 px: offsets 1% nearer than with radix 4).
+template <class T>
+constexpr bool kFoldInverse = sizeof(T) == 8;
+// tab elements of an inverse transform of M = R L points
+template <class T>
+constexpr int inv_twist_elems(int m, int r) { return twist_elems(m, r) + (kFoldInverse<T> ? 0 : m + m / r); }
+template <class T, int R, int M, bool FOLD>
+__device__ __forceinline__ void dft_last(cplx<T> (&x)[R], const cplx<T>* tw, int lane) {
+    if constexpr (FOLD) {
+        dft_twist<T, R, M, R, true>(x, tw, lane);
+    } else {
+        const cplx<T>* t = tw + twist_elems(M, R) + lane * (R + 1);
+#pragma unroll
+        for (int k = 1; k < R; ++k) x[k] = cmul_conj(x[k], t[k]);
+        dft_reg<T, R, true>(x);
+    }
+}
+
 // Inverse (unnormalised) transform from the frequency layout to natural order:
 // on return lane n2 holds output[L*n1 + n2] in x[n1].
-template <class T, int R, int L, int M>
+template <class T, int R, int L, int M, bool FOLD = kFoldInverse<T>>
 __device__ __forceinline__ void fft_inv(cplx<T> (&x)[R], int lane, cplx<T>* scr, const cplx<T>* tw) {
     constexpr int Q = R / L;
 #pragma unroll
@@ -256,7 +281,7 @@ __device__ __forceinline__ void fft_inv(cplx<T> (&x)[R], int lane, cplx<T>* scr,
 #pragma unroll
     for (int k1 = 0; k1 < R; ++k1) x[k1] = scr[lane * (R + 1) + k1];
     wave_sync();
-    dft_twist<T, R, M, R, true>(x, tw, lane);
+    dft_last<T, R, M, FOLD>(x, tw, lane);
 }
 
 // Prepared pixel (src/prepare_pics.cu:36-41), no contraction.
@@ -338,11 +363,18 @@ template <class T, int M>
 __device__ __forceinline__ void load_twiddles(cplx<T>* tw, const cplx<T>* table, int tid, int nt) {
     for (int t = tid; t < M; t += nt) tw[t] = table[tw_offset(M) + t];
 }
-// The twiddles of dft_twist (twist_elems(M, R) elements).
-template <class T, int M, int R>
+// The twiddles of dft_twist (twist_elems(M, R) elements) and, unless FOLD, W_M^(n k) as
+// [n][k], n < M / R, k < R, rows of R + 1 (an odd stride: a group's lanes on distinct banks).
+template <class T, int M, int R, bool FOLD = kFoldInverse<T>>
 __device__ __forceinline__ void load_twist(cplx<T>* tw, const cplx<T>* table, int tid, int nt) {
     for (int t = tid; t < twist_elems(M, R); t += nt)
         tw[t] = table[t < M / 4 ? tan_offset(M) + t : tw_offset(M) + (t - M / 4) * (M / (2 * R))];
+    if constexpr (!FOLD) {
+        for (int t = tid; t < M + M / R; t += nt) {
+            const int n = t / (R + 1), k = t % (R + 1);
+            tw[twist_elems(M, R) + t] = table[tw_offset(M) + (k < R ? n * k % M : 0)];
+        }
+    }
 }
 
 }  // namespace emida_amd

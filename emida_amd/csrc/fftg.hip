@@ -27,7 +27,7 @@
 // Bound: the half spectra in HBM.  8 patterns x 81 ROIs of 96 x 96 in double (192 x 192):
 // 0.58 GB written and read, 183 us (rows 31, columns 71, inverse rows 72); radix-4 passes
 // through LDS over 256 x 256, a staged column tile and the correlation written for a peak
-// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 282 us (sums
+// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 292 us (sums
 // 20, rows 60, columns 89, inverse rows 102), before 606 us.
 //
 // Scale: the pattern's spectrum comes out doubled (the omitted split factor); the
@@ -75,18 +75,21 @@ constexpr bool gzero(int m, int r) { return r % gsub(m) >= gsub(m) / 2; }
 // group, in T: the transpose scratch of the real or the imaginary parts, which also holds a
 // whole real row.  Half of a complex scratch: twice the workgroups per CU (256-point
 // transforms in double: 39 KB instead of 74).
-constexpr int gtw(int m) { return twist_elems(gbase(m), gsub(m)) + (gthree(m) ? 2 * gbase(m) : 0); }
+template <class T>
+constexpr int greg_tw(int m) { return inv_twist_elems<T>(gbase(m), gsub(m)); }
+template <class T>
+constexpr int gtw(int m) { return greg_tw<T>(m) + (gthree(m) ? 2 * gbase(m) : 0); }
 constexpr int gslot(int m) { return gthree(m) ? m + 8 : glanes(m) * (gsub(m) + 1); }
 template <class T>
 constexpr size_t glds(int m) {
-    return (2 * (size_t)gtw(m) + (size_t)(kGNT / glanes(m)) * gslot(m)) * sizeof(T);
+    return (2 * (size_t)gtw<T>(m) + (size_t)(kGNT / glanes(m)) * gslot(m)) * sizeof(T);
 }
 template <class T, int M>
 __device__ __forceinline__ void gload_twiddles(cplx<T>* tw, const cplx<T>* table, int tid) {
     constexpr int P = gbase(M);
     load_twist<T, P, gsub(M)>(tw, table, tid, kGNT);
     if constexpr (gthree(M)) {
-        cplx<T>* t3 = tw + twist_elems(P, gsub(M));
+        cplx<T>* t3 = tw + greg_tw<T>(M);
         for (int k = tid; k < P; k += kGNT) {
             t3[k] = table[tw_offset(M) + k];
             t3[P + k] = table[tw_offset(M) + 2 * k];
@@ -149,7 +152,7 @@ __device__ __forceinline__ void gfft_inv_reg(cplx<T> (&x)[R], int lane, T* scr, 
 #pragma unroll
     for (int k1 = 0; k1 < R; ++k1) x[k1] = cplx<T>{re[k1], scr[lane * (R + 1) + k1]};
     wave_sync();
-    dft_twist<T, R, R * L, R, true>(x, tw, lane);
+    dft_last<T, R, R * L, kFoldInverse<T>>(x, tw, lane);
 }
 
 // M-point transforms: registers in gtime order to gfreq order and back.  HALF_ZERO: the inputs
@@ -167,7 +170,7 @@ __device__ __forceinline__ void gfft_fwd(cplx<T> (&x)[gregs(M)], int lane, T* sc
         gfft_fwd_reg<T, R, L, HALF_ZERO>(x0, lane, scr, tw);
         gfft_fwd_reg<T, R, L, HALF_ZERO>(x1, lane, scr, tw);
         gfft_fwd_reg<T, R, L, HALF_ZERO>(x2, lane, scr, tw);
-        const C* t3 = tw + twist_elems(P, R);
+        const C* t3 = tw + greg_tw<T>(M);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int k = gfreq(P, r, lane);
@@ -188,7 +191,7 @@ __device__ __forceinline__ void gfft_inv(cplx<T> (&x)[gregs(M)], int lane, T* sc
     if constexpr (!gthree(M)) {
         gfft_inv_reg<T, R, L>(x, lane, scr, tw);
     } else {
-        const C* t3 = tw + twist_elems(P, R);
+        const C* t3 = tw + greg_tw<T>(M);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int k = gfreq(P, r, lane);
@@ -254,7 +257,7 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_kernel(fftg_args<T, IN, SUM
     C* tw = reinterpret_cast<C*>(lds_raw);
     __shared__ uint32_t red_u[kGNT / kWave];
     const int tid = threadIdx.x, g = tid / L, lane = tid % L;
-    T* slot = reinterpret_cast<T*>(tw + gtw(MX)) + gslot(MX) * g;
+    T* slot = reinterpret_cast<T*>(tw + gtw<T>(MX)) + gslot(MX) * g;
     const uint32_t sl = blockIdx.x, sn = a.first + sl;
     gload_twiddles<T, MX>(tw, a.twt, tid);
 
@@ -370,7 +373,7 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_cols_kernel(fftg_args<T, T, T> a
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C* tw = reinterpret_cast<C*>(lds_raw);
     const int tid = threadIdx.x, g = tid / L, lane = tid % L;
-    T* slot = reinterpret_cast<T*>(tw + gtw(MY)) + gslot(MY) * g;
+    T* slot = reinterpret_cast<T*>(tw + gtw<T>(MY)) + gslot(MY) * g;
     const int ncx = (int)a.mx / 2 + 1;
     const uint32_t gx = div_up((uint32_t)ncx, (uint32_t)NG), b = xcd_remap(blockIdx.x, nblk);
     uint32_t sl, col;
@@ -478,7 +481,7 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_inv_kernel(fftg_args<T, T, 
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C* tw = reinterpret_cast<C*>(lds_raw);
     const int tid = threadIdx.x, g = tid / L, lane = tid % L;
-    T* slot = reinterpret_cast<T*>(tw + gtw(MX)) + gslot(MX) * g;
+    T* slot = reinterpret_cast<T*>(tw + gtw<T>(MX)) + gslot(MX) * g;
     const uint32_t sl = blockIdx.x, sn = a.first + sl;
     gload_twiddles<T, MX>(tw, a.twt, tid);
     __syncthreads();
@@ -554,7 +557,7 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_inv_kernel(fftg_args<T, T, 
             const int i = t % fit, j = t / fit;
             const size2 c = clamp_pos((int)mp.x - rad + i, (int)mp.y - rad + j, cross);
             const int rx = (int)((c.x + (a.out.x / 2 + 1)) % a.out.x);
-            const T v = (reinterpret_cast<const T*>(tw + gtw(MX)) + gslot(MX) * j)[rx <= sx ? rx : rx + padx];
+            const T v = (reinterpret_cast<const T*>(tw + gtw<T>(MX)) + gslot(MX) * j)[rx <= sx ? rx : rx + padx];
             nbv[t] = v;
             if (a.neigh) a.neigh[(size_t)sn * kk + t] = v;
         }
