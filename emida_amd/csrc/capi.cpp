@@ -123,19 +123,7 @@ int emida_offset_finalize(emida_offset* h, const void* maxes_i, const void* neig
 int emida_offset_get_offset(emida_offset* h, const void* pic, double* offsets, double* coefs) {
     return guarded([&] {
         if (!h || !pic || !offsets) throw arg_error("null argument");
-        h->require_allocated();
-        auto& o = h->out[h->out_i];
-        h->out_i ^= 1;
-        EMIDA_HIP(hipStreamSynchronize(h->out_stream));
-        EMIDA_HIP(hipStreamWaitEvent(h->compute, h->ev_done[0], 0));
-        EMIDA_HIP(hipMemcpyAsync(h->d_in[0], pic, (size_t)h->src.area() * h->batch * h->in_bytes(),
-                                 hipMemcpyHostToDevice, h->compute));
-        h->run(h->d_in[0], h->batch, o.maxes, o.neigh, o.offsets, o.coefs, h->compute);
-        EMIDA_HIP(hipMemcpyAsync(offsets, o.offsets, h->total * 2 * sizeof(double), hipMemcpyDeviceToHost, h->compute));
-        if (coefs)
-            EMIDA_HIP(hipMemcpyAsync(coefs, o.coefs, h->total * 6 * sizeof(double), hipMemcpyDeviceToHost, h->compute));
-        EMIDA_HIP(hipEventRecord(h->ev_done[0], h->compute));
-        EMIDA_HIP(hipStreamSynchronize(h->compute));
+        h->host_call(pic, offsets, coefs);
     });
 }
 

@@ -319,6 +319,40 @@ void launch_prepare(const IN* pics, T* slices, const T* hx, const T* hy, const S
     EMIDA_LAUNCHED("prepare_kernel");
 }
 
+// Bound by the link's latency: every thread has one 16-byte load in flight and the grid
+// covers the copy, so the link is full from the first microsecond on (a grid of 128
+// workgroups holds 512 KB).
+__global__ __launch_bounds__(256) void copy_kernel(uint4* __restrict__ dst, const uint4* __restrict__ src, size_t bytes) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < bytes / 16) dst[i] = src[i];
+    // the last bytes % 16
+    if (i < bytes % 16) ((uint8_t*)dst)[bytes / 16 * 16 + i] = ((const uint8_t*)src)[bytes / 16 * 16 + i];
+}
+
+void launch_copy(void* dst, const void* src, size_t bytes, hipStream_t st) {
+    if (bytes == 0) return;
+    const size_t n = std::max<size_t>(bytes / 16, bytes % 16);
+    copy_kernel<<<(uint32_t)((n + 255) / 256), 256, 0, st>>>((uint4*)dst, (const uint4*)src, bytes);
+    EMIDA_HIP(hipGetLastError());
+}
+
+__global__ __launch_bounds__(256) void copy_results_kernel(double2* __restrict__ dst0, const double2* __restrict__ src0,
+                                                           uint32_t n0, double2* __restrict__ dst1,
+                                                           const double2* __restrict__ src1, uint32_t n1) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n0) dst0[i] = src0[i];
+    else if (i - n0 < n1) dst1[i - n0] = src1[i - n0];
+}
+
+void launch_copy_results(double* dst0, const double* src0, size_t n0, double* dst1, const double* src1, size_t n1,
+                         hipStream_t st) {
+    const uint32_t a = (uint32_t)(n0 / 2), b = (uint32_t)(n1 / 2);  // pairs: 2 and 6 values per slice
+    if (a + b == 0) return;
+    copy_results_kernel<<<div_up(a + b, 256u), 256, 0, st>>>((double2*)dst0, (const double2*)src0, a, (double2*)dst1,
+                                                             (const double2*)src1, b);
+    EMIDA_HIP(hipGetLastError());
+}
+
 #define INST_SUM_PREP(T, HT)                                                                              \
     template bool launch_sum_prepare<T, HT>(const uint16_t*, uint32_t*, T*, const T*, const T*, HT*, HT*,   \
                                             const float*, const float*, float, double*, const T*,              \

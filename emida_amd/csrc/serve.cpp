@@ -23,6 +23,7 @@
 #include <thread>
 #include <unordered_map>
 
+#include "host_copy.hpp"
 #include "offset.hpp"
 
 namespace {
@@ -108,6 +109,7 @@ struct emida_server_s {
     bool stop = false;
     std::string worker_error;
 
+    std::shared_ptr<copy_team> team = copy_team::get();  // submissions copy their patterns with it
     std::mutex mu;
     std::condition_variable cv_sched, cv_done, cv_staging;
     std::thread scheduler;
@@ -257,7 +259,7 @@ struct emida_server_s {
                 std::lock_guard<std::mutex> l2(mu);
                 staging_all.push_back(buf);
             }
-            std::memcpy(buf, pattern, bytes);
+            team->copy(buf, pattern, bytes);
         } catch (...) {
             std::lock_guard<std::mutex> l2(mu);
             --staging_used;
