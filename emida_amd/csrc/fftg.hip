@@ -25,10 +25,10 @@
 // transpose through LDS (fft_common.hpp).
 //
 // Bound: the half spectra in HBM.  8 patterns x 81 ROIs of 96 x 96 in double (192 x 192):
-// 0.58 GB written and read, 183 us (rows 31, columns 71, inverse rows 72); radix-4 passes
+// 0.58 GB written and read, 197 us (rows 31, columns 75, inverse rows 56, peaks 11); radix-4 passes
 // through LDS over 256 x 256, a staged column tile and the correlation written for a peak
-// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 292 us (sums
-// 20, rows 60, columns 89, inverse rows 102), before 606 us.
+// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 277 us (sums
+// 20, rows 57, columns 90, inverse rows 81, peaks 12), before 606 us.
 //
 // Scale: the pattern's spectrum comes out doubled (the omitted split factor); the
 // stored reference spectrum is 2 s.x s.y / (Mx My) times the true one (the same
@@ -84,13 +84,13 @@ template <class T>
 constexpr size_t glds(int m) {
     return (2 * (size_t)gtw<T>(m) + (size_t)(kGNT / glanes(m)) * gslot(m)) * sizeof(T);
 }
-template <class T, int M>
+template <class T, int M, int NT = kGNT>
 __device__ __forceinline__ void gload_twiddles(cplx<T>* tw, const cplx<T>* table, int tid) {
     constexpr int P = gbase(M);
-    load_twist<T, P, gsub(M)>(tw, table, tid, kGNT);
+    load_twist<T, P, gsub(M)>(tw, table, tid, NT);
     if constexpr (gthree(M)) {
         cplx<T>* t3 = tw + greg_tw<T>(M);
-        for (int k = tid; k < P; k += kGNT) {
+        for (int k = tid; k < P; k += NT) {
             t3[k] = table[tw_offset(M) + k];
             t3[P + k] = table[tw_offset(M) + 2 * k];
         }
@@ -442,11 +442,11 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_cols_kernel(fftg_args<T, T, T> a
 }
 
 // ---------------------------------------------------------------- kernel 3: rows, inverse
-// Output rows 2q and 2q + 1 of the reference layout of one slice, by one lane group: on
-// return a lane holds their columns gtime (circular) in x[r].re and x[r].im.
+// Output rows 2q and 2q + 1 of the reference layout of one slice, for one lane group: on
+// return a lane holds their packed half spectra at frequencies gfreq.
 template <class T, int MX>
-__device__ __forceinline__ void inverse_row_pair(cplx<T> (&x)[gregs(MX)], const cplx<T>* w, int q, int sy, int pady,
-                                                 int lane, T* slot, const cplx<T>* tw) {
+__device__ __forceinline__ void load_row_pair(cplx<T> (&x)[gregs(MX)], const cplx<T>* w, int q, int sy, int pady,
+                                              int lane) {
     using C = cplx<T>;
     constexpr int R = gregs(MX), NCX = MX / 2 + 1, S = MX / 2;
     // reference-layout row r <= s is circular row r, r > s is r + M - 2s
@@ -469,11 +469,17 @@ __device__ __forceinline__ void inverse_row_pair(cplx<T> (&x)[gregs(MX)], const 
         }
         x[r] = C{ga.re - gb.im, ga.im + gb.re};
     }
-    gfft_inv<T, MX>(x, lane, slot, tw);
 }
 
-// PEAK: one workgroup per slice, arg-max (lowest index on ties), neighbourhood, fit and
-// finalize as peak_kernel; else the rows of the correlation buffer.
+// One row pair per lane group.  PEAK: the pair's largest value and its lowest index go to the
+// imaginary parts of columns 0 and Mx / 2 of the pair's first row, which a C2R drops; else the
+// rows of the correlation buffer.
+//
+// Grid: (slices, blocks of NG row pairs).  With a slice's row pairs in rounds of one workgroup,
+// its arg-max and its fit behind them, 648 slices were 1.3 rounds of the chip, most lanes idle
+// during every fit, and the loop's registers spilled at 384.  Inverse rows / with peaks, before
+// and now, us: 648 slices of 96 x 96 in double 73 / 56 + 11; 672 of 161 x 95 in float 108 /
+// 81 + 12; a pass over 36 of 250 x 250 in float 151 / 78; over 16 of 128 x 128 in double 49 / 30.
 template <class T, int MX, bool PEAK>
 __global__ __launch_bounds__(kGNT, 2) void fftg_rows_inv_kernel(fftg_args<T, T, T> a) {
     using C = cplx<T>;
@@ -482,103 +488,143 @@ __global__ __launch_bounds__(kGNT, 2) void fftg_rows_inv_kernel(fftg_args<T, T, 
     C* tw = reinterpret_cast<C*>(lds_raw);
     const int tid = threadIdx.x, g = tid / L, lane = tid % L;
     T* slot = reinterpret_cast<T*>(tw + gtw<T>(MX)) + gslot(MX) * g;
-    const uint32_t sl = blockIdx.x, sn = a.first + sl;
-    gload_twiddles<T, MX>(tw, a.twt, tid);
-    __syncthreads();
-    const C* w = a.work + (size_t)sl * a.my * NCX;
+    const uint32_t sl = blockIdx.x;
+    C* w = a.work + (size_t)sl * a.my * NCX;
     // reference-layout index k <= s is circular position k, k > s is k + M - 2s
     const int sx = (int)a.out.x / 2, sy = (int)a.out.y / 2;
     const int padx = MX - (int)a.out.x, pady = (int)a.my - (int)a.out.y;
-    const int npairs = (int)a.out.y / 2;
-    T best = -(T)__builtin_huge_val();
-    uint32_t bi = 0xffffffffu;
-    for (int q = g; q < npairs; q += NG) {
-        C x[R];
-        inverse_row_pair<T, MX>(x, w, q, sy, pady, lane, slot, tw);
-        const uint32_t ia = 2 * (uint32_t)q * a.out.x, ib = ia + a.out.x;
-        if constexpr (PEAK) {
-            // the row's largest value and its first column, row a before row b; later rows have
-            // larger indices, so strictly larger keeps the lowest
-            T va = best, vb;
-            int ca = MX, cb = MX;
+    const int npairs = (int)a.out.y / 2, q = (int)blockIdx.y * NG + g;
+    C x[R];
+    load_row_pair<T, MX>(x, w, min(q, npairs - 1), sy, pady, lane);
+    gload_twiddles<T, MX, kGNT>(tw, a.twt, tid);
+    __syncthreads();
+    if (q >= npairs) return;
+    gfft_inv<T, MX>(x, lane, slot, tw);
+    const uint32_t ia = 2 * (uint32_t)q * a.out.x, ib = ia + a.out.x;
+    if constexpr (PEAK) {
+        // the lane's largest value and its first column, row a before row b (larger indices, so
+        // strictly larger keeps the lowest)
+        T va = -(T)__builtin_huge_val(), vb;
+        int ca = MX, cb = MX;
 #pragma unroll
-            for (int n1 = 0; n1 < R; ++n1) {
-                const int c = gtime(MX, n1, lane);
-                const T v = x[n1].re;
-                if ((c <= sx || c > sx + padx) && (v > va || (gthree(MX) && v == va && c < ca && ca < MX))) va = v, ca = c;
-            }
-            vb = va;
+        for (int n1 = 0; n1 < R; ++n1) {
+            const int c = gtime(MX, n1, lane);
+            const T v = x[n1].re;
+            if ((c <= sx || c > sx + padx) && (v > va || (gthree(MX) && v == va && c < ca && ca < MX))) va = v, ca = c;
+        }
+        vb = va;
 #pragma unroll
-            for (int n1 = 0; n1 < R; ++n1) {
-                const int c = gtime(MX, n1, lane);
-                const T v = x[n1].im;
-                if ((c <= sx || c > sx + padx) && (v > vb || (gthree(MX) && v == vb && c < cb && cb < MX))) vb = v, cb = c;
-            }
-            if (ca < MX) bi = ia + (uint32_t)(ca <= sx ? ca : ca - padx);
-            if (cb < MX) bi = ib + (uint32_t)(cb <= sx ? cb : cb - padx);
-            best = vb;
-        } else {
-            T* out = a.corr + (size_t)sl * a.out.area();
+        for (int n1 = 0; n1 < R; ++n1) {
+            const int c = gtime(MX, n1, lane);
+            const T v = x[n1].im;
+            if ((c <= sx || c > sx + padx) && (v > vb || (gthree(MX) && v == vb && c < cb && cb < MX))) vb = v, cb = c;
+        }
+        uint32_t bi = 0xffffffffu;
+        if (ca < MX) bi = ia + (uint32_t)(ca <= sx ? ca : ca - padx);
+        if (cb < MX) bi = ib + (uint32_t)(cb <= sx ? cb : cb - padx);
 #pragma unroll
-            for (int n1 = 0; n1 < R; ++n1) {
-                const int c = gtime(MX, n1, lane);
-                if (c <= sx || c > sx + padx) {
-                    const int rx = c <= sx ? c : c - padx;
-                    out[ia + rx] = x[n1].re;
-                    out[ib + rx] = x[n1].im;
-                }
+        for (int off = L / 2; off > 0; off >>= 1) {
+            const T v = __shfl_xor(vb, off);
+            const uint32_t i = __shfl_xor(bi, off);
+            if (v > vb || (v == vb && i < bi)) vb = v, bi = i;
+        }
+        if (lane == 0) {
+            C* row = w + (size_t)(2 * q <= sy ? 2 * q : 2 * q + pady) * NCX;
+            row[0].im = vb;
+            *reinterpret_cast<uint32_t*>(&row[NCX - 1].im) = bi;
+        }
+    } else {
+        T* out = a.corr + (size_t)sl * a.out.area();
+#pragma unroll
+        for (int n1 = 0; n1 < R; ++n1) {
+            const int c = gtime(MX, n1, lane);
+            if (c <= sx || c > sx + padx) {
+                const int rx = c <= sx ? c : c - padx;
+                out[ia + rx] = x[n1].re;
+                out[ib + rx] = x[n1].im;
             }
         }
     }
-    if constexpr (PEAK) {
-        __shared__ T sv[kGNT / kWave];
-        __shared__ uint32_t si[kGNT / kWave];
-        __shared__ T nbv[81];
-        __shared__ double cf[6];
-        block_argmax<T, kGNT>(best, bi, sv, si);
-        const size2 cross{a.out.x - 1, a.out.y - 1};
-        const size2 mp = shift_pos(POLICY_FFT, bi, cross);
-        const int fit = a.fit, rad = (fit - 1) / 2, kk = fit * fit;
-        // neighbourhood row j: its row pair again, the row kept in slot j
-        static_assert(NG >= 9, "one lane group per neighbourhood row");
-        if (g < fit) {
-            const size2 c = clamp_pos((int)mp.x, (int)mp.y - rad + g, cross);
-            const int ry = (int)((c.y + (a.out.y / 2 + 1)) % a.out.y);
-            C x[R];
-            inverse_row_pair<T, MX>(x, w, ry >> 1, sy, pady, lane, slot, tw);
+}
+
+// ---------------------------------------------------------------- kernel 4: peaks
+// One small workgroup per slice: arg-max over the row pairs (lowest index on ties), the row
+// pairs of the neighbourhood again, one per lane group, fit and finalize as peak_kernel.
+constexpr int gpeak_nt(int m) { return glanes(m) * 16 < kWave ? kWave : glanes(m) * 16; }
+template <class T>
+constexpr size_t gpeak_lds(int m) {
+    return (2 * (size_t)gtw<T>(m) + (size_t)(gpeak_nt(m) / glanes(m)) * gslot(m)) * sizeof(T);
+}
+template <class T, int MX>
+__global__ __launch_bounds__(gpeak_nt(MX)) void fftg_peak_kernel(fftg_args<T, T, T> a) {
+    using C = cplx<T>;
+    constexpr int NT = gpeak_nt(MX), L = glanes(MX), R = gregs(MX), NCX = MX / 2 + 1;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    C* tw = reinterpret_cast<C*>(lds_raw);
+    const int tid = threadIdx.x, g = tid / L, lane = tid % L;
+    T* slot = reinterpret_cast<T*>(tw + gtw<T>(MX)) + gslot(MX) * g;
+    const uint32_t sl = blockIdx.x, sn = a.first + sl;
+    gload_twiddles<T, MX, NT>(tw, a.twt, tid);
+    const C* w = a.work + (size_t)sl * a.my * NCX;
+    const int sx = (int)a.out.x / 2, sy = (int)a.out.y / 2;
+    const int padx = MX - (int)a.out.x, pady = (int)a.my - (int)a.out.y;
+    T best = -(T)__builtin_huge_val();
+    uint32_t bi = 0xffffffffu;
+    for (int q = tid; q < (int)a.out.y / 2; q += NT) {
+        const C* row = w + (size_t)(2 * q <= sy ? 2 * q : 2 * q + pady) * NCX;
+        const T v = row[0].im;
+        const uint32_t i = *reinterpret_cast<const uint32_t*>(&row[NCX - 1].im);
+        if (v > best || (v == best && i < bi)) best = v, bi = i;
+    }
+    __shared__ T sv[NT / kWave];
+    __shared__ uint32_t si[NT / kWave];
+    __shared__ T nbv[81];
+    __shared__ double cf[6];
+    block_argmax<T, NT>(best, bi, sv, si);
+    const size2 cross{a.out.x - 1, a.out.y - 1};
+    const size2 mp = shift_pos(POLICY_FFT, bi, cross);
+    const int fit = a.fit, rad = (fit - 1) / 2, kk = fit * fit;
+    // neighbourhood row j: its row pair again, the row kept in slot j
+    static_assert(NT / L >= 9, "one lane group per neighbourhood row");
+    __syncthreads();  // twiddles
+    if (g < fit) {
+        const size2 c = clamp_pos((int)mp.x, (int)mp.y - rad + g, cross);
+        const int ry = (int)((c.y + (a.out.y / 2 + 1)) % a.out.y);
+        C x[R];
+        load_row_pair<T, MX>(x, w, ry >> 1, sy, pady, lane);
+        gfft_inv<T, MX>(x, lane, slot, tw);
 #pragma unroll
-            for (int n1 = 0; n1 < R; ++n1) {
-                const T even = x[n1].re, odd = x[n1].im;
-                slot[gtime(MX, n1, lane)] = ry & 1 ? odd : even;
-            }
+        for (int n1 = 0; n1 < R; ++n1) {
+            const T even = x[n1].re, odd = x[n1].im;
+            slot[gtime(MX, n1, lane)] = ry & 1 ? odd : even;
         }
-        __syncthreads();
-        for (int t = tid; t < kk; t += kGNT) {
-            const int i = t % fit, j = t / fit;
-            const size2 c = clamp_pos((int)mp.x - rad + i, (int)mp.y - rad + j, cross);
-            const int rx = (int)((c.x + (a.out.x / 2 + 1)) % a.out.x);
-            const T v = (reinterpret_cast<const T*>(tw + gtw<T>(MX)) + gslot(MX) * j)[rx <= sx ? rx : rx + padx];
-            nbv[t] = v;
-            if (a.neigh) a.neigh[(size_t)sn * kk + t] = v;
+    }
+    __syncthreads();
+    for (int t = tid; t < kk; t += NT) {
+        const int i = t % fit, j = t / fit;
+        const size2 c = clamp_pos((int)mp.x - rad + i, (int)mp.y - rad + j, cross);
+        const int rx = (int)((c.x + (a.out.x / 2 + 1)) % a.out.x);
+        const T v = (reinterpret_cast<const T*>(tw + gtw<T>(MX)) + gslot(MX) * j)[rx <= sx ? rx : rx + padx];
+        nbv[t] = v;
+        if (a.neigh) a.neigh[(size_t)sn * kk + t] = v;
+    }
+    __syncthreads();
+    if (tid < 6) cf[tid] = fit_coef<T>(a.lsq + tid * kk, nbv, kk);
+    __syncthreads();
+    if (tid == 0) {
+        if (a.maxes) {
+            a.maxes[sn].data = best;
+            a.maxes[sn].index = bi;
         }
-        __syncthreads();
-        if (tid < 6) cf[tid] = fit_coef<T>(a.lsq + tid * kk, nbv, kk);
-        __syncthreads();
-        if (tid == 0) {
-            if (a.maxes) {
-                a.maxes[sn].data = best;
-                a.maxes[sn].index = bi;
-            }
-            double px, py, ox, oy;
-            fit_peak(cf, px, py);
-            finalize_offset(bi, cross, POLICY_FFT, fit, px, py, ox, oy);
-            if (a.offsets) {
-                a.offsets[2 * (size_t)sn] = ox;
-                a.offsets[2 * (size_t)sn + 1] = oy;
-            }
-            if (a.coefs)
-                for (int c = 0; c < 6; ++c) a.coefs[6 * (size_t)sn + c] = cf[c];
+        double px, py, ox, oy;
+        fit_peak(cf, px, py);
+        finalize_offset(bi, cross, POLICY_FFT, fit, px, py, ox, oy);
+        if (a.offsets) {
+            a.offsets[2 * (size_t)sn] = ox;
+            a.offsets[2 * (size_t)sn + 1] = oy;
         }
+        if (a.coefs)
+            for (int c = 0; c < 6; ++c) a.coefs[6 * (size_t)sn + c] = cf[c];
     }
 }
 
@@ -638,8 +684,15 @@ void run_rows_inv(const fftg_args<T, T, T>& a, hipStream_t st) {
         auto k = fftg_rows_inv_kernel<T, MX, PEAK>;
         static const bool once = (set_lds(k, glds<T>(MX)), true);
         (void)once;
-        k<<<a.total, kGNT, glds<T>(MX), st>>>(a);
+        k<<<dim3(a.total, div_up(a.out.y / 2, (uint32_t)(kGNT / glanes(MX)))), kGNT, glds<T>(MX), st>>>(a);
         EMIDA_LAUNCHED("fftg_rows_inv_kernel");
+        if constexpr (PEAK) {
+            auto kp = fftg_peak_kernel<T, MX>;
+            static const bool oncep = (set_lds(kp, gpeak_lds<T>(MX)), true);
+            (void)oncep;
+            kp<<<a.total, gpeak_nt(MX), gpeak_lds<T>(MX), st>>>(a);
+            EMIDA_LAUNCHED("fftg_peak_kernel");
+        }
     });
 }
 
