@@ -6,7 +6,7 @@
 // correlation values (zero padding beyond 2s changes no shift |d| < s), read through
 // the reference's 2s.x x 2s.y layout as in fft.hip.
 //
-// Three kernels per launch chunk, with a work buffer of half spectra in HBM
+// Four kernels per launch chunk, with a work buffer of half spectra in HBM
 // ([slice][y][kx], kx <= Mx/2, the layout of an R2C result):
 //  1. rows: two real rows packed as one complex row (prepared from the pattern or
 //     read from prepared slices), an Mx-point transform, split into the two half
@@ -17,18 +17,18 @@
 //     column-major, read by lanes in order);
 //  3. rows, inverse: two output rows packed as Ga + i Gb (Hermitian extension, DC and
 //     Nyquist imaginary parts dropped, as a C2R does), one inverse transform yields both
-//     real rows of the reference's (2s.x x 2s.y) circular correlation; one workgroup per
-//     slice keeps the largest value, runs the row pairs of the neighbourhood again
-//     (cross_res_pos_policy_fft, src/kernels.cuh:36-53), fits and finalizes, so the
-//     correlation itself is not written (the seams write it instead).
+//     real rows of the reference's (2s.x x 2s.y) circular correlation and their largest
+//     value; the correlation itself is not written (the seams write it instead);
+//  4. peaks: the arg-max over a slice's row pairs, the row pairs of the neighbourhood
+//     again (cross_res_pos_policy_fft, src/kernels.cuh:36-53), fit and finalize.
 // A transform runs on L lanes of one wave with R = M / L values each in registers and one
 // transpose through LDS (fft_common.hpp).
 //
 // Bound: the half spectra in HBM.  8 patterns x 81 ROIs of 96 x 96 in double (192 x 192):
 // 0.58 GB written and read, 197 us (rows 31, columns 75, inverse rows 56, peaks 11); radix-4 passes
 // through LDS over 256 x 256, a staged column tile and the correlation written for a peak
-// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 277 us (sums
-// 20, rows 57, columns 90, inverse rows 81, peaks 12), before 606 us.
+// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 261 us (sums
+// 20, rows 43, columns 87, inverse rows 81, peaks 12), before 606 us.
 //
 // Scale: the pattern's spectrum comes out doubled (the omitted split factor); the
 // stored reference spectrum is 2 s.x s.y / (Mx My) times the true one (the same
@@ -245,12 +245,22 @@ struct fftg_args {
     double* coefs;
 };
 
+// Waves per SIMD the registers are budgeted for.  Forward rows of 384 in float and columns of
+// 128 in double need 186 and 172 registers by themselves and none of them in scratch at 168,
+// which lets a third workgroup share a CU (the LDS holds three): 672 slices of 161 x 95 in float
+// 277 -> 261 us, 2304 of 60 x 50 in double 212 -> 200.  The other kernels above 168 would spill
+// 60 bytes to 800 a lane.
+template <class T>
+constexpr int gwaves(int m, int three, int size) {
+    return m == three && sizeof(T) == size ? 3 : 2;
+}
+
 // ---------------------------------------------------------------- kernel 1: rows
 // HZ: the second half of every row is zero padding (slices of at most Mx / 2 columns).
 // Grid: (slices, splits); a slice's splits take its row pairs in turn (uint16: each sums
 // the whole slice for the mean).
 template <class T, class IN, class SUM, int MX, bool FROM_PATTERN, bool HZ>
-__global__ __launch_bounds__(kGNT, 2) void fftg_rows_kernel(fftg_args<T, IN, SUM> a) {
+__global__ __launch_bounds__(kGNT, gwaves<T>(MX, 384, 4)) void fftg_rows_kernel(fftg_args<T, IN, SUM> a) {
     using C = cplx<T>;
     constexpr int L = glanes(MX), R = gregs(MX), NG = kGNT / L, NCX = MX / 2 + 1;
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -366,7 +376,7 @@ enum { COLS_PIPE = 0, COLS_SPECTRUM = 1, COLS_STD_PIPE = 2, COLS_STD_SPECTRUM = 
 // adjacent columns, so the lanes of a row read at least 64 consecutive bytes.  The columns
 // of the patterns of one ROI run back to back on one XCD (one spectrum column in its L2).
 template <class T, int MY, int MODE>
-__global__ __launch_bounds__(kGNT, 2) void fftg_cols_kernel(fftg_args<T, T, T> a, uint32_t nblk) {
+__global__ __launch_bounds__(kGNT, gwaves<T>(MY, 128, 8)) void fftg_cols_kernel(fftg_args<T, T, T> a, uint32_t nblk) {
     using C = cplx<T>;
     constexpr bool HZ = MODE == COLS_PIPE || MODE == COLS_SPECTRUM;
     constexpr int L = glanes(MY), R = gregs(MY), NG = kGNT / L;
