@@ -27,8 +27,8 @@
 // Bound: the half spectra in HBM.  8 patterns x 81 ROIs of 96 x 96 in double (192 x 192):
 // 0.58 GB written and read, 197 us (rows 31, columns 75, inverse rows 56, peaks 11); radix-4 passes
 // through LDS over 256 x 256, a staged column tile and the correlation written for a peak
-// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 261 us (sums
-// 20, rows 43, columns 87, inverse rows 81, peaks 12), before 606 us.
+// kernel took 495 us.  16 patterns x 42 ROIs of 161 x 95 in float (384 x 192): 252 us (sums
+// 14, rows 43, columns 87, inverse rows 81, peaks 12), before 606 us.
 //
 // Scale: the pattern's spectrum comes out doubled (the omitted split factor); the
 // stored reference spectrum is 2 s.x s.y / (Mx My) times the true one (the same
