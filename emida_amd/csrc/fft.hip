@@ -126,15 +126,15 @@ const cplx<T>* fft_twiddles() {
 template const cplx<float>* fft_twiddles<float>();
 template const cplx<double>* fft_twiddles<double>();
 
-// The larger of two transform outputs, a NaN operand ignored.  The outputs are
-// arithmetic results, never signalling NaNs, so float takes v_max_f32 as is (IEEE
-// maxNum) without the quieting of both operands fmax adds.
-__device__ __forceinline__ float max_quiet(float a, float b) {
+// The largest of three transform outputs, NaN operands ignored.  The outputs are
+// arithmetic results, never signalling NaNs, so float takes v_max3_f32 as is (IEEE
+// maxNum) without the quieting of the operands fmax adds.
+__device__ __forceinline__ float max_quiet(float a, float b, float c) {
     float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
-__device__ __forceinline__ double max_quiet(double a, double b) { return fmax(a, b); }
+__device__ __forceinline__ double max_quiet(double a, double b, double c) { return fmax(fmax(a, b), c); }
 
 // The fit's least-squares rows (6 x kk doubles, kk = F^2 <= 81) in LDS: the loads are
 // issued at the start (clamped addresses, no branch around them), stored once the
@@ -302,8 +302,7 @@ __global__ __launch_bounds__((fft_plan<T, M>::NT), (fft_plan<T, M>::WAVES_PER_SI
             const C v = odd ? C{zk.im + zm.im, zm.re - zk.re} : C{zk.re + zm.re, zk.im - zm.im};
             x[n1] = y < s ? v : C{T(0), T(0)};
         }
-#pragma unroll
-        for (int n1 = R / 2; n1 < R; ++n1) x[n1] = C{T(0), T(0)};
+        // (the second half is zero padding that fft_fwd does not read)
         if (c == 0) {
             // packed real columns 0 and S (wave 0 only): Z[0] and Z[S] of the row pair
 #pragma unroll
@@ -420,8 +419,7 @@ __global__ __launch_bounds__((fft_plan<T, M>::NT), (fft_plan<T, M>::WAVES_PER_SI
                 const int xx = L * n1 + lane;
                 slot[xx] = x[n1];
                 const bool in_x = !PAD || xx <= s || xx > s + pad;
-                vmax = max_quiet(vmax, in_x && in_a ? x[n1].re : lo);
-                vmax = max_quiet(vmax, in_x && in_b ? x[n1].im : lo);
+                vmax = max_quiet(vmax, in_x && in_a ? x[n1].re : lo, in_x && in_b ? x[n1].im : lo);
             }
             if (a.corr_out) {
                 T* cout = a.corr_out + (size_t)sn * s2 * s2;
