@@ -41,6 +41,7 @@ class copy_team {
         cpu_set_t set;
         const int cpus = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : 1;
         const int n = std::min(kHelpers, cpus / 4);
+        helpers.reserve(n > 0 ? n : 0);  // from here on only the threads themselves can fail
         try {
             for (int i = 0; i < n; ++i) helpers.emplace_back([this] { work(); });
         } catch (const std::system_error&) {  // fewer helpers, or none
