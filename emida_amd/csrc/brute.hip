@@ -611,7 +611,7 @@ template <class T, int TB>
 __global__ __launch_bounds__(256, 3) void cross_corr_mm_kernel(const T* __restrict__ pics, const T* __restrict__ ref,
                                                                T* __restrict__ res, size2 size, size2 res_size,
                                                                uint32_t nb, uint32_t npat, mm_shape m,
-                                                               uint32_t n_wg) {
+                                                               uint32_t n_wg, uint32_t slab0) {
     using F = mm_frag<T>;
     constexpr int NJ = F::NJ, TX = NJ * TB, NT = 256;
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -624,7 +624,8 @@ __global__ __launch_bounds__(256, 3) void cross_corr_mm_kernel(const T* __restri
     const int rx = (int)(res_size.x - 1) / 2, ry = (int)(res_size.y - 1) / 2;
     // the workgroups of one slice, then the patterns of one ROI, run back to back on one XCD
     const uint32_t L = xcd_remap(blockIdx.x, n_wg);
-    const uint32_t per = (uint32_t)(m.nxb * m.nyb), slab = L / per, in = L - slab * per;
+    const uint32_t per = (uint32_t)(m.nxb * m.nyb), in_launch = L / per, in = L - in_launch * per;
+    const uint32_t slab = slab0 + in_launch;
     const uint32_t roi = slab / npat, sn = (slab - roi * npat) * nb + roi;
     // workgroups that start together on one CU (32 CUs apart in this order) and waves on one
     // SIMD take different y-shift bands: the central ones are several times longer
@@ -737,20 +738,12 @@ uint64_t tiled_workgroups(size2 size, size2 res_size, uint32_t ref_slices, uint3
     return (n_wg >= 256 && n_wg <= (1u << 24)) ? n_wg : 0;
 }
 
-// Workgroups of the matrix-core kernel, or 0 when the thread-per-shift kernel runs instead
-// (slices too wide for its LDS rows).
-template <class T>
-uint64_t mm_workgroups(size2 size, size2 res_size, uint32_t ref_slices, uint32_t batch, mm_shape& m) {
-    const uint64_t total = (uint64_t)ref_slices * batch;
-    const uint64_t n = mm_plan<T>(size, res_size, total, m) ? total * m.nxb * m.nyb : 0;
-    return n <= 0x7fffffffu ? n : 0;
-}
 
 const char* cross_corr_kernel_name(bool is_double, size2 size, size2 res_size, uint32_t ref_slices, uint32_t batch) {
     mm_shape m;
-    const uint64_t n = is_double ? mm_workgroups<double>(size, res_size, ref_slices, batch, m)
-                                 : mm_workgroups<float>(size, res_size, ref_slices, batch, m);
-    return n ? "cross_corr_mm_kernel" : "cross_corr_kernel";
+    const uint64_t total = (uint64_t)ref_slices * batch;
+    const bool mm = is_double ? mm_plan<double>(size, res_size, total, m) : mm_plan<float>(size, res_size, total, m);
+    return mm ? "cross_corr_mm_kernel" : "cross_corr_kernel";
 }
 
 template <class T>
@@ -766,15 +759,19 @@ void launch_cross_corr(const T* pics, const T* ref, T* res, size2 size, size2 re
     if (!n_tiled && total > 65535u) throw arg_error("cross_corr: more than 65535 slices in one launch");
     if constexpr (std::is_floating_point<T>::value) {
         mm_shape m;
-        if (const uint64_t n_wg = mm_workgroups<T>(size, res_size, ref_slices, batch, m)) {
+        if (mm_plan<T>(size, res_size, total, m)) {
             auto launch = [&](auto tb) {
                 auto kern = cross_corr_mm_kernel<T, decltype(tb)::value>;
                 static const hipError_t attr =
                     hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 155648);
                 EMIDA_HIP(attr);
-                kern<<<(uint32_t)n_wg, 256, m.lds, st>>>(pics, ref, res, size, res_size, ref_slices, batch, m,
-                                                         (uint32_t)n_wg);
-                EMIDA_LAUNCHED("cross_corr_mm_kernel");
+                // a grid's extent is below 2^32 threads: whole slices per launch, one launch nearly always
+                const uint32_t per = (uint32_t)(m.nxb * m.nyb), most = ((1u << 24) - 1) / per;
+                for (uint32_t slab = 0; slab < total; slab += std::min(most, total - slab)) {
+                    const uint32_t n_wg = std::min(most, total - slab) * per;
+                    kern<<<n_wg, 256, m.lds, st>>>(pics, ref, res, size, res_size, ref_slices, batch, m, n_wg, slab);
+                    EMIDA_LAUNCHED("cross_corr_mm_kernel");
+                }
             };
             constexpr int NJ = mm_frag<T>::NJ;
             if (m.tb == 32 / NJ) launch(std::integral_constant<int, 32 / NJ>{});
