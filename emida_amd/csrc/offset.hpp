@@ -153,7 +153,7 @@ struct emida_offset_s {
     void* d_sums = nullptr;
     void* d_ref = nullptr;     // brute: prepared reference slices; FFT: spectra
     void* d_slices = nullptr;  // brute: prepared pattern slices
-    void* d_corr = nullptr;    // brute (and refined matrix-core launches of few patterns): correlation buffers
+    void* d_corr = nullptr;    // brute: correlation buffers
     emida_mfma_mode mfma_mode = EMIDA_MFMA_AUTO;  // as set; mfma_mode_used() is the one in effect
     bool mfma_refine = true;   // matrix-core policy: exact peak from T-precision values
     void* d_ref_lo = nullptr;  // matrix-core policy: lo halves of the reference slices
@@ -166,7 +166,8 @@ struct emida_offset_s {
     // matrix-core policy with refinement: the candidates published in place of the
     // screen (screen_lists) and the norms of the T-precision slices
     void* d_cnt = nullptr;
-    void* d_ent = nullptr;
+    void* d_ent = nullptr;     // or the correlation buffers of a launch of few patterns
+    size_t ent_bytes = 0;
     void* d_pn2 = nullptr;
     void* d_rn2 = nullptr;
     // the reference's cross_corr_fft seam (get_cu_pic / get_cu_temp / cross_corr_fft,
@@ -265,6 +266,10 @@ struct emida_offset_s {
     uint32_t mfma_direct() const {
         return policy == EMIDA_CROSS_POLICY_BRUTE_MFMA && mfma_refine ? mfma_direct_patterns(T == EMIDA_F64, slice) : 0;
     }
+    size_t corr_bytes(uint32_t n_pat) const { return (size_t)nb * n_pat * cross.area() * t_bytes(); }
+    // A launch of few patterns leaves the candidate lists unused: its correlation buffers take
+    // their place, as many as fit.
+    uint32_t direct_in(size_t lists) const { return (uint32_t)std::min<size_t>(mfma_direct(), lists / corr_bytes(1)); }
     size_t scratch_bytes(uint32_t n_pat) const {
         size_t parts[kParts];
         return scratch_sizes(n_pat, parts);
@@ -279,18 +284,14 @@ struct emida_offset_s {
             b += parts[i];
         }
         scratch_t sc{ptr[0], ptr[1], ptr[2], ptr[3], ptr[4], ptr[5], ptr[6], ptr[7], ptr[8]};
-        if (const uint32_t n = mfma_direct()) {
-            // a launch of few patterns leaves the candidate lists unused: its correlation
-            // buffers take their place, as many as fit (so the scratch does not grow)
-            sc.corr = sc.ent;
-            sc.direct = (uint32_t)std::min<size_t>(n, parts[7] / ((size_t)nb * cross.area() * t_bytes()));
-        }
+        if ((sc.direct = direct_in(parts[7]))) sc.corr = sc.ent;
         return sc;
     }
     const void* float_hx() const { return d_hxf ? d_hxf : d_hx; }
     const void* float_hy() const { return d_hyf ? d_hyf : d_hy; }
     scratch_t own_scratch() const {
-        return {d_sums, d_slices, d_corr, d_pic_hi, d_pic_lo, d_smax, d_cnt, d_ent, d_pn2, std::min(batch, mfma_direct())};
+        const uint32_t direct = direct_in(ent_bytes);
+        return {d_sums, d_slices, direct ? d_ent : d_corr, d_pic_hi, d_pic_lo, d_smax, d_cnt, d_ent, d_pn2, direct};
     }
 
     size_t ti_bytes() const { return T == EMIDA_F32 ? 8 : 16; }
@@ -504,10 +505,7 @@ struct emida_offset_s {
                 if (mfma_refine) {
                     d_slices = alloc(scratch_total * slice.area() * t_bytes());
                     d_cnt = alloc(scratch_total * cross.y * sizeof(uint32_t));
-                    d_ent = alloc(scratch_total * cross.y * kListCap * sizeof(cand_entry));
                     d_pn2 = alloc(scratch_total * 2 * sizeof(double));  // norms, then zero-shift products
-                    const size_t direct = (size_t)nb * std::min(batch, mfma_direct());
-                    if (direct) d_corr = alloc(direct * cross.area() * t_bytes());
                 } else {
                     d_corr = alloc(scratch_total * cross.area() * sizeof(float));
                 }
@@ -537,6 +535,18 @@ struct emida_offset_s {
         (void)lstsq_device_table();  // the device tables, before any batch (or graph capture)
         (void)fft_twiddles<float>();
         if (temp) prepare_reference(temp);
+        if (policy == EMIDA_CROSS_POLICY_BRUTE_MFMA && mfma_refine && !resident_only) {
+            // last: lists of a batch below about 8 patterns are smaller than the correlation buffers of
+            // a launch of few: room for those where there is any (else such launches run as others)
+            const size_t lists = scratch_total * cross.y * kListCap * sizeof(cand_entry);
+            const size_t corr = corr_bytes(std::min(batch, mfma_direct()));
+            if (corr > lists && hipMalloc(&d_ent, corr) == hipSuccess) {
+                device_bytes += ent_bytes = corr;
+            } else {
+                (void)hipGetLastError();
+                d_ent = alloc(ent_bytes = lists);
+            }
+        }
         if (temp && policy == EMIDA_CROSS_POLICY_FFT && !resident_only)
             h_ref.assign((const unsigned char*)temp, (const unsigned char*)temp + (size_t)src.area() * in_bytes());
         allocated = true;
