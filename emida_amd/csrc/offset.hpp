@@ -122,6 +122,73 @@ inline void* dmalloc(size_t bytes) {
     return p;
 }
 
+// Pinned memory the host calls stage their batches in, shared by the process's plans: at most
+// kBlocks blocks, given back with the last plan that made a host call.  A block costs 0.4 ms a
+// megabyte once (its pages at the first touch; a staged call of 1.5 MB saves 40 us), so the
+// first call gets none: plans and programs that make one or none pay for none.
+class stage_pool {
+  public:
+    struct block {
+        char* p = nullptr;
+        size_t n = 0;
+    };
+    static std::shared_ptr<stage_pool> get() {
+        static std::mutex mu;
+        static std::weak_ptr<stage_pool> current;
+        std::lock_guard<std::mutex> lock(mu);
+        auto p = current.lock();
+        if (!p) current = p = std::make_shared<stage_pool>();
+        return p;
+    }
+    stage_pool() { idle.reserve(kBlocks); }
+    ~stage_pool() {
+        for (auto& b : idle) (void)hipHostFree(b.p);
+    }
+    stage_pool(const stage_pool&) = delete;
+
+    // A block of at least n bytes, or none: the first call, all in use, or no memory.
+    block take(size_t n) {
+        std::lock_guard<std::mutex> lock(mu);
+        if (!called) {
+            called = true;
+            return {};
+        }
+        size_t at = idle.size();
+        for (size_t i = 0; i < idle.size(); ++i)
+            if (idle[i].n >= n && (at == idle.size() || idle[i].n < idle[at].n)) at = i;
+        if (at < idle.size()) {
+            const block b = idle[at];
+            idle.erase(idle.begin() + (ptrdiff_t)at);
+            return b;
+        }
+        if (live == kBlocks) {
+            if (idle.empty()) return {};
+            (void)hipHostFree(idle.back().p);  // too small: a larger one takes its place
+            idle.pop_back();
+            --live;
+        }
+        block b;
+        b.n = (n + kGrain - 1) & ~(kGrain - 1);
+        if (hipHostMalloc((void**)&b.p, b.n, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            return {};
+        }
+        ++live;
+        return b;
+    }
+    void give(const block& b) {
+        std::lock_guard<std::mutex> lock(mu);
+        idle.push_back(b);
+    }
+
+  private:
+    static constexpr size_t kBlocks = 4, kGrain = 256 << 10;
+    std::mutex mu;
+    std::vector<block> idle;
+    size_t live = 0;
+    bool called = false;
+};
+
 }  // namespace emida_amd
 
 using namespace emida_amd;
@@ -201,14 +268,13 @@ struct emida_offset_s {
     uint64_t stamp = 0;
     std::mutex slot_mu;
 
-    // host call (get_offset): pinned staging of a batch up to kStageMax, its results behind it.
+    // host call (get_offset): staging of a batch up to kStageMax and of results up to as much.
     // Staged / by the runtime, us: 0.18 MB 40 / 64, 1.5 MB 90 / 129, 6 MB 261 / 279, 8 MB 286 /
     // 306; above, the runtime's upload reaches the same rate without the memory.
     static constexpr size_t kStageMax = 8 << 20;
     static constexpr size_t kStagePiece = 256 << 10;  // least part of a batch worth a copy of its own
+    std::shared_ptr<stage_pool> stages;
     std::shared_ptr<copy_team> team;
-    char* h_stage = nullptr;
-    double* h_res = nullptr;
     std::mutex stage_mu;
 
     bool timing = false;
@@ -330,7 +396,6 @@ struct emida_offset_s {
             if (s.h_coefs) (void)hipHostFree(s.h_coefs);
             if (s.done) (void)hipEventDestroy(s.done);
         }
-        if (h_stage) (void)hipHostFree(h_stage);
         for (auto& p : tev) {
             (void)hipEventDestroy(p.first);
             (void)hipEventDestroy(p.second);
@@ -461,13 +526,6 @@ struct emida_offset_s {
             ev_done.push_back(b);
         }
         pending.assign(n_in, 0);
-        if (!resident_only && pic_bytes <= kStageMax) {
-            const size_t n = al256(pic_bytes) + (size_t)total * 8 * sizeof(double);
-            EMIDA_HIP(hipHostMalloc((void**)&h_stage, n, hipHostMallocDefault));
-            std::memset(h_stage, 0, n);  // its pages are there for the first call
-            h_res = (double*)(h_stage + al256(pic_bytes));
-            team = copy_team::get();
-        }
         d_begins = (size2*)alloc(begins.size() * sizeof(size2));
         EMIDA_HIP(hipMemcpy(d_begins, begins.data(), begins.size() * sizeof(size2), hipMemcpyHostToDevice));
         with_T(T, [&](auto t) {
@@ -798,17 +856,40 @@ struct emida_offset_s {
         return e == hipErrorInvalidValue || (e == hipSuccess && a.type == hipMemoryTypeUnregistered);
     }
 
+    // Staging of one host call, given back once the stream no longer uses it.
+    struct stage_lease {
+        stage_pool* pool = nullptr;
+        stage_pool::block b;
+        hipStream_t st = nullptr;
+        bool synced = false;
+        ~stage_lease() {
+            if (!b.p) return;
+            if (!synced) (void)hipStreamSynchronize(st);
+            pool->give(b);
+        }
+    };
+
     // One batch from host memory to results in host memory; coefs may be null.
     void host_call(const void* pic, double* offsets, double* coefs) {
         require_allocated();
         std::lock_guard<std::mutex> lock(stage_mu);
         outset& o = out[out_i];
         out_i ^= 1;
-        const size_t bytes = (size_t)src.area() * batch * in_bytes();
-        const bool stage = h_stage && pageable(pic) && pageable(offsets) && (!coefs || pageable(coefs));
+        const size_t bytes = (size_t)src.area() * batch * in_bytes(), res_bytes = (size_t)total * 8 * sizeof(double);
+        stage_lease lease;
+        if (bytes <= kStageMax && res_bytes <= kStageMax && pageable(pic) && pageable(offsets) &&
+            (!coefs || pageable(coefs))) {
+            if (!stages) stages = stage_pool::get();
+            lease.pool = stages.get();
+            lease.st = compute;
+            lease.b = stages->take(al256(bytes) + res_bytes);
+            if (lease.b.p && !team) team = copy_team::get();
+        }
+        char* h_stage = lease.b.p;
+        double* h_res = (double*)(h_stage + al256(bytes));
         EMIDA_HIP(hipStreamSynchronize(out_stream));
         EMIDA_HIP(hipStreamWaitEvent(compute, ev_done[0], 0));
-        if (stage) {
+        if (h_stage) {
             // parts go to the device as they are copied; the caller's memory is read
             // before this returns, the staging until the synchronisation below
             size_t sent = 0;
@@ -822,29 +903,22 @@ struct emida_offset_s {
                 }
                 sent = m;
             });
-            if (failed) {
-                (void)hipStreamSynchronize(compute);
-                std::rethrow_exception(failed);
-            }
+            if (failed) std::rethrow_exception(failed);
         } else {
             EMIDA_HIP(hipMemcpyAsync(d_in[0], pic, bytes, hipMemcpyHostToDevice, compute));
         }
-        try {
-            run(d_in[0], batch, o.maxes, o.neigh, o.offsets, o.coefs, compute);
-            if (stage) {
-                launch_copy_results(h_res, o.offsets, total * 2, h_res + total * 2, o.coefs, coefs ? total * 6 : 0, compute);
-            } else {
-                EMIDA_HIP(hipMemcpyAsync(offsets, o.offsets, total * 2 * sizeof(double), hipMemcpyDeviceToHost, compute));
-                if (coefs)
-                    EMIDA_HIP(hipMemcpyAsync(coefs, o.coefs, total * 6 * sizeof(double), hipMemcpyDeviceToHost, compute));
-            }
-        } catch (...) {
-            (void)hipStreamSynchronize(compute);  // the staging is written again by the next call
-            throw;
+        run(d_in[0], batch, o.maxes, o.neigh, o.offsets, o.coefs, compute);
+        if (h_stage) {
+            launch_copy_results(h_res, o.offsets, total * 2, h_res + total * 2, o.coefs, coefs ? total * 6 : 0, compute);
+        } else {
+            EMIDA_HIP(hipMemcpyAsync(offsets, o.offsets, total * 2 * sizeof(double), hipMemcpyDeviceToHost, compute));
+            if (coefs)
+                EMIDA_HIP(hipMemcpyAsync(coefs, o.coefs, total * 6 * sizeof(double), hipMemcpyDeviceToHost, compute));
         }
         EMIDA_HIP(hipEventRecord(ev_done[0], compute));
         EMIDA_HIP(hipStreamSynchronize(compute));
-        if (stage) {
+        if (h_stage) {
+            lease.synced = true;
             std::memcpy(offsets, h_res, total * 2 * sizeof(double));
             if (coefs) std::memcpy(coefs, h_res + total * 2, total * 6 * sizeof(double));
         }
