@@ -226,13 +226,12 @@ int emida_offset_get_timing(emida_offset* h, const char** kernel_name, double* t
             (void)hipEventDestroy(p.second);
         }
         h->tev.clear();
-        if (kernel_name)
-            *kernel_name = h->policy == EMIDA_CROSS_POLICY_FFT
-                               ? (h->fftg ? "fftg_rows_kernel+fftg_cols_kernel+fftg_rows_inv_kernel"
-                                          : fft_padded(h->side) > 128 ? "fft256_kernel" : "fft_kernel")
-                               : (h->policy == EMIDA_CROSS_POLICY_BRUTE_MFMA && h->batch > h->mfma_direct()
-                                      ? "mfma_corr_kernel"
-                                      : cross_corr_kernel_name(h->T == EMIDA_F64, h->slice, h->cross, h->nb, h->batch));
+        if (h->t_names.empty()) {  // nothing timed yet: a full batch's
+            const bool direct = h->batch <= h->mfma_direct();
+            if (kernel_name) *kernel_name = h->timed_kernel(h->batch, direct);
+        } else if (kernel_name) {
+            *kernel_name = h->t_names.c_str();
+        }
         if (total_ms) *total_ms = h->t_ms;
         if (launches) *launches = h->t_launches;
     });

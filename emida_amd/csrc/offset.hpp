@@ -279,6 +279,7 @@ struct emida_offset_s {
 
     bool timing = false;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> tev;
+    std::string t_names;  // kernels of the timed launches, each once, joined by '+'
     double t_ms = 0;
     uint64_t t_launches = 0;
 
@@ -726,7 +727,7 @@ struct emida_offset_s {
                         launch_prepare<IT, TT, ST>(pics, (TT*)sc.slices, (const TT*)d_hx, (const TT*)d_hy, sums,
                                                    d_begins, src, slice, slice, nb, tn, st);
                     }
-                    if (timing) t0 = record_start(st);
+                    if (timing) t0 = record_start(st, timed_kernel(n_pat, direct));
                     launch_cross_corr<TT>((const TT*)sc.slices, ref, (TT*)sc.corr, slice, cross, nb, n_pat, st);
                     if (timing) record_stop(st, t0);
                     launch_peak<TT>((const TT*)sc.corr, (size_t)tn * cross.area(), cross.area(), cross, POLICY_BRUTE,
@@ -768,7 +769,7 @@ struct emida_offset_s {
                         }
                         const mfma_src msrc{(const uint16_t*)pics, (const uint32_t*)sums, (const float*)float_hx(),
                                             (const float*)float_hy(), d_begins, src};
-                        if (timing) t0 = record_start(st);
+                        if (timing) t0 = record_start(st, timed_kernel(n_pat, direct));
                         launch_mfma_corr<HT>(phi, plo, (const HT*)d_ref, (const HT*)d_ref_lo,
                                              mfma_refine ? nullptr : (float*)sc.corr, slice, cross, nb, n_pat, st,
                                              (uint32_t*)sc.smax, mfma_refine ? &lists : nullptr, u16 ? &msrc : nullptr);
@@ -787,7 +788,7 @@ struct emida_offset_s {
                 } else {
                     if (!std::is_same<IT, uint16_t>::value)
                         launch_sum<IT, ST>(pics, sums, d_begins, src, slice, nb, tn, st);
-                    if (timing) t0 = record_start(st);
+                    if (timing) t0 = record_start(st, timed_kernel(n_pat, direct));
                     if (fftg)
                         launch_fftg_pipe<TT, IT, ST>(pics, sums, (const TT*)d_hx, (const TT*)d_hy, d_begins, src,
                                                      slice, nb, tn, (const cplx<TT>*)d_ref, fit,
@@ -803,7 +804,18 @@ struct emida_offset_s {
         (void)t1;
     }
 
-    hipEvent_t record_start(hipStream_t st) {
+    // What is timed of a launch of n_pat patterns.
+    const char* timed_kernel(uint32_t n_pat, bool direct) const {
+        if (policy == EMIDA_CROSS_POLICY_FFT)
+            return fftg ? "fftg_rows_kernel+fftg_cols_kernel+fftg_rows_inv_kernel+fftg_peak_kernel"
+                        : fft_padded(side) > 128 ? "fft256_kernel" : "fft_kernel";
+        if (policy == EMIDA_CROSS_POLICY_BRUTE_MFMA && !direct) return "mfma_corr_kernel";
+        return cross_corr_kernel_name(T == EMIDA_F64, slice, cross, nb, n_pat);
+    }
+
+    hipEvent_t record_start(hipStream_t st, const std::string& name) {
+        if (("+" + t_names + "+").find("+" + name + "+") == std::string::npos)
+            t_names += (t_names.empty() ? "" : "+") + name;
         hipEvent_t a, b;
         EMIDA_HIP(hipEventCreate(&a));
         EMIDA_HIP(hipEventCreate(&b));

@@ -207,7 +207,8 @@ int emida_offset_set_mfma_refine(emida_offset* h, int enable);
 
 /* Kernel timing with HIP events on the stream the kernels run on.  Returns the
  * summed time and launch count of the dominant kernel (the FFT pipeline kernel
- * for FFT, the correlation kernel for brute) since timing was enabled. */
+ * for FFT, the correlation kernel for brute) since timing was enabled.  kernel_name: the
+ * kernels of the timed launches, joined by '+', valid until the object's next timed launch. */
 int emida_offset_set_timing(emida_offset* h, int enable);
 int emida_offset_get_timing(emida_offset* h, const char** kernel_name, double* total_ms, uint64_t* launches);
 
