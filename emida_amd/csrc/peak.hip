@@ -274,9 +274,14 @@ __global__ void subpixel_kernel(const T* __restrict__ neigh, int s, uint32_t n, 
 // without a finite screen maximum is swept whole: every shift of the window is
 // evaluated exactly, box by box, so its arg-max is the brute policy's as well.
 constexpr int kRefineCap = 512;
-// Boxes tried on candidates too wide for one before the rest are evaluated one chain per
-// lane (128 x 128 double slices: a box 0.05 to 0.1 ms, a round of chains 0.7 ms).
-constexpr int kSpreadBoxes = 6;
+// Candidates too wide for one box take boxes of 16 x 16, up to this many for every round it
+// would take to evaluate them one chain per lane, else the chains.  Boxes are counted first:
+// evaluating six and then the chains all the same cost unrelated 128 x 128 patterns (160
+// slices, more than six boxes) 1.43 ms in float and 1.39 in double, where the chains take 0.57
+// and 0.70; a limit of four boxes 0.92 and 0.83.  In float, whose products wait longer on one
+// another, two boxes cost what the chains do.
+template <class T>
+constexpr int kSpreadBoxes = sizeof(T) == 8 ? 2 : 0;
 constexpr int kRowList = 256;  // screens of at most this many rows use the row maxima
 
 template <class T>
@@ -676,8 +681,8 @@ __global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__
     const int k = fit * fit, rad = (fit - 1) / 2;
     // One box when the candidates' box grown by the fit radius fits: it holds every candidate
     // and the in-window neighbourhood of any of them.  Else one box of the candidates; else
-    // (spread candidates) boxes of 16 x 16 around the first one left, and after a few of them
-    // one chain per lane for the rest; a swept slice takes the whole window in boxes.
+    // (spread candidates) boxes of 16 x 16 around the first one left where few hold them all,
+    // one chain per lane where not; a swept slice takes the whole window in boxes.
     const int cbw = bb[2] - bb[0] + 1, cbh = bb[3] - bb[1] + 1;
     const int ex0 = max(0, bb[0] - rad), ey0 = max(0, bb[1] - rad);
     const int ebw = min((int)cross.x - 1, bb[2] + rad) - ex0 + 1, ebh = min((int)cross.y - 1, bb[3] + rad) - ey0 + 1;
@@ -692,7 +697,33 @@ __global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__
         }
     };
     size2 mp{0, 0};
-    int bx0 = 0, by0 = 0, bw = 0, bh = 0, spread = 0;
+    int bx0 = 0, by0 = 0, bw = 0, bh = 0;
+    constexpr uint32_t kTaken = 1u << 31;  // mark of a candidate whose box has been taken
+    auto next_box = [&] {                  // of the lowest one left
+        uint32_t first = kTaken;
+        for (uint32_t c = tid; c < nc; c += NT) first = min(first, cand[c]);
+        first = block_min_u32<NT>(first, si);
+        bx0 = max(0, (int)(first % cross.x) - 8);
+        by0 = (int)(first / cross.x);
+        bw = min(16, (int)cross.x - bx0);
+        bh = min(16, (int)cross.y - by0);
+        return first < kTaken;
+    };
+    auto in_box = [&](uint32_t i, int& x, int& y) {
+        x = (int)(i % cross.x) - bx0;
+        y = (int)(i / cross.x) - by0;
+        return x >= 0 && y >= 0 && x < bw && y < bh;
+    };
+    bool chains = !sweep && !boxed;
+    if (kSpreadBoxes<T> && chains) {
+        int n = 0, x, y;
+        const int most = kSpreadBoxes<T> * (int)div_up(nc, (uint32_t)NT);
+        while ((chains = next_box()) && ++n <= most) {
+            for (uint32_t c = tid; c < nc; c += NT)
+                if (cand[c] < kTaken && in_box(cand[c], x, y)) cand[c] |= kTaken;
+        }
+        for (uint32_t c = tid; c < nc; c += NT) cand[c] &= ~kTaken;
+    }
     enum { CANDIDATES, SWEEP, PEAK };
     for (int mode = sweep ? SWEEP : CANDIDATES;;) {
         if (mode == CANDIDATES) {
@@ -701,14 +732,8 @@ __global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__
                 by0 = merged ? ey0 : bb[1];
                 bw = merged ? ebw : cbw;
                 bh = merged ? ebh : cbh;
-            } else {
-                uint32_t first = 0xffffffffu;
-                for (uint32_t c = tid; c < nc; c += NT) first = min(first, cand[c]);
-                first = block_min_u32<NT>(first, si);
-                bx0 = max(0, (int)(first % cross.x) - 8);
-                by0 = (int)(first / cross.x);
-                bw = min(16, (int)cross.x - bx0);
-                bh = min(16, (int)cross.y - by0);
+            } else if (!chains) {
+                next_box();
             }
         } else if (mode == SWEEP) {
             bw = min(kBoxW, (int)cross.x - bx0);
@@ -719,28 +744,27 @@ __global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__
             bw = min((int)cross.x - 1, (int)mp.x + rad) - bx0 + 1;
             bh = min((int)cross.y - 1, (int)mp.y + rad) - by0 + 1;
         }
-        eval_box<T, NT, KS>(ps, rs, s, cross, bx0, by0, bw, bh, rbuf, boxv);
+        if (mode == CANDIDATES && chains) {
+            for (uint32_t c = tid; c < nc; c += NT)
+                offer(exact_at<T>((size_t)sn * area + cand[c], corr_len, p, r, s, cross, nb), cand[c]);
+        } else {
+            eval_box<T, NT, KS>(ps, rs, s, cross, bx0, by0, bw, bh, rbuf, boxv);
+        }
         if (mode == PEAK) break;
         if (mode == CANDIDATES) {
-            uint32_t left = 0;
-            for (uint32_t c = tid; c < nc; c += NT) {
-                const uint32_t i = cand[c];
-                if (i == 0xffffffffu) continue;
-                const int x = (int)(i % cross.x) - bx0, y = (int)(i / cross.x) - by0;
-                if (x >= 0 && y >= 0 && x < bw && y < bh) {
-                    offer(boxv[y * kBoxW + x], i);
-                    cand[c] = 0xffffffffu;  // done
-                } else {
-                    ++left;
-                }
-            }
-            if (__syncthreads_or((int)left)) {
-                if (++spread < kSpreadBoxes * (int)div_up(nc, (uint32_t)NT)) continue;
+            if (!chains) {
+                int left = 0, x, y;
                 for (uint32_t c = tid; c < nc; c += NT) {
                     const uint32_t i = cand[c];
-                    if (i != 0xffffffffu)
-                        offer(exact_at<T>((size_t)sn * area + i, corr_len, p, r, s, cross, nb), i);
+                    if (i >= kTaken) continue;
+                    if (in_box(i, x, y)) {
+                        offer(boxv[y * kBoxW + x], i);
+                        cand[c] = kTaken;
+                    } else {
+                        ++left;
+                    }
                 }
+                if (__syncthreads_or(left)) continue;
             }
         } else {
             for (int e = tid; e < bw * bh; e += NT) {
