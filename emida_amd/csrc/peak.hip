@@ -516,9 +516,9 @@ __global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__
     __shared__ uint32_t cand[kRefineCap];
     __shared__ uint32_t ncand, nrow, overflow;
     __shared__ uint16_t rlist[kRowList];  // rows of the screen that can hold candidates
+    __shared__ uint8_t rcnt[kRowList];    // and how many they hold
     __shared__ T nbv[81];
     __shared__ double cf[6];
-    __shared__ int bb[4];
     __shared__ T rbuf[NT / kWave * 2 * kRowBuf];  // reference rows of eval_box
     __shared__ T boxv[kBoxRows * kBoxW];          // the box values it leaves
     if (blockIdx.x >= total) return;
@@ -608,28 +608,38 @@ __global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__
         if (smax && idx < area && v == m && idx < mil) mil = idx;
     };
     if (lists.cnt) {
-        // the rows that can hold a candidate, then the positions they published (a row
-        // with more than kListCap of them makes the slice sweep)
+        // the rows that can hold a candidate, then the positions they published, several loads
+        // in flight; a row with more than kListCap of them, or more rows than the list holds,
+        // make the slice sweep, which needs none
         for (uint32_t r = tid; r < cross.y; r += NT) {
-            const uint32_t code = smax[(size_t)sn * cross.y + r];
+            const uint32_t code = smax[(size_t)sn * cross.y + r], c = lists.cnt[(size_t)sn * cross.y + r];
             if (code && ((double)screen_max_value(code) >= thr || code == mcode)) {
                 const uint32_t k = atomicAdd(&nrow, 1u);
-                if (k < (uint32_t)kRowList) rlist[k] = r;
-                else overflow = 1;  // more rows than the list holds: sweep
+                if (k < (uint32_t)kRowList) {
+                    rlist[k] = r;
+                    rcnt[k] = (uint8_t)min(c, (uint32_t)kListCap);
+                }
+                if (k >= (uint32_t)kRowList || c > (uint32_t)kListCap) overflow = 1;
             }
         }
         __syncthreads();
-        const uint32_t n = min(nrow, (uint32_t)kRowList) * (uint32_t)kListCap;
-        for (uint32_t e = tid; e < n; e += NT) {
-            const uint32_t row = rlist[e / kListCap], k = e % kListCap;
-            const size_t rr = (size_t)sn * cross.y + row;
-            const uint32_t c = lists.cnt[rr];
-            if (c > (uint32_t)kListCap) {
-                if (k == 0) overflow = 1;
-            } else if (k < c) {
-                const cand_entry en = lists.ent[rr * kListCap + k];
-                take(row * cross.x + en.x, en.v);
+        const uint32_t n = overflow ? 0u : nrow * (uint32_t)kListCap;
+        const cand_entry* ent = lists.ent + (size_t)sn * cross.y * kListCap;
+        constexpr int V = 4;
+        for (uint32_t e0 = tid; e0 < n; e0 += NT * V) {
+            cand_entry en[V];
+            uint32_t row[V];
+            bool on[V];
+#pragma unroll
+            for (int q = 0; q < V; ++q) {
+                const uint32_t e = min(e0 + NT * q, n - 1), k = e % kListCap;
+                row[q] = rlist[e / kListCap];
+                on[q] = e == e0 + NT * q && k < rcnt[e / kListCap];
+                en[q] = ent[on[q] ? row[q] * kListCap + k : 0];
             }
+#pragma unroll
+            for (int q = 0; q < V; ++q)
+                if (on[q]) take(row[q] * cross.x + en[q].x, en[q].v);
         }
     } else if (smax && cross.y <= (uint32_t)kRowList) {
         for (uint32_t r = tid; r < cross.y; r += NT) {
@@ -665,19 +675,15 @@ __global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__
     const uint32_t nc = sweep ? 0u : ncand;
     // exact values; arg-max with the lowest index on ties.  Candidates whose bounding
     // box fits one box evaluation take the staged path, others one chain each.
-    if (tid == 0) {
-        bb[0] = bb[1] = 1 << 30;
-        bb[2] = bb[3] = -1;
-    }
-    __syncthreads();
+    // (in registers: with four LDS updates per candidate, 225 ties of a flat 8 x 8 slice took 28 of
+    // the kernel's 41 us)
+    uint32_t ux0 = 0xffffffffu, uy0 = ux0, ux1 = ux0, uy1 = ux0;
     for (uint32_t c = tid; c < nc; c += NT) {
-        const int cx = (int)(cand[c] % cross.x), cy = (int)(cand[c] / cross.x);
-        atomicMin(&bb[0], cx);
-        atomicMin(&bb[1], cy);
-        atomicMax(&bb[2], cx);
-        atomicMax(&bb[3], cy);
+        const uint32_t cx = cand[c] % cross.x, cy = cand[c] / cross.x;
+        ux0 = min(ux0, cx), uy0 = min(uy0, cy), ux1 = min(ux1, ~cx), uy1 = min(uy1, ~cy);
     }
-    __syncthreads();
+    const int bb[4] = {(int)block_min_u32<NT>(ux0, si), (int)block_min_u32<NT>(uy0, si),
+                       (int)~block_min_u32<NT>(ux1, si), (int)~block_min_u32<NT>(uy1, si)};
     const int k = fit * fit, rad = (fit - 1) / 2;
     // One box when the candidates' box grown by the fit radius fits: it holds every candidate
     // and the in-window neighbourhood of any of them.  Else one box of the candidates; else
