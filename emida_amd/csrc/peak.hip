@@ -392,7 +392,7 @@ __device__ __forceinline__ void box_sums(const T* __restrict__ p, const T* __res
                                          int sy0, int y0, int y1, T* rbuf, T* out) {
     using F = box_frag<T>;
     constexpr int NJ = F::NJ, SH = NJ / 4, SPAN = NJ * NF - 1, PER = kRowBuf / kWave;
-    constexpr int GS = KS < 8 ? KS : 8;
+    constexpr int GS = KS % 8 ? 4 : 8;  // steps per group, whose operands load together
     static_assert(4 * KS + SPAN <= kRowBuf, "reference row buffer");
     const int lane = threadIdx.x % kWave, i = lane % 16, k = lane / 16, j = F::col(lane);
     // groups of GS steps that hold terms of the box
@@ -594,6 +594,20 @@ __global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__
     tau = tol_rel * np * nr + tol_abs * (np + nr);
     }
 
+    // Slices that fit the vector L1 are touched while the candidates are found: the box reads
+    // them a row ahead, which hides an L1 hit but not a read from HBM (16 x 128 in float, 784
+    // slices: refinement 78 us, 54 touched; beyond these sizes it gains nothing or evicts).
+    constexpr int LINE = 128 / (int)sizeof(T), LINES = 4 * kWave / NT;
+    constexpr size_t kTouch = NT == kWave ? 8192 : 16384;  // bytes of a slice
+    const bool touch = a * sizeof(T) <= kTouch;
+    T warm[2 * LINES];
+#pragma unroll
+    for (int k = 0; k < LINES; ++k) {
+        const size_t i = touch ? min((size_t)(tid + NT * k) * LINE, a - 1) : 0;
+        warm[2 * k] = ps[i];
+        warm[2 * k + 1] = rs[i];
+    }
+
     // candidates.  Given the row maxima, only rows whose maximum reaches the threshold
     // (or equals the slice maximum) can hold one, and only those rows are read.
     if (tid == 0) ncand = nrow = overflow = 0;
@@ -671,6 +685,8 @@ __global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__
     }
     if (smax) mi = block_min_u32<NT>(mil, si);
     __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2 * LINES; ++k) asm volatile("" ::"v"(warm[k]));  // (keeps the loads)
     const bool sweep = ncand > (uint32_t)kRefineCap || mi == 0xffffffffu || overflow;
     const uint32_t nc = sweep ? 0u : ncand;
     // exact values; arg-max with the lowest index on ties.  Candidates whose bounding
@@ -894,6 +910,8 @@ void launch_refine(const float* screen, size_t corr_len, const T* p, const T* r,
     };
     if (s.x <= 16) launch(std::integral_constant<int, 4>{});
     else if (s.x <= 32) launch(std::integral_constant<int, 8>{});
+    // (40 x 24 in double, 4,000 swept slices: 549 us with 16 steps, 436 with 12)
+    else if (s.x <= 48) launch(std::integral_constant<int, 12>{});
     else if (s.x <= 64) launch(std::integral_constant<int, 16>{});
     else launch(std::integral_constant<int, 32>{});
     EMIDA_LAUNCHED("refine_kernel");
