@@ -6,8 +6,8 @@
 // inner, as fused multiply-adds (the reference's nvcc build contracts
 // `sum += a * b`), so double and float results are bit-identical to that order.
 //
-// Float and double run on the matrix cores (cross_corr_mm_kernel); slices too wide for its
-// LDS rows take the thread-per-shift kernel: one workgroup per (slice, 4-row band of shifts,
+// Float and double run on the matrix cores (cross_corr_mm_kernel); slices of a few pixels and
+// those too wide for its LDS rows take the thread-per-shift kernel: one workgroup per (slice, 4-row band of shifts,
 // 64-column band of shifts), staged in LDS when both slices fit in 64 KiB.  int32 has no
 // matrix instruction with its wrapping sums and keeps the vector kernels: a register-blocked
 // one ("tiled") for slices up to 128 pixels wide, windows up to 256 wide and launches of at
@@ -404,7 +404,7 @@ struct mm_shape {
     int tb;              // fragments per tile
     int x0;              // first x-shift of tile 0
     int ntx, nty;        // tiles of a slice
-    int wx, wy;          // waves along x-shift tiles and y-shift tiles (wx * wy = 4)
+    int wx, wy;          // waves along x-shift tiles and y-shift tiles (wx * wy = 4, or one)
     int ntw;             // x-shift tiles per wave (1 or 2)
     int nxb, nyb;        // workgroups of one slice along x and y
     int cy;              // reference rows per staged chunk
@@ -446,6 +446,14 @@ inline bool mm_plan(size2 size, size2 res, uint64_t total, mm_shape& m) {
     const int per = div_up(m.ntx, m.ntw);
     m.wx = per >= 4 ? 4 : (per >= 2 ? 2 : 1);
     m.wy = 4 / m.wx;
+    // Small slices of one or two tiles take one wave each: beside it the other three would only
+    // stage, which pays for larger slices and tall ones (brute pass over 800 slices of 24 x 8 in
+    // float: 24.1 us with four waves, 19.9 with one; 8 x 8: 16.2 and 14.0; 100 of 24 x 24 with a
+    // 9 x 9 window 17.8 and 19.4).
+    if (size.area() <= 256 && size.y <= 16 && m.nty == 1 && m.ntx <= 2) {
+        m.ntw = m.ntx;
+        m.wx = m.wy = 1;
+    }
     m.nxb = div_up(m.ntx, m.wx * m.ntw);
     m.nyb = div_up(m.nty, m.wy);
     // Pattern rows 2 mod 4 doubles (4 mod 8 floats) apart: the rows of an A fragment fall on
@@ -607,13 +615,13 @@ __device__ __forceinline__ void mm_tile(mm_f4 (&acc)[TB], int y0, int y1, PA&& p
     }
 }
 
-template <class T, int TB>
-__global__ __launch_bounds__(256, 3) void cross_corr_mm_kernel(const T* __restrict__ pics, const T* __restrict__ ref,
+template <class T, int TB, int NW>
+__global__ __launch_bounds__(64 * NW, 3) void cross_corr_mm_kernel(const T* __restrict__ pics, const T* __restrict__ ref,
                                                                T* __restrict__ res, size2 size, size2 res_size,
                                                                uint32_t nb, uint32_t npat, mm_shape m,
                                                                uint32_t n_wg, uint32_t slab0) {
     using F = mm_frag<T>;
-    constexpr int NJ = F::NJ, TX = NJ * TB, NT = 256;
+    constexpr int NJ = F::NJ, TX = NJ * TB, NT = kWave * NW;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* prow = reinterpret_cast<T*>(smem_raw);  // prows pattern rows, then one zero row
     T* zrow = prow + (size_t)m.prows * m.pitch;
@@ -635,7 +643,7 @@ __global__ __launch_bounds__(256, 3) void cross_corr_mm_kernel(const T* __restri
     const T* p = pics + (size_t)sn * size.area();
     const T* q = ref + (size_t)roi * size.area();
 
-    const int wv = (wave + (int)(turn / per)) & 3;
+    const int wv = (wave + (int)(turn / per)) & (NW - 1);
     const int wxi = wv % m.wx, wyi = wv / m.wx;
     const int sy0g = yb * kMmTY * m.wy - ry;       // first y-shift of the workgroup
     const int sy0 = sy0g + kMmTY * wyi;            // and of the wave
@@ -739,11 +747,16 @@ uint64_t tiled_workgroups(size2 size, size2 res_size, uint32_t ref_slices, uint3
 }
 
 
+// Slices up to this many pixels run one thread per shift: the chains are shorter than what the
+// matrix-core kernel does around them (pass over 800 slices in double, us: 4 x 4 16.2 and 12.1,
+// 6 x 6 17.0 and 14.2; 8 x 8 in float 16.2 and 17.8).
+constexpr uint32_t kTinyArea = 48;
+
 const char* cross_corr_kernel_name(bool is_double, size2 size, size2 res_size, uint32_t ref_slices, uint32_t batch) {
     mm_shape m;
     const uint64_t total = (uint64_t)ref_slices * batch;
     const bool mm = is_double ? mm_plan<double>(size, res_size, total, m) : mm_plan<float>(size, res_size, total, m);
-    return mm ? "cross_corr_mm_kernel" : "cross_corr_kernel";
+    return mm && !(total <= 65535u && size.area() <= kTinyArea) ? "cross_corr_mm_kernel" : "cross_corr_kernel";
 }
 
 template <class T>
@@ -759,9 +772,9 @@ void launch_cross_corr(const T* pics, const T* ref, T* res, size2 size, size2 re
     if (!n_tiled && total > 65535u) throw arg_error("cross_corr: more than 65535 slices in one launch");
     if constexpr (std::is_floating_point<T>::value) {
         mm_shape m;
-        if (mm_plan<T>(size, res_size, total, m)) {
-            auto launch = [&](auto tb) {
-                auto kern = cross_corr_mm_kernel<T, decltype(tb)::value>;
+        if (!(total <= 65535u && size.area() <= kTinyArea) && mm_plan<T>(size, res_size, total, m)) {
+            auto launch_nw = [&](auto tb, auto nw) {
+                auto kern = cross_corr_mm_kernel<T, decltype(tb)::value, decltype(nw)::value>;
                 static const hipError_t attr =
                     hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 155648);
                 EMIDA_HIP(attr);
@@ -769,9 +782,14 @@ void launch_cross_corr(const T* pics, const T* ref, T* res, size2 size, size2 re
                 const uint32_t per = (uint32_t)(m.nxb * m.nyb), most = ((1u << 24) - 1) / per;
                 for (uint32_t slab = 0; slab < total; slab += std::min(most, total - slab)) {
                     const uint32_t n_wg = std::min(most, total - slab) * per;
-                    kern<<<n_wg, 256, m.lds, st>>>(pics, ref, res, size, res_size, ref_slices, batch, m, n_wg, slab);
+                    kern<<<n_wg, kWave * nw, m.lds, st>>>(pics, ref, res, size, res_size, ref_slices, batch, m, n_wg,
+                                                          slab);
                     EMIDA_LAUNCHED("cross_corr_mm_kernel");
                 }
+            };
+            auto launch = [&](auto tb) {
+                if (m.wx * m.wy == 1) launch_nw(tb, std::integral_constant<int, 1>{});
+                else launch_nw(tb, std::integral_constant<int, 4>{});
             };
             constexpr int NJ = mm_frag<T>::NJ;
             if (m.tb == 32 / NJ) launch(std::integral_constant<int, 32 / NJ>{});
