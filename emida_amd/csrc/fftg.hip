@@ -212,7 +212,7 @@ __device__ __forceinline__ void gfft_inv(cplx<T> (&x)[gregs(M)], int lane, T* sc
 
 }  // namespace
 
-// Arguments of the three kernels (one launch chunk of slices first .. first + total - 1).
+// Arguments of the four kernels (one launch chunk of slices first .. first + total - 1).
 template <class T, class IN, class SUM>
 struct fftg_args {
     const IN* pics;          // patterns (rows kernel, from pattern)
@@ -245,14 +245,15 @@ struct fftg_args {
     double* coefs;
 };
 
-// Waves per SIMD the registers are budgeted for.  Forward rows of 384 in float and columns of
-// 128 in double need 186 and 172 registers by themselves and none of them in scratch at 168,
-// which lets a third workgroup share a CU (the LDS holds three): 672 slices of 161 x 95 in float
-// 277 -> 261 us, 2304 of 60 x 50 in double 212 -> 200.  The other kernels above 168 would spill
-// 60 bytes to 800 a lane.
+// Waves per SIMD the registers are budgeted for.  The pipeline's forward rows of 384 in float
+// and columns of 128 in double need 186 and 172 registers by themselves and none of them in
+// scratch at 168, which lets a third workgroup share a CU (the LDS holds three): 672 slices of
+// 161 x 95 in float 277 -> 261 us, 2304 of 60 x 50 in double 212 -> 200.  The other kernels
+// above 168 would spill 12 bytes to 800 a lane, among them the same lengths without zero
+// padding (hz).
 template <class T>
-constexpr int gwaves(int m, int three, int size) {
-    return m == three && sizeof(T) == size ? 3 : 2;
+constexpr int gwaves(int m, int three, int size, bool hz) {
+    return m == three && sizeof(T) == size && hz ? 3 : 2;
 }
 
 // ---------------------------------------------------------------- kernel 1: rows
@@ -260,7 +261,7 @@ constexpr int gwaves(int m, int three, int size) {
 // Grid: (slices, splits); a slice's splits take its row pairs in turn (uint16: each sums
 // the whole slice for the mean).
 template <class T, class IN, class SUM, int MX, bool FROM_PATTERN, bool HZ>
-__global__ __launch_bounds__(kGNT, gwaves<T>(MX, 384, 4)) void fftg_rows_kernel(fftg_args<T, IN, SUM> a) {
+__global__ __launch_bounds__(kGNT, gwaves<T>(MX, 384, 4, HZ)) void fftg_rows_kernel(fftg_args<T, IN, SUM> a) {
     using C = cplx<T>;
     constexpr int L = glanes(MX), R = gregs(MX), NG = kGNT / L, NCX = MX / 2 + 1;
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -371,14 +372,15 @@ __global__ __launch_bounds__(kGNT, gwaves<T>(MX, 384, 4)) void fftg_rows_kernel(
 
 // ---------------------------------------------------------------- kernel 2: columns
 enum { COLS_PIPE = 0, COLS_SPECTRUM = 1, COLS_STD_PIPE = 2, COLS_STD_SPECTRUM = 3 };
+constexpr bool gcols_hz(int mode) { return mode == COLS_PIPE || mode == COLS_SPECTRUM; }
 
 // One column per lane group, read and written in place: the NG groups of a workgroup take
 // adjacent columns, so the lanes of a row read at least 64 consecutive bytes.  The columns
 // of the patterns of one ROI run back to back on one XCD (one spectrum column in its L2).
 template <class T, int MY, int MODE>
-__global__ __launch_bounds__(kGNT, gwaves<T>(MY, 128, 8)) void fftg_cols_kernel(fftg_args<T, T, T> a, uint32_t nblk) {
+__global__ __launch_bounds__(kGNT, gwaves<T>(MY, 128, 8, gcols_hz(MODE))) void fftg_cols_kernel(fftg_args<T, T, T> a, uint32_t nblk) {
     using C = cplx<T>;
-    constexpr bool HZ = MODE == COLS_PIPE || MODE == COLS_SPECTRUM;
+    constexpr bool HZ = gcols_hz(MODE);
     constexpr int L = glanes(MY), R = gregs(MY), NG = kGNT / L;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     C* tw = reinterpret_cast<C*>(lds_raw);
@@ -641,13 +643,14 @@ __global__ __launch_bounds__(gpeak_nt(MX)) void fftg_peak_kernel(fftg_args<T, T,
 // ---------------------------------------------------------------- launchers
 namespace {
 
-template <class T, int N, class F>
+// THIRDS: also the lengths 192 and 384 (the reference's own transforms are powers of two).
+template <class T, int N, bool THIRDS, class F>
 void dispatch_n(uint32_t n, F&& f) {
     if constexpr (N <= 512) {
         if (n == (uint32_t)N) return f(std::integral_constant<int, N>{});
-        if constexpr (N == 128 || (N == 256 && sizeof(T) == 4))
+        if constexpr (THIRDS && (N == 128 || (N == 256 && sizeof(T) == 4)))
             if (n == (uint32_t)(N / 2 * 3)) return f(std::integral_constant<int, N / 2 * 3>{});
-        return dispatch_n<T, N * 2>(n, std::forward<F>(f));
+        return dispatch_n<T, N * 2, THIRDS>(n, std::forward<F>(f));
     } else {
         throw unsupported_error("FFT policy: transform side " + std::to_string(n) + " is beyond 512");
     }
@@ -660,7 +663,7 @@ void set_lds(K kern, size_t bytes) {
 
 template <class T, class IN, class SUM, bool FP, bool HZ>
 void run_rows(const fftg_args<T, IN, SUM>& a, hipStream_t st) {
-    dispatch_n<T, 4>(a.mx, [&](auto mc) {
+    dispatch_n<T, 4, HZ>(a.mx, [&](auto mc) {
         constexpr int MX = decltype(mc)::value, NG = kGNT / glanes(MX);
         auto k = fftg_rows_kernel<T, IN, SUM, MX, FP, HZ>;
         static const bool once = (set_lds(k, glds<T>(MX)), true);
@@ -676,7 +679,7 @@ void run_rows(const fftg_args<T, IN, SUM>& a, hipStream_t st) {
 template <class T, int MODE>
 void run_cols(fftg_args<T, T, T> a, hipStream_t st) {
     a.npat = a.first % a.nb == 0 && a.total % a.nb == 0 ? a.total / a.nb : 0;
-    dispatch_n<T, 4>(a.my, [&](auto mc) {
+    dispatch_n<T, 4, gcols_hz(MODE)>(a.my, [&](auto mc) {
         constexpr int MY = decltype(mc)::value;
         auto k = fftg_cols_kernel<T, MY, MODE>;
         static const bool once = (set_lds(k, glds<T>(MY)), true);
@@ -689,7 +692,7 @@ void run_cols(fftg_args<T, T, T> a, hipStream_t st) {
 
 template <class T, bool PEAK>
 void run_rows_inv(const fftg_args<T, T, T>& a, hipStream_t st) {
-    dispatch_n<T, 4>(a.mx, [&](auto mc) {
+    dispatch_n<T, 4, true>(a.mx, [&](auto mc) {
         constexpr int MX = decltype(mc)::value;
         auto k = fftg_rows_inv_kernel<T, MX, PEAK>;
         static const bool once = (set_lds(k, glds<T>(MX)), true);
