@@ -7,9 +7,11 @@
 // `sum += a * b`), so double and float results are bit-identical to that order.
 //
 // Float and double run on the matrix cores (cross_corr_mm_kernel); slices of a few pixels and
-// those too wide for its LDS rows take the thread-per-shift kernel: one workgroup per (slice, 4-row band of shifts,
-// 64-column band of shifts), staged in LDS when both slices fit in 64 KiB.  int32 has no
-// matrix instruction with its wrapping sums and keeps the vector kernels: a register-blocked
+// those of which eight reference rows and the pattern rows of a workgroup's shifts do not fit
+// its LDS (square ones from 200 wide with a narrow window to 570 with a wide one in double, 460
+// to 1,190 in float) take the thread-per-shift kernel: one workgroup per (slice, 4-row band of
+// shifts, 64-column band of shifts), staged in LDS when both slices fit in 64 KiB.  int32 has
+// no matrix instruction with its wrapping sums and keeps the vector kernels: a register-blocked
 // one ("tiled") for slices up to 128 pixels wide, windows up to 256 wide and launches of at
 // least 256 workgroups, one with eight x-shifts per thread sliding a register window over
 // zero-padded rows ("x8") for other slices that fit in LDS, and the thread-per-shift one.

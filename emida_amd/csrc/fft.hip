@@ -681,7 +681,7 @@ void launch_fft_corr_prepared_noalloc(const T* pics, const T* ref, T* res, size2
         throw arg_error("cross_corr_fft without allocation: the reference spectra of " + std::to_string(ref_slices) +
                         " slices need " + std::to_string(spec) + " bytes, more than the " +
                         std::to_string(kFftStaticScratchBytes) + "-byte static scratch");
-    // the rest holds the work buffer of the three-kernel path's launch chunks
+    // the rest holds the work buffer of the general path's launch chunks
     const size_t left = kFftStaticScratchBytes - spec;
     char* base = nullptr;
     if (general) {

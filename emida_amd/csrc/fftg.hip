@@ -788,7 +788,8 @@ void launch_fftg_ref(const IN* pics, const S* sums, const T* hx, const T* hy, co
     a.total = nb;
     a.work = (cplx<T>*)work;
     a.spectra_out = spectra;
-    // the row and column stages double it; s.x s.y / (Mx My) is exact
+    // the row and column stages double it; s.x s.y / (Mx My) is exact for power-of-two lengths,
+    // rounded once for 192 and 384
     a.scale = (T)((double)side.x * side.y / ((double)a.mx * a.my));
     const size_t chunk = fftg_chunk(sizeof(T) == 8, side, nb);
     for (uint32_t f = 0; f < nb; f += (uint32_t)chunk) {

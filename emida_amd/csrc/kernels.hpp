@@ -168,7 +168,7 @@ template <class T>
 void launch_fft_corr_prepared(const T* pics, const T* ref, T* res, size2 side, uint32_t ref_slices, uint32_t batch,
                               hipStream_t st);
 // The same without any allocation: the reference spectra (and the work buffer of the
-// three-kernel path) live in the library's static device array of kFftStaticScratchBytes
+// general path) live in the library's static device array of kFftStaticScratchBytes
 // per GPU (shared by every call on that GPU: overlapping calls race).  Throws
 // arg_error when the spectra (plus one slice's work buffer) exceed it.
 constexpr size_t kFftStaticScratchBytes = (size_t)32 << 20;
@@ -179,7 +179,7 @@ template <class T>
 void launch_hadamard(cplx<T>* pics, const cplx<T>* ref, size2 one, uint32_t ref_slices, uint32_t batch,
                      hipStream_t st);
 
-// ---- fftg.hip: three-kernel FFT path (non-square slices, double sides above 64, sides
+// ---- fftg.hip: the general FFT path, four kernels (non-square slices, double sides above 64, sides
 // above 128; transforms up to 512 per axis), work buffers of half spectra in HBM
 bool fftg_needed(bool is_double, size2 side);               // the single-kernel paths do not take this shape
 size_t fftg_spectrum_bytes(bool is_double, size2 side);      // reference spectrum of one ROI

@@ -200,7 +200,7 @@ struct emida_offset_s {
     size2 src, slice, cross, buf;
     uint32_t nb, batch, total, n_in;
     uint32_t side = 0;  // FFT slice side (x)
-    bool fftg = false;  // FFT policy through the three-kernel path (fftg.hip)
+    bool fftg = false;  // FFT policy through the general path (fftg.hip)
     std::vector<size2> begins;
     size_t sum_bytes = 0;
 

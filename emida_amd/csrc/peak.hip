@@ -341,7 +341,7 @@ __device__ __forceinline__ void box_sync() {
 // columns l / 16 + 4 t of the row Y with Y mod 16 = l % 16); each step loads the one new row
 // into the lanes of the one that left, and the accumulators, which belong to y-shifts, move
 // to the next row of D instead.  Only the reference row passes through LDS (one row per
-// buffer, zeros around it).  That leaves a wave its own LDS of 13 KB and 12 waves on a CU;
+// buffer, zeros around it).  That leaves a wave its own LDS of 11 KB and 12 waves on a CU;
 // pattern rows staged in LDS (one shift per lane, vector FMAs, waves waiting on LDS 77% of
 // the time) took 5.5 ms for 12,800 slices of 128 x 128 in double where this takes 1.95 ms.
 constexpr int kBoxRows = 16;

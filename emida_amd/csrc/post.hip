@@ -1,6 +1,6 @@
 // Deformation post-step: per pattern, the projective map (homography) between the
 // ROI middles and their displaced positions, fitted algebraically, and its strain and
-// rotation.  One workgroup per pattern.
+// rotation.  One wave per pattern, four from 449 ROIs on.
 //
 // Reference (Python post-processing of the offsets):
 //  - python/process_offsets.py:31-97 (and python/test.py:137-198): relative to the
@@ -274,8 +274,11 @@ struct post_args {
     double* omega;
 };
 
-// NW waves per pattern (1: four patterns per workgroup; 4: one), K ROIs per lane, held in
-// registers; n <= 64 NW K.  Every lane runs the solve on the same values.
+// NW waves per pattern (1: four patterns per workgroup; 4: one), K ROIs per lane; n <= 64 NW K.
+// They are held in registers up to 2,048 ROIs (but for 28 to 36 bytes a lane with one wave);
+// the 32 per lane beyond go to scratch (944 bytes a lane): a pattern of 2,049 ROIs takes 110 us
+// where one of 2,048 takes 24, 1,000 patterns of 8,192 450 us (the kernel described below 43 ms).
+// Every lane runs the solve on the same values.
 //
 // Bound: the reads of the offsets and coefficients, and the chain of dependent operations of
 // the solve, which the waves of a SIMD hide for each other.  5,000 patterns x 400 ROIs
