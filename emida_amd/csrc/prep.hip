@@ -13,9 +13,12 @@ namespace emida_amd {
 // (src/sum.cu:65-98, 109-158).  Groups are added in ascending order when a ROI
 // needs more than one (the reference adds them atomically in no fixed order).
 // For uint32 sums the order does not change the result.
-// Bound by memory latency: the N loads of a thread are issued together (behind a condition
-// each they waited for one another: 672 slices of 161 x 95 in float 19.6 us, now 14.2).
-template <class IN, class S>
+// Bound by memory latency: the loads of a thread are issued together (behind a condition
+// each they waited for one another: 672 slices of 161 x 95 in float 19.6 us, now 14.2).  NL: at
+// least the loads that have a pixel, N at most (all ten where a slice has 400 pixels read its
+// last one nine times over: a float FFT pass over 90,000 slices of 20 x 20 took 1,117 us, with
+// the loads one after the other 927, with one 785).
+template <class IN, class S, uint32_t NL>
 __global__ __launch_bounds__(1024) void sum_kernel(const IN* __restrict__ pics, S* __restrict__ sums,
                                                    const size2* __restrict__ begins, size2 src, size2 slice,
                                                    uint32_t nb, uint32_t total) {
@@ -32,14 +35,14 @@ __global__ __launch_bounds__(1024) void sum_kernel(const IN* __restrict__ pics, 
     const uint32_t t = threadIdx.x;
     for (uint32_t b = 0; b < nblk; ++b) {
         S v = 0;
-        IN q[N];
+        IN q[NL];
 #pragma unroll
-        for (uint32_t n = 0; n < N; ++n) {
+        for (uint32_t n = 0; n < NL; ++n) {
             const uint32_t i = min(nblk * B * n + b * B + t, area - 1), py = i / slice.x;
             q[n] = pic[(size_t)py * src.x + (i - py * slice.x)];
         }
 #pragma unroll
-        for (uint32_t n = 0; n < N; ++n) v = nblk * B * n + b * B + t < area ? v + (S)q[n] : v;
+        for (uint32_t n = 0; n < NL; ++n) v = nblk * B * n + b * B + t < area ? v + (S)q[n] : v;
 #pragma unroll
         for (int off = 16; off > 0; off >>= 1) v += __shfl_down(v, off, 32);
         if (t % 32 == 0) part[t / 32] = v;
@@ -309,7 +312,14 @@ template <class IN, class S>
 void launch_sum(const IN* pics, S* sums, const size2* begins, size2 src, size2 slice, uint32_t nb, uint32_t total,
                 hipStream_t st) {
     if (total == 0) return;
-    sum_kernel<IN, S><<<total, 1024, 0, st>>>(pics, sums, begins, src, slice, nb, total);
+    const uint32_t area = slice.area(), nblk = div_up(area, 10u * 1024), loads = div_up(area, nblk * 1024);
+    auto launch = [&](auto nl) {
+        sum_kernel<IN, S, decltype(nl)::value><<<total, 1024, 0, st>>>(pics, sums, begins, src, slice, nb, total);
+    };
+    if (loads <= 1) launch(std::integral_constant<uint32_t, 1>{});
+    else if (loads <= 2) launch(std::integral_constant<uint32_t, 2>{});
+    else if (loads <= 4) launch(std::integral_constant<uint32_t, 4>{});
+    else launch(std::integral_constant<uint32_t, 10>{});
     EMIDA_LAUNCHED("sum_kernel");
 }
 
