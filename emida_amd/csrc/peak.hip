@@ -274,14 +274,17 @@ __global__ void subpixel_kernel(const T* __restrict__ neigh, int s, uint32_t n, 
 // without a finite screen maximum is swept whole: every shift of the window is
 // evaluated exactly, box by box, so its arg-max is the brute policy's as well.
 constexpr int kRefineCap = 512;
-// Candidates too wide for one box take boxes of 16 x 16, up to this many for every round it
-// would take to evaluate them one chain per lane, else the chains.  Boxes are counted first:
-// evaluating six and then the chains all the same cost unrelated 128 x 128 patterns (160
-// slices, more than six boxes) 1.43 ms in float and 1.39 in double, where the chains take 0.57
-// and 0.70; a limit of four boxes 0.92 and 0.83.  In float, whose products wait longer on one
-// another, two boxes cost what the chains do.
+// Candidates too wide for one box take boxes of 16 x 16, up to two for every round it would
+// take to evaluate them one chain per lane (in float, whose products wait longer on one another,
+// none for the first round), else the chains.  Boxes are counted first: evaluating six a round
+// and then the chains all the same cost unrelated 128 x 128 patterns (160 slices, more than six
+// boxes) 1.43 ms in float and 1.39 in double, where the chains take 0.57 and 0.70; a limit of
+// four boxes 0.92 and 0.83.  Many candidates side by side want the boxes: 784 slices of 64 x 64
+// in float, flat tops, 163 us, by chains 317.
 template <class T>
-constexpr int kSpreadBoxes = sizeof(T) == 8 ? 2 : 0;
+constexpr int spread_boxes(int rounds) {
+    return 2 * rounds - (sizeof(T) == 8 ? 0 : 2);
+}
 constexpr int kRowList = 256;  // screens of at most this many rows use the row maxima
 
 template <class T>
@@ -737,9 +740,9 @@ __global__ __launch_bounds__(NT, 3) void refine_kernel(const float* __restrict__
         return x >= 0 && y >= 0 && x < bw && y < bh;
     };
     bool chains = !sweep && !boxed;
-    if (kSpreadBoxes<T> && chains) {
+    if (chains) {
         int n = 0, x, y;
-        const int most = kSpreadBoxes<T> * (int)div_up(nc, (uint32_t)NT);
+        const int most = spread_boxes<T>((int)div_up(nc, (uint32_t)NT));
         while ((chains = next_box()) && ++n <= most) {
             for (uint32_t c = tid; c < nc; c += NT)
                 if (cand[c] < kTaken && in_box(cand[c], x, y)) cand[c] |= kTaken;
