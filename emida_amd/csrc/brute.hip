@@ -448,12 +448,13 @@ inline bool mm_plan(size2 size, size2 res, uint64_t total, mm_shape& m) {
     const int per = div_up(m.ntx, m.ntw);
     m.wx = per >= 4 ? 4 : (per >= 2 ? 2 : 1);
     m.wy = 4 / m.wx;
-    // Small slices of one or two tiles take one wave each: beside it the other three would only
-    // stage, which pays for larger slices and tall ones (brute pass over 800 slices of 24 x 8 in
-    // float: 24.1 us with four waves, 19.9 with one; 8 x 8: 16.2 and 14.0; 100 of 24 x 24 with a
-    // 9 x 9 window 17.8 and 19.4).
-    if (size.area() <= 256 && size.y <= 16 && m.nty == 1 && m.ntx <= 2) {
-        m.ntw = m.ntx;
+    // Small slices take one wave to a workgroup where one or two tiles are all they have (beside
+    // it the other three would only stage, which pays for larger slices and tall ones) or where
+    // there are two and more for every CU.  Pass over 800 slices, us, four waves / one: 24 x 8 in
+    // float 24.1 / 19.9, 8 x 8 16.2 / 14.0, 16 x 16 27.3 / 24.0, 24 x 8 in double 29.7 / 25.6; 25
+    // of 16 x 16 in double 15.8 / 18.3, 100 of 24 x 24 with a 9 x 9 window 17.8 / 19.4.
+    if (size.area() <= 256 && size.y <= 16 && ((m.nty == 1 && m.ntx <= 2) || total >= 512)) {
+        m.ntw = std::min(m.ntx, 2);
         m.wx = m.wy = 1;
     }
     m.nxb = div_up(m.ntx, m.wx * m.ntw);

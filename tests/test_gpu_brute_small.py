@@ -45,3 +45,16 @@ def test_not_finite(dt, size, where):
     got, exp = K.run_cross_corr(pics, ref, size, res, 1, 2), O.cross_corr(pics, ref, size, res, 1, 2)
     assert np.isfinite(exp).any() and not np.isfinite(exp).all()
     np.testing.assert_array_equal(got, exp)
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("size", [(7, 7), (10, 10), (12, 12), (16, 16), (24, 8), (17, 16), (60, 4), (100, 2)])
+def test_two_slices_for_every_cu(dt, size):
+    """From 512 slices on small ones of several tiles take one wave to a workgroup."""
+    for n in (511, 515):
+        rng = np.random.default_rng(n)
+        pics = rng.standard_normal(size[0] * size[1] * n).astype(dt)
+        ref = rng.standard_normal(size[0] * size[1]).astype(dt)
+        res = (2 * size[0] - 1, 2 * size[1] - 1)
+        np.testing.assert_array_equal(K.run_cross_corr(pics, ref, size, res, 1, n),
+                                      O.cross_corr(pics, ref, size, res, 1, n))
