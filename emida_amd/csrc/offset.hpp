@@ -169,7 +169,8 @@ class stage_pool {
         }
         block b;
         b.n = (n + kGrain - 1) & ~(kGrain - 1);
-        if (hipHostMalloc((void**)&b.p, b.n, hipHostMallocPortable) != hipSuccess) {
+        // (the default flag: coherent memory, which kernels of every device read past their caches)
+        if (hipHostMalloc((void**)&b.p, b.n, hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
             return {};
         }
